@@ -2914,8 +2914,8 @@ __global__ __launch_bounds__(256) void k_ring(const uint32_t *__restrict__ dM,
 // Halo sums: FP64 accumulation of the float Pos / Vel of the members in
 // ascending index order from the head (the order the host walks the ring
 // returned in next_out), so the host's Checkhalo / Output_Halos loops give
-// the same bits.  One wavefront per halo: the 64 lanes gather 64 members'
-// records at a time into LDS and then each of the first NQ lanes adds one
+// the same bits.  One wavefront per halo: the 64 lanes stage 64 members at a
+// time in LDS as doubles and then each of the first NQ lanes adds one
 // quantity over them, in order.  Quantities (q = lane):
 //   0-5    Pos x,y,z, Vel x,y,z                          (src_v2/FOF.c:805-810)
 //   with MOM, the second moments (src_v2/FOF.c:811-824):
@@ -2924,21 +2924,24 @@ __global__ __launch_bounds__(256) void k_ring(const uint32_t *__restrict__ dM,
 //   24-29  Pos products of those   30-35  Vel products   (for centred moments)
 // A float difference widened to double is exact here (same-halo members), and
 // products of two such numbers (< 53 significant bits) are exact, so only the
-// additions round.
-__device__ __forceinline__ double halo_quantity(int q, const float (&v)[6], const double (&ref)[6]) {
-  if (q < 6) return (double)v[q];
-  // component pairs of the products: xx yy zz xy xz yz
-  const int r = q < 18 ? q - 6 : (q < 24 ? q - 18 : q - 24);
-  const int blk = r / 6, k = r % 6, o = blk * 3;  // blk 0: Pos, 1: Vel
-  if (q >= 18 && q < 24) {
-    const int c = r;  // 0-5: Pos xyz, Vel xyz
-    return (double)v[c] - ref[c];
-  }
-  const int ca = o + (k < 3 ? k : (k < 5 ? 0 : 1));
-  const int cb = o + (k < 3 ? k : (k == 3 ? 1 : 2));
-  if (q < 18) return (double)v[ca] * (double)v[cb];
-  return ((double)v[ca] - ref[ca]) * ((double)v[cb] - ref[cb]);
-}
+// additions round.  Every quantity is the product of two staged rows: 0-5 the
+// components, 6-11 the deviations (MOM), and a row of ones for those that are
+// no product (times 1.0 is exact).  Members past the last are staged as zeros:
+// a sum that began at +0.0 is never -0.0, so adding +0.0 changes no bit, and
+// the adding loop runs eight members at a time with its LDS reads issued ahead
+// of the additions.
+//
+// What bounds it: the largest halo's chain of dependent additions while
+// there are few halos, the gather (one 128-byte line per member record) when
+// there are many.  For halos above kHaloAhead blocks the records of the next
+// 256 members are in registers and their list entries 256 further, every
+// load unconditional, so that neither of the gather's two dependent loads is
+// waited for in a block.  Before (float rows, one LDS read and one conversion
+// ahead of every addition, the next 64 records loaded during the block):
+// 437 us for the 64^3 box, whose largest halo has about 1e4 members, 2669 with
+// MOM for a 144^3 box and 2.22 ms for a 512^3 box; now 72, 125 and 1.72 ms.
+constexpr int kHaloAhead = 4;   // 64-member blocks in flight
+constexpr int kHaloRow = 66;    // doubles a row: 16-byte aligned, rows in different banks
 
 template <bool MOM>
 __global__ __launch_bounds__(256) void k_halo_sums(const uint32_t *__restrict__ dH,
@@ -2957,66 +2960,126 @@ __global__ __launch_bounds__(256) void k_halo_sums(const uint32_t *__restrict__ 
                                                    uint32_t *__restrict__ hhead,
                                                    unsigned long long *__restrict__ ctr) {
   constexpr int NQ = MOM ? 36 : 6;
-  // two stages per wave: the records of the next 64 members are loaded while
-  // the first NQ lanes add up the current ones
-  __shared__ float stage[4][2][6][64];
+  constexpr int kOnes = 12;
+  constexpr int kRows = MOM ? 13 : 6;
+  __shared__ __align__(16) double stage[4][kRows][kHaloRow];
   const uint32_t H = *dH;
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const uint32_t nw = gridDim.x * (blockDim.x >> 6);
   uint32_t owned_cnt = 0;
   int hint = 0;
+  // the two rows whose product is the lane's quantity
+  int ra = lane < 6 ? lane : 0, rb = kOnes;
+  if (MOM && lane >= 6 && lane < NQ) {
+    if (lane >= 18 && lane < 24) {
+      ra = lane - 18 + 6;
+    } else {  // component pairs of the products: xx yy zz xy xz yz
+      const int r = lane < 18 ? lane - 6 : lane - 24, o = (r / 6) * 3 + (lane < 18 ? 0 : 6), k = r % 6;
+      ra = o + (k < 3 ? k : (k < 5 ? 0 : 1));
+      rb = o + (k < 3 ? k : (k == 3 ? 1 : 2));
+    }
+  }
+  if (MOM) {
+    stage[w][kOnes][lane] = 1.0;
+    wave_sync();
+  }
+  const double *const pa = stage[w][ra], *const pb = stage[w][MOM ? rb : 0];
   for (uint32_t h = blockIdx.x * (blockDim.x >> 6) + w; h < H; h += nw) {
-    const uint32_t k0 = hk[h];
-    const uint32_t lab = skey[k0];
-    const uint32_t n = hsize[lab];
+    // wave-uniform, visibly so: branches on them leave the loads in flight countable
+    const uint32_t k0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)hk[h]);
+    const uint32_t lab = (uint32_t)__builtin_amdgcn_readfirstlane((int)skey[k0]);
+    const uint32_t n = (uint32_t)__builtin_amdgcn_readfirstlane((int)hsize[lab]);
     hint = vol_from(vbeg, nvol, lab, hint);  // halos ascend by head, per wave too
     const int v = hint;
     const VolDev &V = vols[v];
+    const double elo[3] = {V.rmin_buff[0], V.rmin_buff[1], V.rmin_buff[2]};
+    const double ehi[3] = {V.rmax_buff[0], V.rmax_buff[1], V.rmax_buff[2]}, el = V.linklength;
     double acc = 0;
     uint32_t warn = 0;
-    float r[6];
     double ref[6];
-    auto fetch = [&](uint32_t k) {
-      if (lane < min(64u, n - k)) {
-        const uint8_t *rec = base + (uint64_t)sval[k0 + k + lane] * stride;
-        const float *pp = reinterpret_cast<const float *>(rec + offpos);
-        const float *vv = reinterpret_cast<const float *>(rec + offvel);
-        r[0] = pp[0], r[1] = pp[1], r[2] = pp[2], r[3] = vv[0], r[4] = vv[1], r[5] = vv[2];
+    // list entry and record of member k + lane; past the last, the last's again
+    auto entry = [&](uint32_t k) -> uint32_t { return sval[k0 + min(k + (uint32_t)lane, n - 1)]; };
+    auto fetch = [&](uint32_t i, float (&q)[6]) {
+      const uint8_t *rec = base + (uint64_t)i * stride;
+      const float *pp = reinterpret_cast<const float *>(rec + offpos);
+      const float *vv = reinterpret_cast<const float *>(rec + offvel);
+      q[0] = pp[0], q[1] = pp[1], q[2] = pp[2], q[3] = vv[0], q[4] = vv[1], q[5] = vv[2];
+    };
+    auto store = [&](uint32_t m, const float (&r)[6]) {
+      const bool in = (uint32_t)lane < m;
+#pragma unroll
+      for (int d = 0; d < 3; d++) {
+        const double q = r[d];
+        if (in && ((q - elo[d] < el) || (ehi[d] - q < el))) warn |= 1u << d;
+      }
+#pragma unroll
+      for (int c = 0; c < 6; c++) {
+        stage[w][c][lane] = in ? (double)r[c] : 0.0;
+        if (MOM) stage[w][6 + c][lane] = in ? (double)r[c] - ref[c] : 0.0;
       }
     };
-    fetch(0);
-    if (MOM) {  // the head (first member) is the reference point of the deviations
-#pragma unroll
-      for (int c = 0; c < 6; c++) ref[c] = (double)__shfl(r[c], 0, 64);
-    }
-    int b = 0;
-    for (uint32_t k = 0; k < n; k += 64, b ^= 1) {
-      const uint32_t m = min(64u, n - k);
-      if ((uint32_t)lane < m) {
-#pragma unroll
-        for (int c = 0; c < 6; c++) stage[w][b][c][lane] = r[c];
-#pragma unroll
-        for (int d = 0; d < 3; d++) {
-          const double q = r[d];
-          if ((q - V.rmin_buff[d] < V.linklength) || (V.rmax_buff[d] - q < V.linklength))
-            warn |= 1u << d;
-        }
-      }
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-      if (k + 64 < n) fetch(k + 64);
+    auto add = [&](uint32_t m) {
+      wave_sync();
       if (lane < NQ) {
-        if (lane < 6) {
-          for (uint32_t q = 0; q < m; q++) acc += (double)stage[w][b][lane][q];
-        } else {
-          for (uint32_t q = 0; q < m; q++) {
-            float vv[6];
+        for (uint32_t q = 0; q < m; q += 8) {
+          double a[8];
 #pragma unroll
-            for (int c = 0; c < 6; c++) vv[c] = stage[w][b][c][q];
-            acc += halo_quantity(lane, vv, ref);
+          for (int t = 0; t < 8; t++) a[t] = pa[q + t];
+          if (MOM) {
+            double b[8];
+#pragma unroll
+            for (int t = 0; t < 8; t++) b[t] = pb[q + t];
+#pragma unroll
+            for (int t = 0; t < 8; t++) a[t] = a[t] * b[t];
           }
+#pragma unroll
+          for (int t = 0; t < 8; t++) acc += a[t];
         }
       }
+      wave_sync();  // the rows are written again
+    };
+    // the head (first member) is the reference point of the deviations
+    auto set_ref = [&](const float (&r)[6]) {
+#pragma unroll
+      for (int c = 0; c < 6; c++) ref[c] = MOM ? (double)__shfl(r[c], 0, 64) : 0.0;
+    };
+    if (n <= 64u * kHaloAhead) {
+      float r[6];
+      fetch(entry(0), r);
+      set_ref(r);
+      for (uint32_t k = 0; k < n; k += 64) {
+        store(n - k, r);
+        if (k + 64 < n) fetch(entry(k + 64), r);
+        add(min(64u, n - k));
+      }
+    } else {
+      // every load unconditional (their indices stay in the halo), so that a
+      // block waits for its own records only, not for those behind them
+      float r[kHaloAhead][6];
+      uint32_t at[kHaloAhead];
+#pragma unroll
+      for (int j = 0; j < kHaloAhead; j++) at[j] = entry(64 * j);
+#pragma unroll
+      for (int j = 0; j < kHaloAhead; j++) fetch(at[j], r[j]);
+#pragma unroll
+      for (int j = 0; j < kHaloAhead; j++) at[j] = entry(64 * (kHaloAhead + j));
+      set_ref(r[0]);
+      uint32_t k = 0;
+      for (; k + 64 * kHaloAhead <= n; k += 64 * kHaloAhead) {
+#pragma unroll
+        for (int j = 0; j < kHaloAhead; j++) {
+          store(64, r[j]);
+          fetch(at[j], r[j]);
+          at[j] = entry(k + 64 * (2 * kHaloAhead + j));
+          add(64);
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < kHaloAhead; j++)
+        if (k + 64 * j < n) {
+          store(n - k - 64 * j, r[j]);
+          add(min(64u, n - k - 64 * j));
+        }
     }
     const double s0 = __shfl(acc, 0, 64), s1 = __shfl(acc, 1, 64), s2 = __shfl(acc, 2, 64);
     const double s3 = __shfl(acc, 3, 64), s4 = __shfl(acc, 4, 64), s5 = __shfl(acc, 5, 64);
