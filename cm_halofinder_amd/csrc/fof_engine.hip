@@ -2660,16 +2660,31 @@ __global__ __launch_bounds__(256) void k_group_cursors(const uint32_t *__restric
   for (uint32_t i = t; i < R; i += gridDim.x * blockDim.x) cursor[glab[i]] = offs[i];
 }
 
-// Sorting each segment of the member list by index.  Groups of at most
-// kSegWave members are sorted by one wave each in registers (a bitonic
-// network; 64 E elements for E per lane, lane-major, so that the stages
-// below distance E stay inside a lane and the others are lane shuffles);
-// larger ones are listed for k_seg_sort_large: a workgroup each, a bitonic
-// sort in LDS up to kSegLds members, beyond that an LSD radix sort (four
-// 8-bit digits, stable scatter per 256-element tile) through scratch.
+// Sorting each segment of the member list by index.  Groups of at most four
+// members are sorted by a lane each; larger ones are listed, up to kSegWave
+// members for a wave each (a bitonic network in registers; 64 E elements for E
+// per lane, lane-major, so that the stages below distance E stay inside a lane
+// and the others are lane shuffles), the rest for a workgroup each: an LSD
+// radix sort in LDS with as many digits as the indices have bits, up to
+// kSegLds members by 256 threads and up to kSegLdsBig by 1024; beyond that
+// runs of kSegLdsBig merged pairwise through scratch.
+//
+// Why lists: groups come in label order and a label is the group's lowest
+// index, so the first few hundred groups of a volume are its largest; a wave
+// that took 64 consecutive groups sorted all of those alone.  64^3 box: 216 us
+// there and 112 us in four radix passes through global memory over the largest
+// group, now 5 + 33 + 23 us; 512^3 box 307 + 676 us, now 160 + 580 + 240 (of
+// these, merging chunks in LDS by binary search in place of the radix passes
+// took 45 us for the largest group of the 64^3 box, and a bitonic sort of
+// kSegLds members by 256 threads 676).  What bounds it now: the ranking of
+// the largest group on one compute unit while there are few groups (eight
+// ballots for 64 keys), shuffles and latency when many.  Four waves per SIMD:
+// six spill (508 us at 512^3, 37 at 64^3).
 constexpr uint32_t kSegWave = 1024;
-constexpr uint32_t kSegLds = 4096;
-constexpr int kSmLarge = 9;  // groups listed for k_seg_sort_large
+constexpr uint32_t kSegLds = 4096, kSegLdsBig = 16384;
+constexpr int kSmLarge = 9;  // groups listed for a workgroup each, up to kSegLds members
+constexpr int kSmMid = 12;   // groups listed for a wave each
+constexpr int kSmHuge = 13;  // larger groups, a workgroup of 1024 threads each
 
 // n <= 64: one element a lane, the network only as wide as n needs
 __device__ __forceinline__ void seg_sort_lane(uint32_t *__restrict__ p, uint32_t n, uint32_t lane) {
@@ -2685,9 +2700,11 @@ __device__ __forceinline__ void seg_sort_lane(uint32_t *__restrict__ p, uint32_t
   if (lane < n) p[lane] = v;
 }
 
-// 32 E < n <= 64 E: element a = E lane + e in register e of the lane
+// n <= 64 E elements of p to o (may be p): element a = E lane + e in register
+// e of the lane
 template <int E>
-__device__ __forceinline__ void seg_sort_regs(uint32_t *__restrict__ p, uint32_t n, uint32_t lane) {
+__device__ __forceinline__ void seg_sort_regs(const uint32_t *p, uint32_t *o, uint32_t n,
+                                              uint32_t lane) {
   constexpr uint32_t P = 64u * E;
   uint32_t v[E];
 #pragma unroll
@@ -2722,24 +2739,40 @@ __device__ __forceinline__ void seg_sort_regs(uint32_t *__restrict__ p, uint32_t
 #pragma unroll
   for (int e = 0; e < E; e++) {
     const uint32_t a = lane * E + e;
-    if (a < n) p[a] = v[e];
+    if (a < n) o[a] = v[e];
   }
 }
 
-// A wave takes 64 consecutive groups at a time: groups of at most four
-// members are sorted by their lane alone (most groups are pairs), the others
-// one at a time by the whole wave; groups above kSegWave members are
-// appended to the list for k_seg_sort_large.
+// The lanes sort the groups of at most four members and list the others
+// (gathered per workgroup in LDS: one append a full list, so the two device
+// counters see few atomics).
+constexpr uint32_t kSegList = 1024;
+
 __global__ __launch_bounds__(256) void k_seg_sort(const uint32_t *__restrict__ dR,
                                                   const uint32_t *__restrict__ offs,
                                                   uint32_t *__restrict__ mval,
+                                                  uint32_t *__restrict__ mid,
+                                                  uint32_t *__restrict__ dMid,
                                                   uint32_t *__restrict__ large,
-                                                  uint32_t *__restrict__ dL) {
+                                                  uint32_t *__restrict__ dL,
+                                                  uint32_t *__restrict__ huge,
+                                                  uint32_t *__restrict__ dHuge) {
+  __shared__ uint32_t lst[kSegList], nl, base;
   const uint32_t R = *dR;
   const uint32_t lane = threadIdx.x & 63;
-  const uint32_t w0 = blockIdx.x * 4 + (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  for (uint32_t c0 = w0 * 64; c0 < R; c0 += gridDim.x * 4 * 64) {
-    const uint32_t g = c0 + lane;
+  if (threadIdx.x == 0) nl = 0;
+  __syncthreads();
+  auto flush = [&]() {
+    __syncthreads();
+    if (threadIdx.x == 0) base = nl ? atomicAdd(dMid, nl) : 0u;
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < nl; i += 256) mid[base + i] = lst[i];
+    __syncthreads();
+    if (threadIdx.x == 0) nl = 0;
+    __syncthreads();
+  };
+  for (uint32_t c0 = blockIdx.x * 256; c0 < R; c0 += gridDim.x * 256) {
+    const uint32_t g = c0 + threadIdx.x;
     uint32_t s = 0, n = 0;
     if (g < R) s = offs[g], n = offs[g + 1] - s;
     if (n <= 4) {  // a comparator network on the lane's own group
@@ -2755,103 +2788,171 @@ __global__ __launch_bounds__(256) void k_seg_sort(const uint32_t *__restrict__ d
       for (int e = 0; e < 4; e++)
         if ((uint32_t)e < n) mval[s + e] = v[e];
     }
-    unsigned long long big = __ballot(n > 4);
-    while (big) {
-      const int l = __builtin_ctzll(big);
-      big &= big - 1;
-      const uint32_t sb = (uint32_t)__builtin_amdgcn_readlane((int)s, l);
-      const uint32_t nb = (uint32_t)__builtin_amdgcn_readlane((int)n, l);
-      uint32_t *p = mval + sb;
-      if (nb <= 64) seg_sort_lane(p, nb, lane);
-      else if (nb <= 128) seg_sort_regs<2>(p, nb, lane);
-      else if (nb <= 256) seg_sort_regs<4>(p, nb, lane);
-      else if (nb <= 512) seg_sort_regs<8>(p, nb, lane);
-      else if (nb <= kSegWave) seg_sort_regs<16>(p, nb, lane);
-      else if (lane == 0) large[atomicAdd(dL, 1u)] = c0 + (uint32_t)l;
+    const bool m = n > 4 && n <= kSegWave;
+    const unsigned long long bm = __ballot(m);
+    if (bm) {
+      uint32_t b = 0;
+      if (lane == 0) b = atomicAdd(&nl, (uint32_t)__popcll(bm));
+      b = (uint32_t)__builtin_amdgcn_readfirstlane((int)b);
+      if (m) lst[b + (uint32_t)__popcll(bm & ((1ull << lane) - 1))] = g;
     }
+    if (n > kSegLds) huge[atomicAdd(dHuge, 1u)] = g;
+    else if (n > kSegWave) large[atomicAdd(dL, 1u)] = g;
+    __syncthreads();
+    if (nl > kSegList - 256) flush();  // uniform: nl is read after the barrier by all
+    __syncthreads();
+  }
+  flush();
+}
+
+// One merge round of width W (a power of two) from a[0 .. n) to o[0 .. n) by
+// NT threads: an element's place in its merged pair of runs is its rank in its
+// own run plus its rank in the partner run (the values are distinct), found
+// for four elements at once so that their reads overlap.
+template <int NT>
+__device__ __forceinline__ void merge_round(const uint32_t *a, uint32_t *o, uint32_t n, uint32_t W) {
+  for (uint32_t i0 = threadIdx.x; i0 < n; i0 += 4 * NT) {
+    uint32_t key[4], at[4], run[4], rl[4], lo[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const uint32_t i = min(i0 + j * NT, n - 1);
+      const uint32_t b = i & ~(2 * W - 1), mid = min(b + W, n), end = min(b + 2 * W, n);
+      const bool left = i < mid;
+      key[j] = a[i];
+      run[j] = left ? mid : b;
+      rl[j] = left ? end - mid : mid - b;
+      at[j] = left ? i : b + (i - mid);
+      lo[j] = 0;
+    }
+    for (uint32_t st = W; st > 0; st >>= 1) {
+#pragma unroll
+      for (int j = 0; j < 4; j++)
+        if (lo[j] + st <= rl[j] && a[run[j] + lo[j] + st - 1] < key[j]) lo[j] += st;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+      if (i0 + j * NT < n) o[at[j] + lo[j]] = key[j];
   }
 }
 
-__global__ __launch_bounds__(256) void k_seg_sort_large(const uint32_t *__restrict__ dL,
-                                                        const uint32_t *__restrict__ large,
-                                                        const uint32_t *__restrict__ offs,
-                                                        uint32_t *__restrict__ mval,
-                                                        uint32_t *__restrict__ scratch) {
-  __shared__ uint32_t sk[kSegLds];
-  __shared__ uint32_t hist[256], wc[4][256], wsum[4];
-  const uint32_t nl = *dL;
-  const uint32_t t = threadIdx.x, lane = t & 63, w = t >> 6;
+// Groups of list `large` by workgroups of NT threads (up to LDS members in
+// LDS), then, in the 256-thread form, the groups of list `mid` by waves.
+template <int NT, uint32_t LDS, bool MID>
+__global__ __launch_bounds__(NT, 4) void k_seg_sort_list(const uint32_t *__restrict__ dL,
+                                                      const uint32_t *__restrict__ large,
+                                                      const uint32_t *__restrict__ dMid,
+                                                      const uint32_t *__restrict__ mid,
+                                                      const uint32_t *__restrict__ offs,
+                                                      uint32_t *__restrict__ mval,
+                                                      uint32_t *__restrict__ scratch, int bits) {
+  constexpr int kWaves = NT / 64, kR = LDS / NT;  // waves, elements a thread holds
+  static_assert(NT >= 256, "a thread for each digit");
+  __shared__ uint32_t sk[LDS], wcnt[kWaves][256], wsum[4];
+  const uint32_t t = threadIdx.x, lane = t & 63;
+  const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane((int)(t >> 6));
   const unsigned long long lt = (1ull << lane) - 1;
-  for (uint32_t q = blockIdx.x; q < nl; q += gridDim.x) {
-    const uint32_t g = large[q];
-    const uint32_t s = offs[g], n = offs[g + 1] - s;
-    if (n <= kSegLds) {
-      uint32_t P = 128;
-      while (P < n) P <<= 1;
+  const int passes = (bits + 7) / 8, width = (bits + passes - 1) / passes;
+  // n <= LDS elements at p, sorted in place: LSD radix, the keys of a pass in
+  // registers between its ranking and its scatter; wave w ranks the elements
+  // [w per, (w + 1) per) 64 at a time, lanes of one digit by ballots
+  auto sort_lds = [&](uint32_t *p, uint32_t n) {
+    const uint32_t per = (n + NT - 1) / NT * 64, i0 = w * per, i1 = min(n, i0 + per);
+    for (int k = 0; k < passes; k++) {
+      const int shift = k * width;
+      const uint32_t mask = (1u << width) - 1;
       __syncthreads();
-      for (uint32_t i = t; i < P; i += 256) sk[i] = i < n ? mval[s + i] : 0xFFFFFFFFu;
+      for (uint32_t q = t; q < kWaves * 256u; q += NT) (&wcnt[0][0])[q] = 0;
       __syncthreads();
-      for (uint32_t k = 2; k <= P; k <<= 1)
-        for (uint32_t j = k >> 1; j > 0; j >>= 1) {
-          for (uint32_t i = t; i < P / 2; i += 256) {
-            const uint32_t a = ((i & ~(j - 1)) << 1) | (i & (j - 1)), b = a + j;
-            const uint32_t x = sk[a], y = sk[b];
-            if ((x > y) == ((a & k) == 0)) sk[a] = y, sk[b] = x;
-          }
-          __syncthreads();
+      uint32_t key[kR], rk[kR];
+#pragma unroll
+      for (int r = 0; r < kR; r++) {
+        if (64u * r >= per) break;
+        const uint32_t i = i0 + 64 * r + lane;
+        const bool valid = i < i1;
+        key[r] = valid ? (k ? sk[i] : p[i]) : 0u;
+      }
+#pragma unroll
+      for (int r = 0; r < kR; r++) {
+        if (64u * r >= per) break;
+        const bool valid = i0 + 64 * r + lane < i1;
+        const uint32_t d = (key[r] >> shift) & mask;
+        unsigned long long peers = __ballot(valid);
+        for (int b = 0; b < width; b++) {
+          const bool on = (d >> b) & 1u;
+          const unsigned long long bb = __ballot(on);
+          peers &= on ? bb : ~bb;
         }
-      for (uint32_t i = t; i < n; i += 256) mval[s + i] = sk[i];
-      continue;
-    }
-    uint32_t *src = mval + s, *dst = scratch + s;
-    for (int shift = 0; shift < 32; shift += 8) {
+        const uint32_t below = (uint32_t)__popcll(peers & lt);
+        uint32_t old = 0;
+        if (valid) old = wcnt[w][d];
+        wave_sync();
+        if (valid && below == 0) wcnt[w][d] = old + (uint32_t)__popcll(peers);
+        wave_sync();
+        rk[r] = old + below;
+      }
       __syncthreads();
-      hist[t] = 0;
-      __syncthreads();
-      for (uint32_t i = t; i < n; i += 256) atomicAdd(&hist[(src[i] >> shift) & 255u], 1u);
-      __syncthreads();
-      {  // exclusive scan of the 256 digit counts: the digits' cursors
-        const uint32_t c = hist[t];
-        uint32_t inc = c;
+      uint32_t c = 0, inc = 0;
+      if (t < 256) {  // each digit's total, scanned over the digits
+#pragma unroll
+        for (int q = 0; q < kWaves; q++) {
+          const uint32_t x = wcnt[q][t];
+          wcnt[q][t] = c;
+          c += x;
+        }
+        inc = c;
 #pragma unroll
         for (int o = 1; o < 64; o <<= 1) {
           const uint32_t u = __shfl_up(inc, o, 64);
           if (lane >= (uint32_t)o) inc += u;
         }
         if (lane == 63) wsum[w] = inc;
-        __syncthreads();
+      }
+      __syncthreads();
+      if (t < 256) {
         uint32_t pre = inc - c;
-        for (uint32_t q2 = 0; q2 < w; q2++) pre += wsum[q2];
-        hist[t] = pre;
-      }
-      for (uint32_t b0 = 0; b0 < n; b0 += 256) {
-        const uint32_t i = b0 + t;
-        const bool valid = i < n;
-        const uint32_t key = valid ? src[i] : 0u;
-        const uint32_t d = (key >> shift) & 255u;
-        unsigned long long peers = __ballot(valid);
+        for (uint32_t q = 0; q < w; q++) pre += wsum[q];
 #pragma unroll
-        for (int bit = 0; bit < 8; bit++) {
-          const bool on = (d >> bit) & 1u;
-          const unsigned long long bb = __ballot(on);
-          peers &= on ? bb : ~bb;
-        }
-        __syncthreads();  // the previous tile's reads of wc and hist are done
-        wc[w][lane] = 0, wc[w][lane + 64] = 0, wc[w][lane + 128] = 0, wc[w][lane + 192] = 0;
-        __syncthreads();
-        if (valid && (peers & lt) == 0) wc[w][d] = (uint32_t)__popcll(peers);
-        __syncthreads();
-        if (valid) {
-          uint32_t at = hist[d] + (uint32_t)__popcll(peers & lt);
-          for (uint32_t q2 = 0; q2 < w; q2++) at += wc[q2][d];
-          dst[at] = key;
-        }
-        __syncthreads();
-        hist[t] += wc[0][t] + wc[1][t] + wc[2][t] + wc[3][t];
+        for (int q = 0; q < kWaves; q++) wcnt[q][t] += pre;
       }
-      uint32_t *tmp = src;
-      src = dst, dst = tmp;
+      __syncthreads();
+#pragma unroll
+      for (int r = 0; r < kR; r++) {
+        if (64u * r >= per) break;
+        if (i0 + 64 * r + lane < i1) sk[wcnt[w][(key[r] >> shift) & mask] + rk[r]] = key[r];
+      }
     }
+    __syncthreads();
+    for (uint32_t i = t; i < n; i += NT) p[i] = sk[i];
+  };
+  const uint32_t nl = *dL;
+  for (uint32_t q = blockIdx.x; q < nl; q += gridDim.x) {
+    const uint32_t g = large[q];
+    const uint32_t s = offs[g], n = offs[g + 1] - s;
+    uint32_t *src = mval + s, *dst = scratch + s;
+    for (uint32_t c = 0; c < n; c += LDS) sort_lds(src + c, min(LDS, n - c));
+    for (uint32_t W = LDS; W < n; W <<= 1) {
+      __syncthreads();  // the workgroup's writes are visible to it
+      merge_round<NT>(src, dst, n, W);
+      uint32_t *x = src;
+      src = dst, dst = x;
+    }
+    if (src != mval + s) {
+      __syncthreads();
+      for (uint32_t i = t; i < n; i += NT) mval[s + i] = src[i];
+    }
+  }
+  if (!MID) return;
+  const uint32_t nm = *dMid;
+  for (uint32_t q = blockIdx.x * (NT / 64) + w; q < nm; q += gridDim.x * (NT / 64)) {
+    const uint32_t g = mid[q];
+    const uint32_t s = (uint32_t)__builtin_amdgcn_readfirstlane((int)offs[g]);
+    const uint32_t n = (uint32_t)__builtin_amdgcn_readfirstlane((int)offs[g + 1]) - s;
+    uint32_t *p = mval + s;
+    if (n <= 64) seg_sort_lane(p, n, lane);
+    else if (n <= 128) seg_sort_regs<2>(p, p, n, lane);
+    else if (n <= 256) seg_sort_regs<4>(p, p, n, lane);
+    else if (n <= 512) seg_sort_regs<8>(p, p, n, lane);
+    else seg_sort_regs<16>(p, p, n, lane);
   }
 }
 
@@ -3908,7 +4009,10 @@ static int enqueue_run(Run &r, hipStream_t st) {
   uint32_t *offs = sk1, *glist = sv1 + 64;
   uint32_t *cursor = rtab;             // per label, from its group's first slot
   uint32_t *p32 = reinterpret_cast<uint32_t *>(pos4);
-  uint32_t *large = p32 + 3 * N, *hflags = p32 + 2 * N;
+  // groups above kSegLds, kSegWave and four members (at most N / 4096,
+  // N / 1024 and N / 5 of them)
+  uint32_t *huge = p32 + 3 * N, *large = huge + N / kSegLds, *mid = large + N / kSegWave;
+  uint32_t *hflags = p32 + 2 * N;
   if ((rc = tb(9))) return rc;
   if ((rc = fill_u32(gbits, nw, 0u, st))) return rc;
   k_group_bits<<<gN, 256, 0, st>>>(NN, par, gsize, minorig, pos4, gbits, lsize, single, dV, dVB,
@@ -3955,10 +4059,16 @@ static int enqueue_run(Run &r, hipStream_t st) {
   // free cell-sorted positions)
   if ((rc = tb(10))) return rc;
   k_seg_sort<<<(uint32_t)std::min<uint64_t>((rcap + 255) / 256, 8192), 256, 0, st>>>(
-      small + kSmR, offs, sv0, large, small + kSmLarge);
+      small + kSmR, offs, sv0, mid, small + kSmMid, large, small + kSmLarge, huge, small + kSmHuge);
   FOF_HIP(hipGetLastError());
-  k_seg_sort_large<<<(uint32_t)std::min<uint64_t>(N / kSegWave + 1, 8192), 256, 0, st>>>(
-      small + kSmLarge, large, offs, sv0, p32);
+  if (N > kSegLds) {
+    k_seg_sort_list<1024, kSegLdsBig, false>
+        <<<(uint32_t)std::min<uint64_t>(N / kSegLds, 512), 1024, 0, st>>>(
+            small + kSmHuge, huge, nullptr, nullptr, offs, sv0, p32, bits_for(N));
+    FOF_HIP(hipGetLastError());
+  }
+  k_seg_sort_list<256, kSegLds, true><<<(uint32_t)std::min<uint64_t>(N / 20 + 1, 8192), 256, 0, st>>>(
+      small + kSmLarge, large, small + kSmMid, mid, offs, sv0, p32, bits_for(N));
   FOF_HIP(hipGetLastError());
   if ((rc = te(10))) return rc;
   // 9: the rings
