@@ -445,20 +445,41 @@ constexpr uint32_t kBigCell = 256;
 
 // ---------------------------------------------------------------------------
 // 1-3 (dense grid): counting sort by cell without global atomics.
-// Cells are grouped into fine buckets of 2^14 consecutive cells and those into
-// coarse buckets of 256 fine buckets.
-//   A: per tile of kPartTile particles, cell keys and an LDS histogram of
-//      coarse buckets; scan; scatter {key}, {x,y,z,index} by coarse bucket
-//   B: the same inside each coarse bucket, by fine bucket (256 ways)
-//   C: one workgroup per fine bucket: LDS counters for its 2^14 cells,
+// Cells are grouped into fine buckets of 2^fb consecutive cells and, where
+// there are more than kMaxBuckets of those, into coarse buckets of 256.
+//   A: per tile of particles, cell keys and an LDS histogram of the (coarse)
+//      buckets; scan; scatter {key}, {x,y,z,index} by bucket
+//   B: (coarse buckets only) the same inside each coarse bucket, 256 ways
+//   C: one workgroup per fine bucket: LDS counters for its 2^fb cells,
 //      scan -> cell starts and dense-cell lists, LDS cursors -> cell order
 // 256-way partitions keep a tile's open output lines few enough to be
 // combined in L2; all counting is in LDS.
+//
+// Sizes: tiles of kPartTile particles and buckets of 2^14 cells for large
+// calls; smaller ones shrink both (part_tile, fine_bits) until about 1024
+// tiles and 256 buckets are in flight, since one workgroup's serial pass over
+// 32768 particles is what a small call waits for (64^3 box, 11 tiles and 22
+// buckets, passes A, B and C: 57 + 94, 35 + 44 and 35 us; now 7 + 8 and 15).
+// Up to kMaxBuckets fine buckets pass A places them directly and pass B is
+// not run: with the 1100 buckets of a 256^3 box 426 us for A's scatter against
+// 201 + 46 + 234 for the two (and seven launches fewer), although a sub-tile
+// then holds only two particles a bucket; more buckets than that leave the
+// scatter no room for a second workgroup on a compute unit.
 // ---------------------------------------------------------------------------
 constexpr uint32_t kPartTile = 32768;
-constexpr int kFineBits = 14;
+constexpr int kFineBits = 14;  // of the largest fine buckets
 constexpr uint32_t kFineCells = 1u << kFineBits;
-constexpr int kMaxCoarse = 512;  // C < 2^31 cells
+constexpr int kMaxBuckets = 1280;  // of pass A
+constexpr int kMaxCoarse = 512;    // coarse buckets (C < 2^31 cells)
+
+static uint32_t part_tile(uint64_t N) {
+  return (uint32_t)std::min<uint64_t>(kPartTile, std::max<uint64_t>(1, (N / 1024 + 1023) / 1024) * 1024);
+}
+static int fine_bits(uint64_t C) {
+  int fb = kFineBits;
+  while (fb > 11 && (C >> fb) < 256) fb--;
+  return fb;
+}
 
 __device__ __forceinline__ uint32_t cell_of_xyz(float x, float y, float z, const VolDev &V,
                                                 uint32_t *__restrict__ err) {
@@ -481,14 +502,15 @@ __global__ __launch_bounds__(256) void k_pa_count(const uint8_t *__restrict__ ba
                                                   const VolDev *__restrict__ vols,
                                                   const uint32_t *__restrict__ vbeg, int nvol,
                                                   uint32_t Bc, uint32_t ntiles,
+                                                  uint32_t ptile, int shift,
                                                   uint32_t *__restrict__ key,
                                                   uint32_t *__restrict__ hist,
                                                   uint32_t *__restrict__ err) {
-  __shared__ uint32_t h[kMaxCoarse];
+  __shared__ uint32_t h[kMaxBuckets];
   const uint32_t tile = blockIdx.x;
   for (uint32_t b = threadIdx.x; b < Bc; b += blockDim.x) h[b] = 0;
   __syncthreads();
-  const uint32_t p0 = tile * kPartTile, p1 = min(N, p0 + kPartTile);
+  const uint32_t p0 = tile * ptile, p1 = min(N, p0 + ptile);
   int hint = 0;
   // kCnt records per thread loaded before any is used; the volume's
   // constants are read once per batch when the batch lies in one volume
@@ -530,7 +552,7 @@ __global__ __launch_bounds__(256) void k_pa_count(const uint8_t *__restrict__ ba
       const uint32_t p = q0 + threadIdx.x + k * 256;
       if (p < p1) {
         key[p] = c[k];
-        atomicAdd(&h[c[k] >> (kFineBits + 8)], 1u);
+        atomicAdd(&h[c[k] >> shift], 1u);
       }
     }
   }
@@ -612,25 +634,28 @@ __device__ __forceinline__ void staged_part(uint32_t nsub, const uint32_t (&kk)[
   __syncthreads();
 }
 
-// A, scatter: keys and {x,y,z,index} to the tile's slots of each coarse bucket.
+// A, scatter: keys and {x,y,z,index} to the tile's slots of each of at most
+// NB buckets.
+template <int NB>
 __global__ __launch_bounds__(kPartNT) void k_pa_scatter(const uint8_t *__restrict__ base,
                                                     uint32_t stride, uint32_t offpos, uint32_t N,
                                                     uint32_t Bc, uint32_t ntiles,
+                                                    uint32_t ptile, int shift,
                                                     const uint32_t *__restrict__ key,
                                                     const uint32_t *__restrict__ off,
                                                     uint32_t *__restrict__ okey,
                                                     float4 *__restrict__ opos) {
-  __shared__ uint32_t cur[kMaxCoarse], lcnt[kMaxCoarse], loff[kMaxCoarse];
+  __shared__ uint32_t cur[NB], lcnt[NB], loff[NB];
   __shared__ uint32_t skey[kSub], sbk[kSub];
   __shared__ float4 spos[kSub];
   __shared__ uint32_t ws[kPartNT / 64];
   const uint32_t tile = blockIdx.x;
-  for (uint32_t b = threadIdx.x; b < kMaxCoarse; b += blockDim.x) {
+  for (uint32_t b = threadIdx.x; b < NB; b += blockDim.x) {
     cur[b] = b < Bc ? off[(uint64_t)b * ntiles + tile] : 0u;
     lcnt[b] = 0;
   }
   __syncthreads();
-  const uint32_t p0 = tile * kPartTile, p1 = min(N, p0 + kPartTile);
+  const uint32_t p0 = tile * ptile, p1 = min(N, p0 + ptile);
   for (uint32_t q0 = p0; q0 < p1; q0 += kSub) {
     const uint32_t nsub = min((uint32_t)kSub, p1 - q0);
     uint32_t kk[kPer], bk[kPer];
@@ -643,16 +668,16 @@ __global__ __launch_bounds__(kPartNT) void k_pa_scatter(const uint8_t *__restric
         const uint32_t c = key[p];
         const float *fp = reinterpret_cast<const float *>(base + (uint64_t)p * stride + offpos);
         kk[k] = c;
-        bk[k] = c >> (kFineBits + 8);
+        bk[k] = c >> shift;
         pp[k] = make_float4(fp[0], fp[1], fp[2], __uint_as_float(p));
       }
     }
-    staged_part<kMaxCoarse>(nsub, kk, pp, bk, Bc, cur, lcnt, loff, skey, spos, sbk, ws, okey,
+    staged_part<NB>(nsub, kk, pp, bk, Bc, cur, lcnt, loff, skey, spos, sbk, ws, okey,
                             opos);
   }
 }
 
-// Coarse bucket starts (Bc + 1 entries) out of the scanned A histogram.
+// Pass A's bucket starts (Bc + 1 entries) out of its scanned histogram.
 __global__ void k_pa_starts(uint32_t Bc, uint32_t ntiles, const uint32_t *__restrict__ off,
                             uint32_t *__restrict__ cstart) {
   for (uint32_t b = blockIdx.x * blockDim.x + threadIdx.x; b <= Bc; b += gridDim.x * blockDim.x)
@@ -665,13 +690,14 @@ __global__ void k_pa_starts(uint32_t Bc, uint32_t ntiles, const uint32_t *__rest
 // kernels are launched for the most tiles the buckets can need
 // (ntiles_A + Bc) and the blocks past t0[Bc] do no work.
 __global__ __launch_bounds__(kMaxCoarse) void k_pb_tiles(uint32_t Bc, uint32_t ntmax,
+                                                         uint32_t ptile,
                                                          const uint32_t *__restrict__ cstart,
                                                          uint32_t *__restrict__ t0,
                                                          uint32_t *__restrict__ tinfo,
                                                          uint32_t *__restrict__ ntb) {
   __shared__ uint32_t ws[kMaxCoarse / 64];
   const uint32_t c = threadIdx.x, lane = c & 63, w = c >> 6;
-  const uint32_t nt = c < Bc ? (cstart[c + 1] - cstart[c] + kPartTile - 1) / kPartTile : 0u;
+  const uint32_t nt = c < Bc ? (cstart[c + 1] - cstart[c] + ptile - 1) / ptile : 0u;
   uint32_t inc = nt;
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) {
@@ -695,18 +721,20 @@ __global__ __launch_bounds__(kMaxCoarse) void k_pb_tiles(uint32_t Bc, uint32_t n
   }
   for (uint32_t t = tot + c; t < ntmax; t += blockDim.x) tinfo[t] = kNone;
 }
-__device__ __forceinline__ void pb_tile(uint32_t t, const uint32_t *__restrict__ tinfo,
+__device__ __forceinline__ void pb_tile(uint32_t t, uint32_t ptile,
+                                        const uint32_t *__restrict__ tinfo,
                                         const uint32_t *__restrict__ t0,
                                         const uint32_t *__restrict__ cstart, uint32_t &c,
                                         uint32_t &i0, uint32_t &i1, uint32_t &nt, uint32_t &k) {
   c = tinfo[t];
   k = t - t0[c];
   nt = t0[c + 1] - t0[c];
-  i0 = cstart[c] + k * kPartTile;
-  i1 = min(cstart[c + 1], i0 + kPartTile);
+  i0 = cstart[c] + k * ptile;
+  i1 = min(cstart[c + 1], i0 + ptile);
 }
 
-__global__ __launch_bounds__(256) void k_pb_count(const uint32_t *__restrict__ tinfo,
+__global__ __launch_bounds__(256) void k_pb_count(uint32_t ptile, int fb,
+                                                  const uint32_t *__restrict__ tinfo,
                                                   const uint32_t *__restrict__ t0,
                                                   const uint32_t *__restrict__ cstart,
                                                   const uint32_t *__restrict__ ikey,
@@ -717,16 +745,17 @@ __global__ __launch_bounds__(256) void k_pb_count(const uint32_t *__restrict__ t
     return;
   }
   uint32_t c, i0, i1, nt, k;
-  pb_tile(blockIdx.x, tinfo, t0, cstart, c, i0, i1, nt, k);
+  pb_tile(blockIdx.x, ptile, tinfo, t0, cstart, c, i0, i1, nt, k);
   h[threadIdx.x] = 0;
   __syncthreads();
   for (uint32_t i = i0 + threadIdx.x; i < i1; i += blockDim.x)
-    atomicAdd(&h[(ikey[i] >> kFineBits) & 255u], 1u);
+    atomicAdd(&h[(ikey[i] >> fb) & 255u], 1u);
   __syncthreads();
   hist[256ull * t0[c] + (uint64_t)threadIdx.x * nt + k] = h[threadIdx.x];
 }
 
-__global__ __launch_bounds__(kPartNT) void k_pb_scatter(const uint32_t *__restrict__ tinfo,
+__global__ __launch_bounds__(kPartNT) void k_pb_scatter(uint32_t ptile, int fb,
+                                                    const uint32_t *__restrict__ tinfo,
                                                     const uint32_t *__restrict__ t0,
                                                     const uint32_t *__restrict__ cstart,
                                                     const uint32_t *__restrict__ off,
@@ -740,7 +769,7 @@ __global__ __launch_bounds__(kPartNT) void k_pb_scatter(const uint32_t *__restri
   __shared__ uint32_t ws[kPartNT / 64];
   if (tinfo[blockIdx.x] == kNone) return;  // past the last tile
   uint32_t c, i0, i1, nt, k;
-  pb_tile(blockIdx.x, tinfo, t0, cstart, c, i0, i1, nt, k);
+  pb_tile(blockIdx.x, ptile, tinfo, t0, cstart, c, i0, i1, nt, k);
   for (uint32_t b = threadIdx.x; b < 256; b += kPartNT) {
     cur[b] = off[256ull * t0[c] + (uint64_t)b * nt + k];
     lcnt[b] = 0;
@@ -756,7 +785,7 @@ __global__ __launch_bounds__(kPartNT) void k_pb_scatter(const uint32_t *__restri
       // staged_part), so the arrays live in registers, not scratch
       const uint32_t i = min(threadIdx.x + q * kPartNT, nsub - 1);
       kk[q] = ikey[q0 + i];
-      bk[q] = (kk[q] >> kFineBits) & 255u;
+      bk[q] = (kk[q] >> fb) & 255u;
       const float4 v = ipos[q0 + i];
       pp[q] = make_float4(v.x, v.y, v.z, v.w);
     }
@@ -796,7 +825,8 @@ __device__ __forceinline__ int vol_of_cell(const VolDev *__restrict__ vols, int 
 constexpr int kPcThreads = 1024;
 constexpr uint32_t kPcListS = 1536, kPcListB = 512;
 
-__global__ __launch_bounds__(kPcThreads) void k_pc_sort(uint64_t C, const uint32_t *__restrict__ fstart,
+__global__ __launch_bounds__(kPcThreads) void k_pc_sort(uint64_t C, int fb,
+                                                 const uint32_t *__restrict__ fstart,
                                                  const uint32_t *__restrict__ ikey,
                                                  const float4 *__restrict__ ipos,
                                                  uint32_t *__restrict__ start,
@@ -816,16 +846,17 @@ __global__ __launch_bounds__(kPcThreads) void k_pc_sort(uint64_t C, const uint32
   __shared__ uint32_t nres[2], nfit[2], gbase[2];
   const uint32_t f = blockIdx.x;
   const uint32_t q0 = fstart[f], q1 = fstart[f + 1];
-  const uint64_t c0 = (uint64_t)f << kFineBits;
-  const uint32_t nc = (uint32_t)min((uint64_t)kFineCells, C - c0);
-  for (uint32_t e = threadIdx.x; e < kFineCells + kFineCells / 64 + 1; e += blockDim.x) lc[e] = 0;
+  const uint64_t c0 = (uint64_t)f << fb;
+  const uint32_t cells = 1u << fb;
+  const uint32_t nc = (uint32_t)min((uint64_t)cells, C - c0);
+  for (uint32_t e = threadIdx.x; e < cells + cells / 64 + 1; e += blockDim.x) lc[e] = 0;
   if (threadIdx.x < 2) nres[threadIdx.x] = 0, nfit[threadIdx.x] = threadIdx.x ? kPcListB : kPcListS;
   __syncthreads();
   for (uint32_t i = q0 + threadIdx.x; i < q1; i += blockDim.x)
-    atomicAdd(&lc[P(ikey[i] & (kFineCells - 1))], 1u);
+    atomicAdd(&lc[P(ikey[i] & (cells - 1))], 1u);
   __syncthreads();
-  // exclusive scan of the 2^14 counters: kPer consecutive per thread
-  constexpr uint32_t kPer = kFineCells / kPcThreads;
+  // exclusive scan of the 2^fb counters: kPer consecutive per thread
+  const uint32_t kPer = cells / kPcThreads;
   const uint32_t e0 = threadIdx.x * kPer;
   uint32_t loc = 0;
   for (uint32_t q = 0; q < kPer; q++) loc += lc[P(e0 + q)];
@@ -845,7 +876,7 @@ __global__ __launch_bounds__(kPcThreads) void k_pc_sort(uint64_t C, const uint32
     lc[P(e0 + q)] = pre;
     pre += v;
   }
-  if (threadIdx.x == kPcThreads - 1) lc[P(kFineCells)] = pre;  // bucket total
+  if (threadIdx.x == kPcThreads - 1) lc[P(cells)] = pre;  // bucket total
   __syncthreads();
   // one wave's dense cells of one kind: into the LDS list while it fits
   // (the fitting reservations are a prefix of the list), else appended
@@ -894,7 +925,7 @@ __global__ __launch_bounds__(kPcThreads) void k_pc_sort(uint64_t C, const uint32
   for (uint32_t k = threadIdx.x; k < nfit[1]; k += blockDim.x) dbig[gbase[1] + k] = lbig[k];
   // scatter with LDS cursors
   for (uint32_t i = q0 + threadIdx.x; i < q1; i += blockDim.x) {
-    const uint32_t slot = q0 + atomicAdd(&lc[P(ikey[i] & (kFineCells - 1))], 1u);
+    const uint32_t slot = q0 + atomicAdd(&lc[P(ikey[i] & (cells - 1))], 1u);
     pos4[slot] = ipos[i];
   }
 }
@@ -3456,7 +3487,9 @@ struct Plan {
   size_t vt_entries = 0;
   bool varlink = false;
   // dense grid partitions
-  uint32_t F = 0, Bc = 0, ntA = 0, ntBmax = 0;
+  uint32_t F = 0, Bc = 0, ntA = 0, ntBmax = 0, ptile = kPartTile;
+  int fb = kFineBits;      // log2 of the cells of a fine bucket
+  bool two_level = false;  // coarse buckets first (passes A and B)
   uint64_t nA = 0, nB = 0;
   uint64_t ndense_cap = 0, Hbound = 0, Hstage = 0;
   bool single_halos = false;  // some volume keeps groups of one (Nphalomin <= 1)
@@ -3616,11 +3649,14 @@ static int make_plan(const fof_particles_v1 *P, const fof_volume_v1 *vols, uint3
   pl.Hstage = std::min<uint64_t>(pl.Hbound, out->halo_cap);
   pl.tmpb = std::max(sort_tmp_bytes(N), compact_tmp_bytes(N));
   if (!pl.sparse) {
-    pl.F = (uint32_t)((pl.C + kFineCells - 1) >> kFineBits);
-    pl.Bc = (pl.F + 255) >> 8;
-    if (pl.Bc > (uint32_t)kMaxCoarse) return FOF_E_RANGE;
-    pl.ntA = (uint32_t)((N + kPartTile - 1) / kPartTile);
-    pl.ntBmax = pl.ntA + pl.Bc;
+    pl.ptile = part_tile(N);
+    pl.fb = fine_bits(pl.C);
+    pl.F = (uint32_t)((pl.C + (1u << pl.fb) - 1) >> pl.fb);
+    pl.two_level = pl.F > (uint32_t)kMaxBuckets;
+    pl.Bc = pl.two_level ? (pl.F + 255) >> 8 : pl.F;
+    if (pl.two_level && pl.Bc > (uint32_t)kMaxCoarse) return FOF_E_RANGE;
+    pl.ntA = (uint32_t)((N + pl.ptile - 1) / pl.ptile);
+    pl.ntBmax = pl.two_level ? pl.ntA + pl.Bc : 0;
     pl.nA = (uint64_t)pl.Bc * pl.ntA;
     pl.nB = 256ull * pl.ntBmax;
     pl.tmpb = std::max(pl.tmpb, scan_tmp_bytes(std::max(pl.nA, pl.nB) + 1));
@@ -3849,30 +3885,46 @@ static int enqueue_run(Run &r, hipStream_t st) {
     uint32_t *k1 = gsize, *k2 = label;     // free until the union-find finish / k_label
     float4 *p1 = pos4;                     // pass A output, consumed before pass C writes
     float4 *p2 = reinterpret_cast<float4 *>(sk0);
+    const uint32_t ptile = pl.ptile;
+    const int fb = pl.fb, shift = pl.two_level ? fb + 8 : fb;
     if ((rc = tb(0))) return rc;
-    k_pa_count<<<ntA, 256, 0, st>>>(dbase, stride, offpos, NN, dV, dVB, (int)nvol, Bc, ntA, key,
-                                    histA, small + kSmErr);
+    k_pa_count<<<ntA, 256, 0, st>>>(dbase, stride, offpos, NN, dV, dVB, (int)nvol, Bc, ntA, ptile,
+                                    shift, key, histA, small + kSmErr);
     FOF_HIP(hipGetLastError());
     if ((rc = te(0))) return rc;
     if ((rc = tb(1))) return rc;
     if ((rc = scan_u32(histA, offA, nA, B.tmp, st))) return rc;
-    k_pa_starts<<<grid_for(Bc + 1), 256, 0, st>>>(Bc, ntA, offA, cst);
+    uint32_t *starts = pl.two_level ? cst : fst;
+    k_pa_starts<<<grid_for(Bc + 1), 256, 0, st>>>(Bc, ntA, offA, starts);
     FOF_HIP(hipGetLastError());
-    k_pb_tiles<<<1, kMaxCoarse, 0, st>>>(Bc, ntBmax, cst, t0, tinfo, small + kSmNtB);
-    FOF_HIP(hipGetLastError());
+    if (pl.two_level) {
+      k_pb_tiles<<<1, kMaxCoarse, 0, st>>>(Bc, ntBmax, ptile, cst, t0, tinfo, small + kSmNtB);
+      FOF_HIP(hipGetLastError());
+    }
     if ((rc = te(1))) return rc;
     if ((rc = tb(2))) return rc;
-    k_pa_scatter<<<ntA, kPartNT, 0, st>>>(dbase, stride, offpos, NN, Bc, ntA, key, offA, k1, p1);
+    // one level: straight to pass C's input
+    uint32_t *ka = pl.two_level ? k1 : k2;
+    float4 *pa = pl.two_level ? p1 : p2;
+    if (Bc <= (uint32_t)kMaxCoarse)
+      k_pa_scatter<kMaxCoarse><<<ntA, kPartNT, 0, st>>>(dbase, stride, offpos, NN, Bc, ntA, ptile,
+                                                        shift, key, offA, ka, pa);
+    else
+      k_pa_scatter<kMaxBuckets><<<ntA, kPartNT, 0, st>>>(dbase, stride, offpos, NN, Bc, ntA, ptile,
+                                                         shift, key, offA, ka, pa);
     FOF_HIP(hipGetLastError());
-    k_pb_count<<<ntBmax, 256, 0, st>>>(tinfo, t0, cst, k1, histB);
-    FOF_HIP(hipGetLastError());
-    if ((rc = scan_u32(histB, offB, nB, B.tmp, st))) return rc;
-    k_pb_scatter<<<ntBmax, kPartNT, 0, st>>>(tinfo, t0, cst, offB, k1, p1, k2, p2);
-    FOF_HIP(hipGetLastError());
-    k_pb_starts<<<grid_for(F + 1), 256, 0, st>>>(F, t0, cst, offB, NN, fst);
-    FOF_HIP(hipGetLastError());
-    k_pc_sort<<<F, kPcThreads, 0, st>>>((uint64_t)pl.C, fst, k2, p2, start, pos4, dV, (int)nvol, T,
-                                        dense, small + kSmNDense, dbig, small + kSmNBig);
+    if (pl.two_level) {
+      k_pb_count<<<ntBmax, 256, 0, st>>>(ptile, fb, tinfo, t0, cst, k1, histB);
+      FOF_HIP(hipGetLastError());
+      if ((rc = scan_u32(histB, offB, nB, B.tmp, st))) return rc;
+      k_pb_scatter<<<ntBmax, kPartNT, 0, st>>>(ptile, fb, tinfo, t0, cst, offB, k1, p1, k2, p2);
+      FOF_HIP(hipGetLastError());
+      k_pb_starts<<<grid_for(F + 1), 256, 0, st>>>(F, t0, cst, offB, NN, fst);
+      FOF_HIP(hipGetLastError());
+    }
+    k_pc_sort<<<F, kPcThreads, 0, st>>>((uint64_t)pl.C, fb, fst, k2, p2, start, pos4, dV,
+                                        (int)nvol, T, dense, small + kSmNDense, dbig,
+                                        small + kSmNBig);
     FOF_HIP(hipGetLastError());
     if ((rc = te(2))) return rc;
   } else {

@@ -1,0 +1,60 @@
+"""The cell sort's ways over grid and particle counts: dense addressing (fine
+buckets of 2^11 to 2^14 cells, one or two partition levels, tiles of 1024
+particles upwards) against occupied-cell addressing, which sorts by another
+method.  Bar: every output bit-identical."""
+import numpy as np
+import pytest
+
+from cm_halofinder_amd import _lib as L
+
+pytestmark = pytest.mark.gpu
+
+
+def linked(ctx, P, n, dom, flags):
+    import torch
+
+    v = L.Volume()
+    v.offset, v.n, v.domain = 0, n, dom
+    nxt = torch.zeros(n, dtype=torch.int32, device="cuda")
+    lab = torch.zeros(n, dtype=torch.int32, device="cuda")
+    hal = torch.zeros((n // 2 + 1, 8), dtype=torch.float64, device="cuda")
+    st = L.Stats()
+    rc, nh = ctx.link_ex(L.particles(P, n), [v], L.opts(flags), nxt, lab, None, hal, None,
+                         n // 2 + 1, None, st)
+    L.check(rc)
+    return nxt, lab, hal.view(torch.int32), nh, st
+
+
+# cells per axis (lcell = 1): one bucket; 255, 256 and 257 buckets of 2^11;
+# 512 and 513 of 2^14; 1280 (one level) and 1284 (two levels)
+@pytest.mark.parametrize("grid,n", [
+    ((2, 2, 2), 1), ((16, 16, 8), 1023), ((16, 16, 8), 1025), ((64, 64, 127), 200001),
+    ((64, 64, 128), 2049), ((65, 64, 128), 70000), ((256, 256, 128), 1500000),
+    ((256, 256, 64), 1048577), ((256, 256, 129), 1500001), ((256, 256, 320), 5700000), ((256, 256, 321), 5800001)])
+def test_dense_sort_matches_occupied_cells(ctx, grid, n):
+    import torch
+
+    print("grid", grid, "n", n, flush=True)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(n)
+    ext = torch.tensor([float(c - 1) for c in grid], device="cuda")
+    rec = torch.zeros((n, 8), dtype=torch.float32, device="cuda")
+    pos = torch.rand((n, 3), generator=g, device="cuda") * ext
+    # a third of them gathered near a few points, some on the upper faces
+    k = n // 3
+    cen = torch.rand((17, 3), generator=g, device="cuda") * ext
+    who = torch.randint(0, 17, (k,), generator=g, device="cuda")
+    pos[:k] = cen[who] + torch.randn((k, 3), generator=g, device="cuda")
+    pos[: k // 50] = ext
+    rec[:, 2:5] = torch.minimum(pos.clamp_min(0.0), ext)
+    rec[:, 5:8] = torch.randn((n, 3), generator=g, device="cuda")
+    rec = rec[torch.randperm(n, generator=g, device="cuda")].contiguous()
+    hi = [float(c - 1) for c in grid]
+    dom = L.domain([0] * 3, hi, [0] * 3, hi, [1.0] * 3, 0.2, 2)
+    a = linked(ctx, rec, n, dom, 0)
+    b = linked(ctx, rec, n, dom, L.OPT_SPARSE)
+    assert a[4].sparse == 0 and b[4].sparse == 1
+    assert a[4].ncells == int(np.prod(grid))
+    assert a[3] == b[3]
+    for x, y in zip(a[:3], b[:3]):
+        assert torch.equal(x, y)
