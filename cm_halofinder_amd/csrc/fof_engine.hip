@@ -393,6 +393,15 @@ __device__ __forceinline__ uint32_t uf_join(uint32_t *par, uint32_t rx, uint32_t
   }
 }
 
+// LDS written by some lanes of a wave and read by others afterwards: the
+// wave's LDS operations execute in order; this keeps the compiler from
+// moving them across.
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Statistics counters are spread over kCtrSlots copies, one 128-byte line
 // each, picked by workgroup: a million waves adding to one address serialise
 // at one L2 channel.  The host sums the copies.  Counter k of a slot:
@@ -431,7 +440,6 @@ constexpr int kSmErr = 0;       // bit 0: particle outside [rmin_buff, rmax_buff
 constexpr int kSmNDense = 1;    // dense cells below kBigCell particles
 constexpr int kSmM = 2;         // members of groups of two or more (member list)
 constexpr int kSmH = 3;         // halos
-constexpr int kSmOverflow = 4;  // run-table overflow
 constexpr int kSmU = 5;         // occupied cells (sparse addressing)
 constexpr int kSmNBig = 7;      // dense cells from kBigCell particles
 constexpr int kSmR = 8;         // groups of two or more (their roots)
@@ -1400,43 +1408,6 @@ __device__ __forceinline__ void lunion(volatile uint32_t *lp, uint32_t a, uint32
   }
 }
 
-// Any linking pair between two runs (both cliques)?  Early exit.  Partner
-// positions are loaded two at a time: the dense kernels run at 6-8 waves per
-// SIMD, where wider batches cost more in registers than they hide latency.
-__device__ __forceinline__ bool runs_link(const float4 *__restrict__ pos4, uint32_t ha,
-                                          uint32_t ea, uint32_t hb, uint32_t eb, const Rule &R,
-                                          uint32_t &tests, uint32_t &rechecks) {
-  if (ea == ha + 1 && eb == hb + 1) {  // two single particles: both loads at once
-    const float4 a = pos4[ha], b = pos4[hb];
-    tests++;
-    return pair_linked(a, b, R, rechecks);
-  }
-  for (uint32_t i = ha; i < ea; i++) {
-    const float4 pi = pos4[i];
-    uint32_t j = hb;
-    for (; j + 2 <= eb; j += 2) {
-      float4 q[2];
-#pragma unroll
-      for (int k = 0; k < 2; k++) q[k] = ld4(pos4 + j + k);
-      bool any = false;
-#pragma unroll
-      for (int k = 0; k < 2; k++) any |= pair_linked(pi, q[k], R, rechecks);
-      tests += 2;
-      if (any) return true;
-    }
-    for (; j < eb; j++) {
-      tests++;
-      if (pair_linked(pi, pos4[j], R, rechecks)) return true;
-    }
-  }
-  return false;
-}
-
-// Run pairs with more than BIGPAIR particle pairs (a template parameter of
-// k_link_dense) are queued in LDS and tested by 16-lane groups: 16 particle
-// pairs per step, ballot exit.  Smaller pairs are tested in place by the
-// thread that found them.
-
 // Home-cell sub-cell coordinates (0..11) packed 4 bits per axis.
 __device__ __forceinline__ uint16_t pack_home(int x, int y, int z) {
   return (uint16_t)(x | (y << 4) | (z << 8));
@@ -1444,10 +1415,9 @@ __device__ __forceinline__ uint16_t pack_home(int x, int y, int z) {
 
 // Cells with more runs than this enumerate candidates through a bitmap of
 // A's occupied sub-cells, one x-row of the window at a time; cells with fewer
-// test every run pair.  The 256-thread kernel walks the window twice: first
-// the sub-cells that touch the run's own (|offset| <= 1 on every axis), whose
-// pairs link most often, so that their merges prune the second walk over the
-// rest.
+// test every run pair.  The window is walked twice: first the sub-cells that
+// touch the run's own (|offset| <= 1 on every axis), whose pairs link most
+// often, so that their merges prune the second walk over the rest.
 constexpr int kMapRuns = 24;
 
 // 0, 1, -1, 2, -2, ...: window rows visited from the centre out.
@@ -1466,14 +1436,44 @@ __device__ __forceinline__ void nb_offset(int k, int dd[3]) {
 }
 
 // Bytes of dynamic LDS for ra home-run slots and MAXRUNSB neighbour slots:
-// ahead, agr, lp (ra + MAXRUNSB), arel (u16).
+// ahead (and the cell's end), agr, lp (ra + MAXRUNSB), arel (u16).
 constexpr size_t dense_lds(uint32_t ra, uint32_t maxrunsb) {
-  return 4 * ((size_t)3 * ra + maxrunsb) + 2 * (size_t)ra + 8;
+  return 4 * ((size_t)3 * ra + 1 + maxrunsb) + 2 * (size_t)ra + 8;
+}
+
+// a / d for a < 2^23 (inv = 1 / d in float): the quotient in float is off by
+// at most one.
+__device__ __forceinline__ uint32_t div_small(uint32_t a, uint32_t d, float inv) {
+  uint32_t q = (uint32_t)((float)a * inv);
+  const uint32_t r = a - q * d;
+  if ((int)r < 0) q--;
+  else if (r >= d) q++;
+  return q;
 }
 
 // WPE: waves per SIMD to fit (the register budget; LDS per workgroup is
 // sized at launch to the runs a cell of the batch can have).
-template <int NT, int WPE, int MAXRUNS, int MAXRUNSB, int BIGQ, int ROUND, uint32_t BIGPAIR>
+//
+// The cell's data (run heads, window bitmaps, union-find) is shared by the
+// workgroup; the waves take 64 slots at a time -- (row of the window, run) or
+// (row, neighbour item) -- from a counter in LDS and work on their own: a lane
+// walks its row's occupied sub-cells, candidate pairs not yet joined go to the
+// wave's queue, and 64 queued pairs are tested together, a lane each (the
+// first kTile x kTile particles, which settles nearly all), what is left by
+// 16-lane groups.  Enumerating reads no global memory and no barrier stands
+// between enumerating and testing.
+//
+// What bounds it: one cell's chain of dependent steps while there are few
+// cells, VALU issue and latency (LDS finds, positions) when many.  Before, the
+// workgroup went through rounds of 768 slots, tested single pairs where they
+// were found and drained a common queue four pairs a wave at a time, each
+// behind two walks of the global union-find: the kernel took 630 us for the
+// 64^3 box (132 cells), 2.88 ms for 256^3 and 7.25 ms for 512^3; now 264, 773
+// and 3.43.  Walking whole rows first instead of the touching sub-cells made
+// half as many pairs again (30 against 15 G cycles at 512^3).  Six waves per
+// SIMD: at eight (64 registers) the spills doubled the cycles per cell, five
+// was 10% slower.
+template <int NT, int WPE, int MAXRUNS, int MAXRUNSB>
 __global__ __launch_bounds__(NT, WPE) void k_link_dense(const uint32_t *__restrict__ dense,
                                                     const uint32_t *__restrict__ ndense,
                                                     const float4 *__restrict__ pos4,
@@ -1488,15 +1488,14 @@ __global__ __launch_bounds__(NT, WPE) void k_link_dense(const uint32_t *__restri
                                                     const uint32_t *__restrict__ vbeg,
                                                     int nvol,
                                                     unsigned long long *__restrict__ ctr,
-                                                    uint32_t *__restrict__ overflow,
                                                     uint32_t ra, uint32_t *__restrict__ dq) {
   // per-run slots of the home cell (ra <= MAXRUNS of them: the most
   // sub-cells of a cell in the batch), in dynamic LDS
   extern __shared__ uint32_t dyn[];
-  uint32_t *const ahead = dyn, *const agr = dyn + ra, *const lp = dyn + 2 * ra;
-  uint16_t *const arel = reinterpret_cast<uint16_t *>(dyn + 3 * ra + MAXRUNSB);
+  uint32_t *const ahead = dyn, *const agr = dyn + ra + 1, *const lp = dyn + 2 * ra + 1;
+  uint16_t *const arel = reinterpret_cast<uint16_t *>(dyn + 3 * ra + 1 + MAXRUNSB);
   __shared__ uint32_t bhead[MAXRUNSB], brel[MAXRUNSB], bgr[MAXRUNSB];
-  __shared__ uint32_t bigq[BIGQ];
+  __shared__ uint32_t wq[NT / 64][128];  // the waves' queues of pairs to test
   // occupied sub-cells of A (<= 12^3) and the occupied count before each
   // word: A's runs are listed in sub-cell order, so the run slot of an
   // occupied sub-cell is its rank in the bitmap
@@ -1511,9 +1510,11 @@ __global__ __launch_bounds__(NT, WPE) void k_link_dense(const uint32_t *__restri
   __shared__ uint32_t mainr;
   __shared__ uint32_t nbS[26], nbOff[27];
   __shared__ uint8_t nbDense[26];
-  __shared__ uint32_t cnt, qn, dnext;
+  __shared__ uint32_t cntx, cnty, slots[3], dnext;
   uint32_t tests = 0, rechecks = 0, joined = 0;
   const uint32_t lane = threadIdx.x & 63;
+  const unsigned long long lt = (1ull << lane) - 1;
+  uint32_t *const wqw = wq[__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6))];
   const uint32_t nd = *ndense;
   // cells are taken from a queue (*dq, zero at launch) one at a time: their
   // costs differ by orders of magnitude, and a fixed share per workgroup
@@ -1576,13 +1577,16 @@ __global__ __launch_bounds__(NT, WPE) void k_link_dense(const uint32_t *__restri
       if (k < 26) nbOff[k + 1] = items;
       if (k == 0) nbOff[0] = 0;
     }
-    if (threadIdx.x == 0) qn = 0, mainr = kNone;
-    if (threadIdx.x < kOccW) occ[threadIdx.x] = 0, smap[threadIdx.x] = 0;
-    __syncthreads();
-    const int wy = 2 * reach[1] + 1;
     // the home cell's runs (one per occupied sub-cell, in sub-cell order)
     // from its run table; runs <= min(particles, sub-cells) <= ra
     const int na = (int)rtoff[sA];
+    if (threadIdx.x == 0) {
+      mainr = kNone, slots[0] = slots[1] = 0;
+      ahead[na] = G.start[c + 1];  // runs follow one another: each ends where the next begins
+    }
+    if (threadIdx.x < kOccW) occ[threadIdx.x] = 0, smap[threadIdx.x] = 0;
+    __syncthreads();
+    const int wy = 2 * reach[1] + 1, wz = 2 * reach[2] + 1;
     for (uint32_t k = threadIdx.x; k < (uint32_t)na; k += blockDim.x) {
       const uint32_t j = rtab[sA + k];
       const unsigned long long f = fine[j];
@@ -1623,136 +1627,184 @@ __global__ __launch_bounds__(NT, WPE) void k_link_dense(const uint32_t *__restri
     const bool bmap = na > kMapRuns;
     // bits of x in [c - 1, c + 1] for a row starting at x0, given s = c - 1 - x0
     auto touchbits = [](int s) -> uint32_t { return s >= 0 ? 7u << s : 7u >> -s; };
-    // a run pair (LDS slots sa, sb with heads ha, hb) not yet joined: small
-    // pairs are tested here, big ones go to the wave queue
-    auto test_pair = [&](uint32_t sa, uint32_t sb, uint32_t ha, uint32_t hb) {
-      const uint32_t ea = run_end[ha], eb = run_end[hb];
-      if ((ea - ha) * (eb - hb) > BIGPAIR) {
-        const uint32_t q = atomicAdd(&qn, 1u);
-        if (q < (uint32_t)BIGQ) {
-          bigq[q] = (sa << 16) | sb;
-          return;
-        }
+    // the run of an LDS slot: particles [h, h + n)
+    auto run_of = [&](uint32_t sl, uint32_t &h, uint32_t &n) {
+      if (sl < (uint32_t)na) {
+        h = ahead[sl], n = ahead[sl + 1] - h;
+      } else {
+        h = bhead[sl - na], n = brel[sl - na] >> 24;
+        if (n == 255) n = run_end[h] - h;  // the packed size saturates
       }
-      if (runs_link(pos4, ha, ea, hb, eb, R, tests, rechecks)) lunion(lp, sa, sb);
     };
-    // the queued pairs, four per wave (16-lane groups): skip when joined in
-    // LDS, join when under the same global root now, else a group-wide test
-    auto drain = [&]() {
-      __syncthreads();
-      const uint32_t nq = min(qn, (uint32_t)BIGQ);
-      const uint32_t grp = lane >> 4, gl = lane & 15;
-      for (uint32_t k0 = (threadIdx.x >> 6) * 4; k0 < nq; k0 += (blockDim.x >> 6) * 4) {
-        const uint32_t k = k0 + grp;
-        uint32_t sa = 0, sb = 0, ha = 0, hb = 0;
-        if (k < nq) {
-          const uint32_t e = bigq[k];
-          sa = e >> 16, sb = e & 0xFFFFu;
-          ha = ahead[sa], hb = sb < (uint32_t)na ? ahead[sb] : bhead[sb - na];
+    uint32_t qn = 0;  // pairs in the wave's queue (uniform)
+    // test the last m (<= 64) queued pairs of LDS slots, a lane each
+    constexpr uint32_t kTile = 4;
+    auto flush = [&](uint32_t m) {
+      wave_sync();
+      qn -= m;
+      uint32_t sa = 0, sb = 0, ha = 0, hb = 0, n1 = 0, n2 = 0;
+      bool live = lane < m, link = false;
+      if (live) {
+        const uint32_t e = wqw[qn + lane];
+        sa = e >> 16, sb = e & 0xFFFFu;
+        if (lfind(lp, sa) == lfind(lp, sb)) live = false, joined++;
+      }
+      if (live) {
+        run_of(sa, ha, n1), run_of(sb, hb, n2);
+        const uint32_t t1 = min(n1, kTile), t2 = min(n2, kTile);
+        float4 a[kTile];
+#pragma unroll
+        for (uint32_t k = 0; k < kTile; k++) a[k] = ld4(pos4 + ha + min(k, t1 - 1));
+        for (uint32_t j = 0; j < t2 && !link; j++) {
+          const float4 q = ld4(pos4 + hb + j);
+#pragma unroll
+          for (uint32_t k = 0; k < kTile; k++) link |= pair_linked(a[k], q, R, rechecks);
+          tests += t1;
         }
-        uint32_t v = 2u;  // 2: nothing to do, 1: join, 0: test
-        if (k < nq && gl == 0) {
-          if (lfind(lp, sa) != lfind(lp, sb)) v = (uf_find(par, ha) == uf_find(par, hb)) ? 1u : 0u;
-          joined += (v != 0u) ? 1u : 0u;
+        if (link) lunion(lp, sa, sb);
+      }
+      // pairs with more particles, not linked so far: four at a time
+      unsigned long long rest = __ballot(live && !link && (n1 > kTile || n2 > kTile));
+      const uint32_t gl = lane & 15;
+      while (rest) {
+        uint32_t src = 0;  // the group's pair: the grp-th set bit
+        unsigned long long left = rest;
+        bool mine = false;
+#pragma unroll
+        for (uint32_t g = 0; g < 4; g++) {
+          if (left) {
+            const uint32_t l = (uint32_t)__builtin_ctzll(left);
+            left &= left - 1;
+            if (g == (lane >> 4)) src = l, mine = true;
+          }
         }
-        v = __shfl(v, lane & ~15u, 64);
-        const uint32_t sza = v == 0u ? run_end[ha] - ha : 0u;
-        const uint32_t szb = v == 0u ? run_end[hb] - hb : 1u;
-        const uint32_t total = sza * szb;
-        bool linked = (v == 1u), done = (v != 0u);
-        for (uint32_t base = 0;; base += 16) {
+        rest = left;
+        const uint32_t xa = __shfl(sa, src, 64), xb = __shfl(sb, src, 64);
+        const uint32_t ga = __shfl(ha, src, 64), gb = __shfl(hb, src, 64);
+        const uint32_t m1 = __shfl(n1, src, 64), m2 = __shfl(n2, src, 64);
+        // joined by now?  (the group's first lane asks: one answer a group)
+        bool done = !mine;
+        if (mine && gl == 0) done = lfind(lp, xa) == lfind(lp, xb);
+        done = __shfl((int)done, lane & ~15u, 64) != 0;
+        if (mine && done && gl == 0) joined++;
+        const uint32_t total = done ? 0u : m1 * m2;
+        bool hit = false;
+        for (uint32_t base = 0;; base += 32) {
           bool l = false;
-          const uint32_t idx = base + gl;
-          if (!done && idx < total) {
-            const uint32_t i = idx / szb, j = idx - i * szb;
-            l = pair_linked(pos4[ha + i], pos4[hb + j], R, rechecks);
-            tests++;
+#pragma unroll
+          for (uint32_t k = 0; k < 32; k += 16) {
+            const uint32_t idx = base + k + gl;
+            if (!done && idx < total) {
+              const uint32_t i = idx / m2;
+              l |= pair_linked(pos4[ga + i], pos4[gb + idx - i * m2], R, rechecks);
+              tests++;
+            }
           }
           const uint32_t gbits = (uint32_t)(__ballot(l) >> (lane & ~15u)) & 0xFFFFu;
-          if (!done && gbits) linked = true, done = true;
-          if (base + 16 >= total) done = true;
+          if (!done && gbits) hit = true, done = true;
+          if (base + 32 >= total) done = true;
           if (!__ballot(!done)) break;
         }
-        if (linked && gl == 0) lunion(lp, sa, sb);
+        if (hit && gl == 0) lunion(lp, xa, xb);
       }
-      __syncthreads();
-      if (threadIdx.x == 0) {
-        qn = 0;
-        if (mainr != kNone) mainr = lfind(lp, mainr);  // merges may hook it
-      }
-      __syncthreads();
+      wave_sync();
     };
-    // a candidate pair of slots: skip if joined, join on equal snapshots,
-    // else test
-    auto consider = [&](uint32_t sa, uint32_t sb, uint32_t ga, uint32_t gb, uint32_t ha,
-                        uint32_t hb) {
-      if (lfind(lp, sa) == lfind(lp, sb)) {
-        joined++;
-        return;
+    // one candidate a lane (all lanes call): a pair of slots not joined yet
+    // is joined on equal snapshots of the global roots, else queued
+    auto offer = [&](bool any, uint32_t sa, uint32_t sb, uint32_t ga, uint32_t gb) {
+      bool want = false;
+      if (any) {
+        if (lfind(lp, sa) == lfind(lp, sb)) {
+          joined++;
+        } else if (ga == gb) {
+          joined++;
+          lunion(lp, sa, sb);
+        } else {
+          want = true;
+        }
       }
-      if (ga == gb) {
-        joined++;
-        lunion(lp, sa, sb);
-      } else {
-        test_pair(sa, sb, ha, hb);
+      const unsigned long long bal = __ballot(want);
+      if (want) wqw[qn + (uint32_t)__popcll(bal & lt)] = (sa << 16) | sb;
+      qn += (uint32_t)__popcll(bal);
+      if (qn >= 64) flush(64);
+    };
+    // the wave's next 64 slots of a phase (its first)
+    auto take = [&](int ph) -> uint32_t {
+      uint32_t p = 0;
+      if (lane == 0) p = atomicAdd(&slots[ph], 64u);
+      return (uint32_t)__builtin_amdgcn_readfirstlane((int)p);
+    };
+    // the occupied sub-cells `bits` (of `all`, from x0, first slot r0) of a
+    // lane's row against its run or item: offset dxo from it in x
+    auto walk = [&](uint32_t bits, uint32_t all, uint32_t r0, int x0, int bx, int dy, int dz,
+                    uint32_t other, uint32_t gother) {
+      while (__ballot(bits != 0)) {
+        bool any = false;
+        uint32_t sa = 0, sb = 0, ga = 0, gb = 0;
+        if (bits) {
+          const int b = __builtin_ctz(bits);
+          bits &= bits - 1;
+          if (gap_ok(x0 + b - bx, dy, dz)) {
+            const uint32_t ia = r0 + __popc(all & ((1u << b) - 1));
+            any = true;
+            sa = min(ia, other), sb = max(ia, other);
+            ga = agr[ia], gb = gother;
+          }
+        }
+        offer(any, sa, sb, ga, gb);
       }
     };
-    // (A, A), in rounds each followed by a drain, so that merges found early
-    // prune the later rounds (a full queue falls back to testing in place)
+    // (A, A)
+    const float ina = 1.0f / (float)na;
     if (bmap) {
-      // items (row of the forward window, run), row-major, rows centre-out;
+      // slots (row of the forward window, run), row-major, rows centre-out;
       // the first walk (touching sub-cells: the 5 forward rows at |dy|, dz
       // <= 1) before the second (every forward row)
       const int ry = reach[1], rz = reach[2];
       const uint32_t nrow1 = 5, nrow2 = (uint32_t)(ry + 1 + rz * wy);
-      auto aa_items = [&](bool first) {
-      const uint32_t to = (first ? nrow1 : nrow2) * (uint32_t)na;
-      for (uint32_t base = 0; base < to; base += ROUND) {
-        const uint32_t pe = min(to, base + (uint32_t)ROUND);
-        const bool masked = mainr != kNone;
-        for (uint32_t p = base + threadIdx.x; p < pe; p += blockDim.x) {
-          const uint32_t r2 = p / (uint32_t)na, ia = p - r2 * (uint32_t)na;
-          int dz, dy;
-          if (first) {
-            dz = r2 < 2 ? 0 : 1;
-            dy = zig((int)(r2 < 2 ? r2 : r2 - 2));
-          } else if (r2 <= (uint32_t)ry) {
-            dz = 0;
-            dy = (int)r2;
-          } else {
-            const uint32_t t = r2 - (uint32_t)(ry + 1);
-            dz = 1 + (int)(t / (uint32_t)wy);
-            dy = zig((int)(t % (uint32_t)wy));
+      auto aa_slots = [&](bool first) {
+        const uint32_t to = (first ? nrow1 : nrow2) * (uint32_t)na;
+        for (uint32_t p0 = take(first ? 0 : 1); p0 < to; p0 = take(first ? 0 : 1)) {
+          const uint32_t p = p0 + lane;
+          uint32_t bits = 0, all = 0, r0 = 0, ia = 0;
+          int x0 = 0, ax = 0, dy = 0, dz = 0;
+          if (p < to) {
+            const uint32_t r2 = div_small(p, (uint32_t)na, ina);
+            ia = p - r2 * (uint32_t)na;
+            if (first) {
+              dz = r2 < 2 ? 0 : 1;
+              dy = zig((int)(r2 < 2 ? r2 : r2 - 2));
+            } else if (r2 <= (uint32_t)ry) {
+              dy = (int)r2;
+            } else {
+              const uint32_t t = r2 - (uint32_t)(ry + 1);
+              dz = 1 + (int)(t / (uint32_t)wy);
+              dy = zig((int)(t % (uint32_t)wy));
+            }
+            const bool trow = dz <= 1 && dy >= -1 && dy <= 1;
+            const uint32_t rr = arel[ia];
+            const int ay = (rr >> 4) & 15, az = rr >> 8;
+            ax = rr & 15;
+            const int by = ay + dy, bz = az + dz;
+            x0 = (dz == 0 && dy == 0) ? ax + 1 : max(ax - reach[0], 0);
+            const int x1 = min(ax + reach[0], mm[0] - 1);
+            if (bz < mm[2] && by >= 0 && by < mm[1] && x0 <= x1 && gap_ok(0, dy, dz)) {
+              const int bin0 = (bz * mm[1] + by) * mm[0] + x0;
+              bits = all = rowbits(bin0, x1 - x0 + 1);
+              r0 = rank(bin0);
+              if (trow) bits &= first ? touchbits(ax - 1 - x0) : ~touchbits(ax - 1 - x0);
+              if (!first && mainr != kNone) {  // a run of the dominant set: only the stragglers
+                const int abin = (az * mm[1] + ay) * mm[0] + ax;
+                if (!((smap[abin >> 6] >> (abin & 63)) & 1ull)) bits &= srowbits(bin0, x1 - x0 + 1);
+              }
+            }
           }
-          const bool trow = dz <= 1 && dy >= -1 && dy <= 1;
-          const uint32_t ra = arel[ia];
-          const int ax = ra & 15, ay = (ra >> 4) & 15, az = ra >> 8;
-          const int by = ay + dy, bz = az + dz;
-          if (bz >= mm[2] || by < 0 || by >= mm[1] || !gap_ok(0, dy, dz)) continue;
-          const int x0 = (dz == 0 && dy == 0) ? ax + 1 : max(ax - reach[0], 0);
-          const int x1 = min(ax + reach[0], mm[0] - 1);
-          if (x0 > x1) continue;
-          const int bin0 = (bz * mm[1] + by) * mm[0] + x0;
-          const uint32_t all = rowbits(bin0, x1 - x0 + 1), r0 = rank(bin0);
-          uint32_t bits = all;
-          if (trow) bits &= first ? touchbits(ax - 1 - x0) : ~touchbits(ax - 1 - x0);
-          if (masked) {  // a run of the dominant set: only the stragglers
-            const int abin = (az * mm[1] + ay) * mm[0] + ax;
-            if (!((smap[abin >> 6] >> (abin & 63)) & 1ull)) bits &= srowbits(bin0, x1 - x0 + 1);
-          }
-          while (bits) {
-            const int b = __builtin_ctz(bits);
-            bits &= bits - 1;
-            if (!gap_ok(x0 + b - ax, dy, dz)) continue;
-            const uint32_t ib = r0 + __popc(all & ((1u << b) - 1));
-            const uint32_t s0 = min(ia, ib), s1 = max(ia, ib);
-            consider(s0, s1, agr[s0], agr[s1], ahead[s0], ahead[s1]);
-          }
+          walk(bits, all, r0, x0, ax, dy, dz, ia, p < to ? agr[ia] : 0u);
         }
-        drain();
-      }
+        if (qn) flush(qn);
+        __syncthreads();
       };
-      aa_items(true);
+      aa_slots(true);
       // the dominant set: a vote of 64 runs spread over the cell (wave 0);
       // kept when it holds at least a quarter of them
       if (threadIdx.x < 64) {
@@ -1778,29 +1830,29 @@ __global__ __launch_bounds__(NT, WPE) void k_link_dense(const uint32_t *__restri
           }
       }
       __syncthreads();
-      aa_items(false);
+      aa_slots(false);
     } else {
       const uint32_t total = (uint32_t)na * (uint32_t)na;  // na <= kMapRuns
-      for (uint32_t base = 0; base < total; base += ROUND) {
-        const uint32_t pe = min(total, base + (uint32_t)ROUND);
-        for (uint32_t p = base + threadIdx.x; p < pe; p += blockDim.x) {
-          const uint32_t ia = p / (uint32_t)na, ib = p - ia * (uint32_t)na;
-          if (ib <= ia) continue;
-          const uint32_t ra = arel[ia], rb = arel[ib];
-          if (!gap_ok((int)(rb & 15) - (int)(ra & 15),
-                      (int)((rb >> 4) & 15) - (int)((ra >> 4) & 15),
-                      (int)(rb >> 8) - (int)(ra >> 8)))
-            continue;
-          consider(ia, ib, agr[ia], agr[ib], ahead[ia], ahead[ib]);
+      for (uint32_t p0 = take(0); p0 < total; p0 = take(0)) {
+        const uint32_t p = p0 + lane;
+        const uint32_t ia = div_small(p, (uint32_t)na, ina), ib = p - ia * (uint32_t)na;
+        bool any = p < total && ib > ia;
+        if (any) {
+          const uint32_t rra = arel[ia], rrb = arel[ib];
+          any = gap_ok((int)(rrb & 15) - (int)(rra & 15),
+                       (int)((rrb >> 4) & 15) - (int)((rra >> 4) & 15),
+                       (int)(rrb >> 8) - (int)(rra >> 8));
         }
-        drain();
+        offer(any, ia, ib, any ? agr[ia] : 0u, any ? agr[ib] : 0u);
       }
+      if (qn) flush(qn);
+      __syncthreads();
     }
     // (A, B): the neighbours' items in chunks of MAXRUNSB
     const uint32_t ntot = nbOff[26];
     for (uint32_t c0 = 0; c0 < ntot; c0 += MAXRUNSB) {
       const uint32_t c1 = min(ntot, c0 + (uint32_t)MAXRUNSB);
-      if (threadIdx.x == 0) cnt = 0;
+      if (threadIdx.x == 0) cntx = cnty = slots[2] = 0;
       __syncthreads();
       for (uint32_t g = c0 + threadIdx.x; g < c1; g += blockDim.x) {
         int q = 0, qh = 25;  // the last neighbour whose items start at or before g
@@ -1812,8 +1864,10 @@ __global__ __launch_bounds__(NT, WPE) void k_link_dense(const uint32_t *__restri
         const uint32_t item = g - nbOff[q];
         const uint32_t j = nbDense[q] ? rtab[nbS[q] + item] : nbS[q] + item;
         int fx, fy, fz;
+        uint32_t len = 1;
         if (nbDense[q]) {
           const unsigned long long f = fine[j];
+          len = min(run_end[j] - j, 255u);
           fx = fine_x(f), fy = fine_y(f), fz = fine_z(f);
         } else {
           const float4 pj = pos4[j];
@@ -1828,69 +1882,88 @@ __global__ __launch_bounds__(NT, WPE) void k_link_dense(const uint32_t *__restri
         for (int a = 0; a < 3; a++)
           far |= (dd[a] == 1 && rr[a] > mm[a] - 1 + reach[a]) || (dd[a] == -1 && rr[a] < -reach[a]);
         if (far) continue;
-        const int rx = rr[0], ry = rr[1], rz = rr[2];
-        const uint32_t k = atomicAdd(&cnt, 1u);  // < MAXRUNSB: one per item at most
+        // the x neighbours' items from the front, the others' from the back
+        // (MAXRUNSB items at most)
+        const uint32_t k = dd[1] == 0 && dd[2] == 0 ? atomicAdd(&cntx, 1u)
+                                                    : MAXRUNSB - 1 - atomicAdd(&cnty, 1u);
         bhead[k] = j;
-        brel[k] = pack_rel(rx, ry, rz);
+        brel[k] = pack_rel(rr[0], rr[1], rr[2]) | len << 24;
         bgr[k] = uf_find(par, j);
         lp[na + k] = na + k;
       }
       __syncthreads();
-      const uint32_t nb = cnt;
-      // every (home run, neighbour item) pair within reach, in rounds
+      const uint32_t nbx = cntx, nb = nbx + cnty;
+      // slot of the chunk's item j
+      auto item = [&](uint32_t j) -> uint32_t { return j < nbx ? j : MAXRUNSB - 1 - (j - nbx); };
+      const float inb = 1.0f / (float)max(nb, 1u), inbx = 1.0f / (float)max(nbx, 1u);
+      // every (home run, neighbour item) pair within reach
       if (bmap) {
-        // items (row of the window, item), row-major, rows centre-out: the
-        // 9 touching rows (touching sub-cells) first, then every row
-        const uint32_t nrow = (uint32_t)((2 * reach[2] + 1) * wy);
-        const uint32_t total = (9 + nrow) * nb;
-        for (uint32_t base = 0; base < total; base += ROUND) {
-          const uint32_t pe = min(total, base + (uint32_t)ROUND);
-          const uint32_t mr = mainr;
-          for (uint32_t p = base + threadIdx.x; p < pe; p += blockDim.x) {
-            const uint32_t r2 = p / nb, jb = p - r2 * nb;
-            const bool first = r2 < 9;
-            const uint32_t ri = first ? r2 : r2 - 9;
-            const uint32_t rw = first ? 3u : (uint32_t)wy;
-            const int dz = zig((int)(ri / rw)), dy = zig((int)(ri % rw));
-            const bool trow = dz >= -1 && dz <= 1 && dy >= -1 && dy <= 1;
+        // slots (row of A, item), row-major: the touching sub-cells first,
+        // then every row.  Of A's rows an item can reach, a neighbour in y
+        // (z) has at most reach planes of ay (az), nearest first, on any
+        // other axis the 2 reach + 1 around its own; so an x neighbour's
+        // items have wy wz rows, the others' at most nr
+        const uint32_t nr1 = 3, nr2 = (uint32_t)max(reach[2] * wy, reach[1] * wz);
+        const uint32_t t1 = nr1 * nb + (9 - nr1) * nbx;
+        const uint32_t total = t1 + nr2 * nb + ((uint32_t)(wy * wz) - nr2) * nbx;
+        for (uint32_t p0 = take(2); p0 < total; p0 = take(2)) {
+          const uint32_t p = p0 + lane;
+          const uint32_t mr = mainr == kNone ? kNone : lfind(lp, mainr);
+          uint32_t bits = 0, all = 0, r0 = 0, jb = 0;
+          int x0 = 0, bx = 0, dy = 0, dz = 0;
+          if (p < total) {
+            const bool first = p < t1;
+            const uint32_t q = first ? p : p - t1, nr = first ? nr1 : nr2, both = nr * nb;
+            const int py = first ? 1 : reach[1], pz = first ? 1 : reach[2];
+            uint32_t r, j;
+            if (q < both) r = div_small(q, nb, inb), j = q - r * nb;
+            else r = div_small(q - both, nbx, inbx), j = q - both - r * nbx, r += nr;
+            jb = item(j);
             const uint32_t rb = brel[jb];
-            const int bx = rel_x(rb), ay = rel_y(rb) + dy, az = rel_z(rb) + dz;
-            if (az < 0 || az >= mm[2] || ay < 0 || ay >= mm[1] || !gap_ok(0, dy, dz)) continue;
-            const int x0 = max(bx - reach[0], 0), x1 = min(bx + reach[0], mm[0] - 1);
-            if (x0 > x1) continue;
-            const int bin0 = (az * mm[1] + ay) * mm[0] + x0;
-            const uint32_t all = rowbits(bin0, x1 - x0 + 1), r0 = rank(bin0);
-            uint32_t bits = all;
-            if (trow) bits &= first ? touchbits(bx - 1 - x0) : ~touchbits(bx - 1 - x0);
-            // an item already in the dominant set: only the stragglers
-            if (mr != kNone && lfind(lp, na + jb) == mr) bits &= srowbits(bin0, x1 - x0 + 1);
-            while (bits) {
-              const int b = __builtin_ctz(bits);
-              bits &= bits - 1;
-              if (!gap_ok(x0 + b - bx, dy, dz)) continue;
-              const uint32_t ia = r0 + __popc(all & ((1u << b) - 1));
-              consider(ia, na + jb, agr[ia], bgr[jb], ahead[ia], bhead[jb]);
+            bx = rel_x(rb);
+            const int by = rel_y(rb), bz = rel_z(rb);
+            const bool iny = by >= 0 && by < mm[1], inz = bz >= 0 && bz < mm[2];
+            const int ny = iny ? 2 * py + 1 : py;
+            const int kz = (int)r / ny, ky = (int)r - kz * ny;
+            const int az = inz ? bz + zig(kz) : (bz < 0 ? kz : mm[2] - 1 - kz);
+            const int ay = iny ? by + zig(ky) : (by < 0 ? ky : mm[1] - 1 - ky);
+            dz = az - bz, dy = ay - by;
+            const bool trow = dz >= -1 && dz <= 1 && dy >= -1 && dy <= 1;
+            x0 = max(bx - reach[0], 0);
+            const int x1 = min(bx + reach[0], mm[0] - 1);
+            if (kz < (inz ? 2 * pz + 1 : pz) && az >= 0 && az < mm[2] && ay >= 0 && ay < mm[1] &&
+                x0 <= x1 && (!first || trow) && gap_ok(0, dy, dz)) {
+              const int bin0 = (az * mm[1] + ay) * mm[0] + x0;
+              bits = all = rowbits(bin0, x1 - x0 + 1);
+              r0 = rank(bin0);
+              if (trow) bits &= first ? touchbits(bx - 1 - x0) : ~touchbits(bx - 1 - x0);
+              // an item already in the dominant set: only the stragglers
+              if (bits && mr != kNone && lfind(lp, na + jb) == mr) bits &= srowbits(bin0, x1 - x0 + 1);
             }
           }
-          drain();
+          walk(bits, all, r0, x0, bx, dy, dz, na + jb, p < total ? bgr[jb] : 0u);
         }
       } else {
         const uint32_t total = (uint32_t)na * nb;
-        for (uint32_t base = 0; base < total; base += ROUND) {
-          const uint32_t pe = min(total, base + (uint32_t)ROUND);
-          for (uint32_t p = base + threadIdx.x; p < pe; p += blockDim.x) {
-            const uint32_t ib = p / (uint32_t)na, ia = p - ib * (uint32_t)na;
-            const uint32_t ra = arel[ia], rb = brel[ib];
-            if (!gap_ok(rel_x(rb) - (int)(ra & 15), rel_y(rb) - (int)((ra >> 4) & 15),
-                        rel_z(rb) - (int)(ra >> 8)))
-              continue;
-            consider(ia, na + ib, agr[ia], bgr[ib], ahead[ia], bhead[ib]);
+        for (uint32_t p0 = take(2); p0 < total; p0 = take(2)) {
+          const uint32_t p = p0 + lane;
+          const uint32_t ib = div_small(p, (uint32_t)na, ina), ia = p - ib * (uint32_t)na;
+          bool any = p < total;
+          uint32_t jb = 0;
+          if (any) {
+            jb = item(ib);
+            const uint32_t rra = arel[ia], rb = brel[jb];
+            any = gap_ok(rel_x(rb) - (int)(rra & 15), rel_y(rb) - (int)((rra >> 4) & 15),
+                         rel_z(rb) - (int)(rra >> 8));
           }
-          drain();
+          offer(any, ia, na + jb, any ? agr[ia] : 0u, any ? bgr[jb] : 0u);
         }
       }
+      if (qn) flush(qn);
+      __syncthreads();
       // commit: a neighbour run joined in LDS joins its (home-cell) root's run
-      for (uint32_t ib = threadIdx.x; ib < nb; ib += blockDim.x) {
+      for (uint32_t j = threadIdx.x; j < nb; j += blockDim.x) {
+        const uint32_t ib = item(j);
         const uint32_t r = lfind(lp, na + ib);
         if (r != na + ib) uf_union(par, bhead[ib], ahead[r]);
       }
@@ -1949,15 +2022,6 @@ struct SmallLds {
   float qx[kSmallQ], qy[kSmallQ], qz[kSmallQ];  // queued neighbour candidates
   uint32_t qidx[kSmallQ];
 };
-
-// LDS written by some lanes of a wave and read by others afterwards: the
-// wave's LDS operations execute in order; this keeps the compiler from
-// moving them across.
-__device__ __forceinline__ void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 
 // The lane's particle (xi, yi, zi) against the kBlk partners p[0..kBlk-1]
 // in LDS, the same for every lane (broadcast reads, all issued before the
@@ -3111,7 +3175,7 @@ __global__ __launch_bounds__(256) void k_halo_sums(const uint32_t *__restrict__ 
       rb = o + (k < 3 ? k : (k == 3 ? 1 : 2));
     }
   }
-  if (MOM) {
+  if constexpr (MOM) {
     stage[w][kOnes][lane] = 1.0;
     wave_sync();
   }
@@ -4017,15 +4081,9 @@ static int enqueue_run(Run &r, hipStream_t st) {
     if ((rc = tb(6))) return rc;
     constexpr int kRB = 448;
     const uint32_t ra = std::min(maxbins, (uint32_t)kMaxRuns);
-    // rounds of 768 candidates: 256 and 384 gave 51.8 and 51.1 ms at 1024^3,
-    // 512 and 768 49.5-50.6 and 49.2-49.4, 1024 50.5-50.7, 2048 59.5 (the
-    // test queue overflows into in-place tests); a queue of 384 entries
-    // 48.6-48.8 against 48.9-49.1 for 256 and 320, 49.1-49.2 for 512 and
-    // 53-54 for 768 or 1024
-    k_link_dense<256, 8, kMaxRuns, kRB, 384, 768, 1>
-        <<<gbig, 256, dense_lds(ra, kRB), st>>>(
-            dbig, small + kSmNBig, pos4, G, runend, fine, rtoff, rtab, T, par, dV, dVB, (int)nvol,
-            ctr, small + kSmOverflow, ra, small + kSmDq);
+    k_link_dense<256, 6, kMaxRuns, kRB><<<gbig, 256, dense_lds(ra, kRB), st>>>(
+        dbig, small + kSmNBig, pos4, G, runend, fine, rtoff, rtab, T, par, dV, dVB, (int)nvol, ctr,
+        ra, small + kSmDq);
     FOF_HIP(hipGetLastError());
     if ((rc = te(6))) return rc;
   }
@@ -4481,17 +4539,15 @@ static int run_call(fof_ctx *ctx, const fof_particles_v1 *P, const fof_volume_v1
 
   // ---- results ----
   uint64_t H = 0;
-  bool dom_err = false, ovf = false;
+  bool dom_err = false;
   for (auto &r : runs) {
     if (r.pl.N == 0) continue;
     const uint32_t *hsm = reinterpret_cast<const uint32_t *>(r.pp->hres.data());
     dom_err = dom_err || hsm[kSmErr];
-    ovf = ovf || hsm[kSmOverflow];
     H += run_nhalos(r);
   }
   out->nhalos = H;
   if (dom_err) return FOF_E_DOMAIN;
-  if (ovf) return FOF_E_RANGE;  // run table overflow (cannot happen with m <= 12)
   if (want_halos && H > out->halo_cap && (out->halos || out->moments)) {
     if (out->halo_offsets) out->halo_offsets[nvol] = H;  // the capacity needed
     if (stats) stats->nhalos = H;
