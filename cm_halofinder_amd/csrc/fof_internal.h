@@ -104,6 +104,9 @@ struct Pipe {
   std::vector<uint8_t> hres;   // counts, flags and counters read back
   hipEvent_t ev[2 * FOF_NPHASE] = {};
   bool events = false;
+  // a side stream of the link kernels, forked from and joined to `stream`
+  hipStream_t side = nullptr;
+  hipEvent_t side_fork = nullptr, side_join = nullptr;
 };
 
 constexpr int kMaxPipes = 8;  // concurrent pipelines of one call
