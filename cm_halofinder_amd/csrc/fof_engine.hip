@@ -481,7 +481,7 @@ constexpr int kMaxBuckets = 1280;  // of pass A
 constexpr int kMaxCoarse = 512;    // coarse buckets (C < 2^31 cells)
 
 static uint32_t part_tile(uint64_t N) {
-  return (uint32_t)std::min<uint64_t>(kPartTile, std::max<uint64_t>(1, (N / 1024 + 1023) / 1024) * 1024);
+  return (uint32_t)std::min<uint64_t>(kPartTile, std::max<uint64_t>(1, (N / 1024 + 2047) / 2048) * 2048);
 }
 static int fine_bits(uint64_t C) {
   int fb = kFineBits;
@@ -504,7 +504,8 @@ __device__ __forceinline__ uint32_t cell_of_xyz(float x, float y, float z, const
 }
 
 // A, count: keys, validation, hist[b * ntiles + tile] (bucket-major, so one
-// exclusive scan gives each (bucket, tile) its first output slot).
+// exclusive scan gives each (bucket, tile) its first output slot), and the
+// outputs' defaults (own label, own 1-based ring entry) where given.
 __global__ __launch_bounds__(256) void k_pa_count(const uint8_t *__restrict__ base,
                                                   uint32_t stride, uint32_t offpos, uint32_t N,
                                                   const VolDev *__restrict__ vols,
@@ -513,6 +514,8 @@ __global__ __launch_bounds__(256) void k_pa_count(const uint8_t *__restrict__ ba
                                                   uint32_t ptile, int shift,
                                                   uint32_t *__restrict__ key,
                                                   uint32_t *__restrict__ hist,
+                                                  uint32_t *__restrict__ label_out,
+                                                  uint32_t *__restrict__ next_out,
                                                   uint32_t *__restrict__ err) {
   __shared__ uint32_t h[kMaxBuckets];
   const uint32_t tile = blockIdx.x;
@@ -541,9 +544,11 @@ __global__ __launch_bounds__(256) void k_pa_count(const uint8_t *__restrict__ ba
       hint = va;
       one = qe < vbeg[va + 1];
     }
-    uint32_t c[kCnt];
+    uint32_t c[kCnt], b[kCnt];
     if (one) {
       const VolDev V = vols[va];
+#pragma unroll
+      for (int k = 0; k < kCnt; k++) b[k] = V.pbeg;
 #pragma unroll
       for (int k = 0; k < kCnt; k++)
         c[k] = q0 + threadIdx.x + k * 256 < p1 ? cell_of_xyz(x[k], y[k], z[k], V, err) : 0u;
@@ -551,8 +556,12 @@ __global__ __launch_bounds__(256) void k_pa_count(const uint8_t *__restrict__ ba
 #pragma unroll
       for (int k = 0; k < kCnt; k++) {
         const uint32_t p = q0 + threadIdx.x + k * 256;
-        c[k] = p < p1 ? cell_of_xyz(x[k], y[k], z[k], vols[vol_of_run(vbeg, nvol, p, N, hint)], err)
-                      : 0u;
+        c[k] = b[k] = 0;
+        if (p < p1) {
+          const VolDev &V = vols[vol_of_run(vbeg, nvol, p, N, hint)];
+          c[k] = cell_of_xyz(x[k], y[k], z[k], V, err);
+          b[k] = V.pbeg;
+        }
       }
     }
 #pragma unroll
@@ -560,6 +569,8 @@ __global__ __launch_bounds__(256) void k_pa_count(const uint8_t *__restrict__ ba
       const uint32_t p = q0 + threadIdx.x + k * 256;
       if (p < p1) {
         key[p] = c[k];
+        if (label_out) label_out[p] = p - b[k];
+        if (next_out) next_out[p] = p - b[k] + 1u;
         atomicAdd(&h[c[k] >> shift], 1u);
       }
     }
@@ -685,7 +696,7 @@ __global__ __launch_bounds__(kPartNT) void k_pa_scatter(const uint8_t *__restric
   }
 }
 
-// Pass A's bucket starts (Bc + 1 entries) out of its scanned histogram.
+// Coarse bucket starts (Bc + 1 entries) out of the scanned A histogram.
 __global__ void k_pa_starts(uint32_t Bc, uint32_t ntiles, const uint32_t *__restrict__ off,
                             uint32_t *__restrict__ cstart) {
   for (uint32_t b = blockIdx.x * blockDim.x + threadIdx.x; b <= Bc; b += gridDim.x * blockDim.x)
@@ -833,8 +844,11 @@ __device__ __forceinline__ int vol_of_cell(const VolDev *__restrict__ vols, int 
 constexpr int kPcThreads = 1024;
 constexpr uint32_t kPcListS = 1536, kPcListB = 512;
 
+// The bucket's particles start at fstart[f * fstride].  Also each particle's
+// union-find start (par, run_end, gsize).
 __global__ __launch_bounds__(kPcThreads) void k_pc_sort(uint64_t C, int fb,
                                                  const uint32_t *__restrict__ fstart,
+                                                 uint32_t fstride,
                                                  const uint32_t *__restrict__ ikey,
                                                  const float4 *__restrict__ ipos,
                                                  uint32_t *__restrict__ start,
@@ -843,7 +857,10 @@ __global__ __launch_bounds__(kPcThreads) void k_pc_sort(uint64_t C, int fb,
                                                  uint32_t T, uint32_t *__restrict__ dense,
                                                  uint32_t *__restrict__ ndense,
                                                  uint32_t *__restrict__ dbig,
-                                                 uint32_t *__restrict__ nbig) {
+                                                 uint32_t *__restrict__ nbig,
+                                                 uint32_t *__restrict__ par,
+                                                 uint32_t *__restrict__ run_end,
+                                                 uint32_t *__restrict__ gsize) {
   // counters padded by one word per 64 so that the per-thread segments of
   // the scan fall in different LDS banks
   __shared__ uint32_t lc[kFineCells + kFineCells / 64 + 1];
@@ -853,7 +870,7 @@ __global__ __launch_bounds__(kPcThreads) void k_pc_sort(uint64_t C, int fb,
   // entries reserved, first reservation that did not fit, global bases
   __shared__ uint32_t nres[2], nfit[2], gbase[2];
   const uint32_t f = blockIdx.x;
-  const uint32_t q0 = fstart[f], q1 = fstart[f + 1];
+  const uint32_t q0 = fstart[(uint64_t)f * fstride], q1 = fstart[(uint64_t)(f + 1) * fstride];
   const uint64_t c0 = (uint64_t)f << fb;
   const uint32_t cells = 1u << fb;
   const uint32_t nc = (uint32_t)min((uint64_t)cells, C - c0);
@@ -935,6 +952,9 @@ __global__ __launch_bounds__(kPcThreads) void k_pc_sort(uint64_t C, int fb,
   for (uint32_t i = q0 + threadIdx.x; i < q1; i += blockDim.x) {
     const uint32_t slot = q0 + atomicAdd(&lc[P(ikey[i] & (cells - 1))], 1u);
     pos4[slot] = ipos[i];
+    par[i] = i;
+    run_end[i] = i + 1;
+    gsize[i] = 0;
   }
 }
 
@@ -946,6 +966,8 @@ __global__ __launch_bounds__(256) void k_keys_sparse(const uint8_t *__restrict__
                                                      Grid G, uint32_t *__restrict__ klo,
                                                      uint32_t *__restrict__ khi,
                                                      uint32_t *__restrict__ val,
+                                                     uint32_t *__restrict__ label_out,
+                                                     uint32_t *__restrict__ next_out,
                                                      uint32_t *__restrict__ err) {
   for (uint32_t p = blockIdx.x * blockDim.x + threadIdx.x; p < N;
        p += gridDim.x * blockDim.x) {
@@ -964,6 +986,8 @@ __global__ __launch_bounds__(256) void k_keys_sparse(const uint8_t *__restrict__
     klo[p] = (uint32_t)k;
     khi[p] = (uint32_t)(k >> 32);
     val[p] = p;
+    if (label_out) label_out[p] = p - V.pbeg;
+    if (next_out) next_out[p] = p - V.pbeg + 1u;
   }
 }
 
@@ -1059,11 +1083,13 @@ __global__ __launch_bounds__(256) void k_cells_finish(
 }
 
 __global__ __launch_bounds__(256) void k_init_uf(uint32_t N, uint32_t *__restrict__ par,
-                                                 uint32_t *__restrict__ run_end) {
+                                                 uint32_t *__restrict__ run_end,
+                                                 uint32_t *__restrict__ gsize) {
   for (uint32_t x = blockIdx.x * blockDim.x + threadIdx.x; x < N;
        x += gridDim.x * blockDim.x) {
     par[x] = x;
     run_end[x] = x + 1;
+    gsize[x] = 0;
   }
 }
 
@@ -2504,6 +2530,18 @@ __global__ __launch_bounds__(256) void k_flatten(uint32_t N, uint32_t *__restric
   if ((threadIdx.x & 63) == 0 && t) ctr_add(ctr, kCtrGroups, t);
 }
 
+// The accumulators of k_flatten (minimum index, with idroot minimum ID) and
+// the label bitmap.
+__global__ __launch_bounds__(256) void k_init_groups(uint32_t N, uint32_t *__restrict__ minorig,
+                                                     unsigned long long *__restrict__ idroot,
+                                                     uint32_t nw, uint32_t *__restrict__ bits) {
+  for (uint32_t x = blockIdx.x * blockDim.x + threadIdx.x; x < N; x += gridDim.x * blockDim.x) {
+    minorig[x] = ~0u;
+    if (idroot) idroot[x] = ~0ull;
+    if (x < nw) bits[x] = 0;
+  }
+}
+
 // Members of groups of two or more: label[orig] = group minimum index |
 // kFlag, and each member's (label, orig) at the next free slot of its group
 // in the member list (the group's cursor, indexed by its label, starts
@@ -2515,7 +2553,7 @@ __global__ __launch_bounds__(256) void k_flatten(uint32_t N, uint32_t *__restric
 //          while its cells are processed (the 4^3-batched 1024^3 box: 11 ms
 //          less than the partitioned writes); with label_out given (no
 //          minimum-ID output wanted) straight into the caller's output, as
-//          volume-local labels over the defaults k_label_init wrote;
+//          volume-local labels over the defaults the key pass wrote;
 //  else    scatter_u32 from the member list afterwards, partitioned by index
 //          (one 1.09e9-particle volume: 4 ms less than direct writes spread
 //          over 4.4 GB).
@@ -2558,7 +2596,7 @@ __global__ __launch_bounds__(256) void k_label(uint32_t N, const uint32_t *__res
       const uint32_t x = (uint32_t)xx;
       r = par[x];
       const uint32_t g = gsize[r];
-      // singletons: k_label_init wrote them, unless their volume keeps
+      // singletons: their defaults are written, unless their volume keeps
       // groups of one (those join the member list)
       if (!(r == x && g == 0) || (single && !(1.0 < vols[vol_of(vbeg, nvol, x)].nphalomin))) {
         mem = true;
@@ -2616,31 +2654,22 @@ static inline uint32_t tiles_for(uint64_t n) { return (uint32_t)std::max<uint64_
 __global__ __launch_bounds__(256) void k_label_init(uint32_t N, const VolDev *__restrict__ vols,
                                                     const uint32_t *__restrict__ vbeg, int nvol,
                                                     uint32_t *__restrict__ label,
-                                                    uint32_t *__restrict__ hsize,
-                                                    uint32_t *__restrict__ label_out,
-                                                    uint32_t *__restrict__ next_out) {
+                                                    uint32_t *__restrict__ hsize) {
   const uint64_t i0 = (uint64_t)blockIdx.x * kTileN, i1 = min((uint64_t)N, i0 + kTileN);
   if (i0 >= i1) return;
-  // internal defaults (label, hsize) or, when k_label writes label_out
-  // itself, the outputs' defaults: own label and own ring entry, 1-based
-  auto body = [&](uint32_t i, double nphalomin, uint32_t b) {
-    if (label) label[i] = i | (!(1.0 < nphalomin) ? kFlag : 0u);
-    if (hsize) hsize[i] = 1u;
-    if (label_out) label_out[i] = i - b;
-    if (next_out) next_out[i] = i - b + 1u;
+  auto body = [&](uint32_t i, double nphalomin) {
+    label[i] = i | (!(1.0 < nphalomin) ? kFlag : 0u);
+    hsize[i] = 1u;
   };
   const int va = vol_of(vbeg, nvol, (uint32_t)i0);
   if (i1 <= vbeg[va + 1]) {  // the tile lies in one volume
     const double nph = vols[va].nphalomin;
-    const uint32_t b = vbeg[va];
-    for (uint32_t i = (uint32_t)i0 + threadIdx.x; i < i1; i += blockDim.x) body(i, nph, b);
+    for (uint32_t i = (uint32_t)i0 + threadIdx.x; i < i1; i += blockDim.x) body(i, nph);
     return;
   }
   int hint = va;
-  for (uint32_t i = (uint32_t)i0 + threadIdx.x; i < i1; i += blockDim.x) {
-    const int v = vol_of_run(vbeg, nvol, i, N, hint);
-    body(i, vols[v].nphalomin, vbeg[v]);
-  }
+  for (uint32_t i = (uint32_t)i0 + threadIdx.x; i < i1; i += blockDim.x)
+    body(i, vols[vol_of_run(vbeg, nvol, i, N, hint)].nphalomin);
 }
 
 // Outputs for every particle: label_out (volume-local), for particles not in
@@ -2693,8 +2722,14 @@ __global__ __launch_bounds__(256) void k_out_init(uint32_t N, const uint32_t *__
 // The group list in label order without a sort: each group of two or more
 // (and, where a volume keeps groups of one -- Nphalomin <= 1 -- each such
 // particle) sets the bit of its label (the group's lowest input index) in a
-// bitmap over the input indices and puts its size at lsize[label]; a scan of
-// the words' bit counts ranks the labels.
+// bitmap over the input indices and puts its size at lsize[label].  Blocks of
+// consecutive words then total their groups, members and halos (groups passing
+// the size cut) in k_group_sums, and k_group_emit, each block behind the totals
+// of those before it, lists the labels in ascending order, each group's first
+// member slot, its cursor (by label) and the halos' first slots.  Two launches
+// in place of thirteen (bit counts, two scans, the list, the cursors, the halo
+// flags and their compaction), which is what a small call waits for; the sizes
+// are gathered twice for it.
 __global__ __launch_bounds__(256) void k_group_bits(uint32_t N, const uint32_t *__restrict__ par,
                                                     const uint32_t *__restrict__ gsize,
                                                     const uint32_t *__restrict__ minorig,
@@ -2713,46 +2748,125 @@ __global__ __launch_bounds__(256) void k_group_bits(uint32_t N, const uint32_t *
   }
 }
 
-__global__ __launch_bounds__(256) void k_word_counts(uint64_t nw, const uint32_t *__restrict__ bits,
-                                                     uint32_t *__restrict__ cnt) {
-  for (uint64_t w = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; w < nw;
-       w += (uint64_t)gridDim.x * blockDim.x)
-    cnt[w] = (uint32_t)__popc(bits[w]);
+constexpr uint32_t kGroupBlocks = 4096;  // at most: each block reads the totals before it
+
+// Words of a block: kGroupWords(nw) consecutive runs of 256.
+static inline uint32_t group_runs(uint64_t nw) {
+  return (uint32_t)((nw + 256ull * kGroupBlocks - 1) / (256ull * kGroupBlocks));
 }
 
-// Labels in ascending order and their groups' sizes (scanned in place into
-// first slots); the group count to the device counts.
-__global__ __launch_bounds__(256) void k_group_list(uint64_t nw, const uint32_t *__restrict__ bits,
-                                                    const uint32_t *__restrict__ wpre,
-                                                    const uint32_t *__restrict__ lsize,
-                                                    uint32_t *__restrict__ glab,
-                                                    uint32_t *__restrict__ offs,
-                                                    uint32_t *__restrict__ dR) {
-  const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t == 0) *dR = wpre[nw];
-  for (uint64_t w = t; w < nw; w += (uint64_t)gridDim.x * blockDim.x) {
-    uint32_t m = bits[w], at = wpre[w];
-    while (m) {
-      const uint32_t lab = (uint32_t)(w * 32) + (uint32_t)__builtin_ctz(m);
-      m &= m - 1;
-      glab[at] = lab;
-      offs[at] = lsize[lab];
-      at++;
-    }
+struct GroupTot {
+  uint32_t groups, members, halos, pad;
+};
+
+// One bitmap word's groups, members and halos (labels ascend with the bits).
+template <class F>
+__device__ __forceinline__ void word_groups(uint32_t m, uint64_t w,
+                                            const uint32_t *__restrict__ lsize,
+                                            const VolDev *__restrict__ vols,
+                                            const uint32_t *__restrict__ vbeg, int nvol, F f) {
+  int v = -1;
+  while (m) {
+    const uint32_t lab = (uint32_t)(w * 32) + (uint32_t)__builtin_ctz(m);
+    m &= m - 1;
+    if (v < 0 || lab >= vbeg[v + 1]) v = vol_of(vbeg, nvol, lab);
+    const uint32_t n = lsize[lab];
+    f(lab, n, !((double)n < vols[v].nphalomin));  // src_v2/FOF.c:202, :290-298
   }
 }
 
-// Each group's cursor (indexed by its label) at its first slot; the member
-// count to the device counts.
-__global__ __launch_bounds__(256) void k_group_cursors(const uint32_t *__restrict__ dR,
-                                                       const uint32_t *__restrict__ glab,
-                                                       const uint32_t *__restrict__ offs,
-                                                       uint32_t *__restrict__ cursor,
-                                                       uint32_t *__restrict__ dM) {
-  const uint32_t R = *dR;
-  const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t == 0) *dM = offs[R];
-  for (uint32_t i = t; i < R; i += gridDim.x * blockDim.x) cursor[glab[i]] = offs[i];
+// Block-wide exclusive scan of (a, b) over 256 threads and their totals.
+__device__ __forceinline__ void block_scan2(uint32_t &a, uint32_t &b, uint32_t &ta, uint32_t &tb,
+                                            uint32_t (&ws)[2][4]) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  uint32_t ia = a, ib = b;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t x = __shfl_up(ia, o, 64), y = __shfl_up(ib, o, 64);
+    if (lane >= o) ia += x, ib += y;
+  }
+  __syncthreads();
+  if (lane == 63) ws[0][w] = ia, ws[1][w] = ib;
+  __syncthreads();
+  a = ia - a, b = ib - b;
+  ta = tb = 0;
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    if (q < w) a += ws[0][q], b += ws[1][q];
+    ta += ws[0][q], tb += ws[1][q];
+  }
+}
+
+__global__ __launch_bounds__(256) void k_group_sums(uint64_t nw, uint32_t runs,
+                                                    const uint32_t *__restrict__ bits,
+                                                    const uint32_t *__restrict__ lsize,
+                                                    const VolDev *__restrict__ vols,
+                                                    const uint32_t *__restrict__ vbeg, int nvol,
+                                                    GroupTot *__restrict__ tot) {
+  __shared__ uint32_t ws[2][4];
+  uint32_t gh = 0, mem = 0;  // groups | halos << 16 of a run
+  GroupTot t = {0, 0, 0, 0};
+  for (uint32_t j = 0; j < runs; j++) {
+    const uint64_t w = ((uint64_t)blockIdx.x * runs + j) * 256 + threadIdx.x;
+    if (w >= nw) break;
+    word_groups(bits[w], w, lsize, vols, vbeg, nvol, [&](uint32_t, uint32_t n, bool halo) {
+      t.groups++, t.members += n, t.halos += halo ? 1u : 0u;
+    });
+  }
+  uint32_t g = t.groups, m = t.members, x, y;
+  block_scan2(g, m, gh, mem, ws);
+  uint32_t h = t.halos, z = 0;
+  block_scan2(h, z, x, y, ws);
+  if (threadIdx.x == 0) tot[blockIdx.x] = {gh, mem, x, 0};
+}
+
+__global__ __launch_bounds__(256) void k_group_emit(uint64_t nw, uint32_t runs,
+                                                    const uint32_t *__restrict__ bits,
+                                                    const uint32_t *__restrict__ lsize,
+                                                    const VolDev *__restrict__ vols,
+                                                    const uint32_t *__restrict__ vbeg, int nvol,
+                                                    const GroupTot *__restrict__ tot,
+                                                    uint32_t *__restrict__ glab,
+                                                    uint32_t *__restrict__ offs,
+                                                    uint32_t *__restrict__ cursor,
+                                                    uint32_t *__restrict__ hk,
+                                                    uint32_t *__restrict__ small) {
+  __shared__ uint32_t ws[2][4];
+  GroupTot pre = {0, 0, 0, 0};
+  for (uint32_t b = threadIdx.x; b < blockIdx.x; b += 256) {
+    const GroupTot t = tot[b];
+    pre.groups += t.groups, pre.members += t.members, pre.halos += t.halos;
+  }
+  {
+    uint32_t a = pre.groups, b = pre.members, c = pre.halos, d = 0, z;
+    block_scan2(a, b, pre.groups, pre.members, ws);
+    block_scan2(c, d, pre.halos, z, ws);
+  }
+  for (uint32_t j = 0; j < runs; j++) {
+    const uint64_t w = ((uint64_t)blockIdx.x * runs + j) * 256 + threadIdx.x;
+    if (w - threadIdx.x >= nw) break;
+    const uint32_t m = w < nw ? bits[w] : 0u;
+    uint32_t gh = 0, mem = 0, tgh, tmem;  // groups | halos << 16: at most 8192 each in a run
+    word_groups(m, w, lsize, vols, vbeg, nvol, [&](uint32_t, uint32_t n, bool halo) {
+      gh += halo ? 0x10001u : 1u, mem += n;
+    });
+    block_scan2(gh, mem, tgh, tmem, ws);
+    uint32_t g = pre.groups + (gh & 0xFFFFu), h = pre.halos + (gh >> 16), at = pre.members + mem;
+    word_groups(m, w, lsize, vols, vbeg, nvol, [&](uint32_t lab, uint32_t n, bool halo) {
+      glab[g] = lab;
+      offs[g++] = at;
+      cursor[lab] = at;
+      if (halo && hk) hk[h++] = at;
+      at += n;
+    });
+    pre.groups += tgh & 0xFFFFu, pre.halos += tgh >> 16, pre.members += tmem;
+  }
+  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) {
+    offs[pre.groups] = pre.members;
+    small[kSmR] = pre.groups;
+    small[kSmM] = pre.members;
+    if (hk) small[kSmH] = pre.halos;
+  }
 }
 
 // Sorting each segment of the member list by index.  Groups of at most four
@@ -3051,59 +3165,35 @@ __global__ __launch_bounds__(NT, 4) void k_seg_sort_list(const uint32_t *__restr
   }
 }
 
-// Halo flags of the groups in label order: the first slot | kFlag for a
-// group passing its volume's size cut (src_v2/FOF.c:290-298), else 0.
-__global__ __launch_bounds__(256) void k_halo_flags(const uint32_t *__restrict__ dR,
-                                                    const uint32_t *__restrict__ rkey,
-                                                    const uint32_t *__restrict__ offs,
-                                                    const VolDev *__restrict__ vols,
-                                                    const uint32_t *__restrict__ vbeg, int nvol,
-                                                    uint32_t *__restrict__ hsrc) {
-  const uint32_t R = *dR;
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < R; i += gridDim.x * blockDim.x) {
-    const uint32_t n = offs[i + 1] - offs[i];
-    const double nph = vols[vol_of(vbeg, nvol, rkey[i])].nphalomin;
-    hsrc[i] = !((double)n < nph) ? (offs[i] | kFlag) : 0u;
-  }
-}
-
 __global__ __launch_bounds__(256) void k_ring(const uint32_t *__restrict__ dM,
                                               const uint32_t *__restrict__ skey,
                                               const uint32_t *__restrict__ sval,
-                                              const uint32_t *__restrict__ hsize,
-                                              const VolDev *__restrict__ vols,
                                               const uint32_t *__restrict__ vbeg, int nvol,
                                               uint32_t *__restrict__ next_out,
                                               uint32_t *__restrict__ pidx,
-                                              uint32_t *__restrict__ pval,
-                                              uint32_t *__restrict__ hflag) {
+                                              uint32_t *__restrict__ pval) {
   const uint32_t M = *dM;
   const uint64_t k0 = (uint64_t)blockIdx.x * kTileN, k1 = min((uint64_t)M, k0 + kTileN);
   if (k0 >= k1) return;
-  auto body = [&](uint32_t k, uint32_t lab, uint32_t b, double nphalomin) {
+  auto body = [&](uint32_t k, uint32_t lab, uint32_t b) {
     const uint32_t i = sval[k];
     const uint32_t nx = (k + 1 < M && skey[k + 1] == lab) ? sval[k + 1] : lab;
     if (pidx) pidx[k] = i, pval[k] = nx - b + 1u;
     else if (next_out) next_out[i] = nx - b + 1u;
-    if (hflag) {
-      const bool gstart = (k == 0) || (skey[k - 1] != lab);
-      hflag[k] = (gstart && !((double)hsize[lab] < nphalomin)) ? kFlag : 0u;
-    }
   };
   // the list is sorted by label, so by volume; a member shares its head's
   // volume, and a tile whose first and last labels share one has no other
   const int va = vol_of(vbeg, nvol, skey[k0]);
   if (skey[k1 - 1] < vbeg[va + 1]) {
     const uint32_t b = vbeg[va];
-    const double nph = vols[va].nphalomin;
-    for (uint32_t k = (uint32_t)k0 + threadIdx.x; k < k1; k += blockDim.x) body(k, skey[k], b, nph);
+    for (uint32_t k = (uint32_t)k0 + threadIdx.x; k < k1; k += blockDim.x) body(k, skey[k], b);
     return;
   }
   int hint = va;
   for (uint32_t k = (uint32_t)k0 + threadIdx.x; k < k1; k += blockDim.x) {
     const uint32_t lab = skey[k];
     const int v = vol_of_sorted(vbeg, nvol, lab, hint);
-    body(k, lab, vbeg[v], vols[v].nphalomin);
+    body(k, lab, vbeg[v]);
   }
 }
 
@@ -3152,8 +3242,7 @@ __global__ __launch_bounds__(256) void k_halo_sums(const uint32_t *__restrict__ 
                                                    const uint32_t *__restrict__ vbeg, int nvol,
                                                    fof_halo_v1 *__restrict__ out,
                                                    fof_moments_v1 *__restrict__ mout,
-                                                   uint64_t cap,
-                                                   uint32_t *__restrict__ hhead,
+                                                   uint64_t cap, uint64_t *__restrict__ hoff,
                                                    unsigned long long *__restrict__ ctr) {
   constexpr int NQ = MOM ? 36 : 6;
   constexpr int kOnes = 12;
@@ -3180,6 +3269,18 @@ __global__ __launch_bounds__(256) void k_halo_sums(const uint32_t *__restrict__ 
     wave_sync();
   }
   const double *const pa = stage[w][ra], *const pb = stage[w][MOM ? rb : 0];
+  // hoff[v] = first halo whose head lies in volume v or later
+  for (uint64_t v = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; v <= (uint64_t)nvol;
+       v += (uint64_t)gridDim.x * blockDim.x) {
+    uint32_t lo = v == (uint64_t)nvol ? H : 0, hi = v == 0 ? 0 : H;
+    const uint32_t head = vbeg[v];
+    while (lo < hi) {
+      const uint32_t mid = (lo + hi) >> 1;
+      if (skey[hk[mid]] < head) lo = mid + 1;
+      else hi = mid;
+    }
+    hoff[v] = lo;
+  }
   for (uint32_t h = blockIdx.x * (blockDim.x >> 6) + w; h < H; h += nw) {
     // wave-uniform, visibly so: branches on them leave the loads in flight countable
     const uint32_t k0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)hk[h]);
@@ -3324,7 +3425,6 @@ __global__ __launch_bounds__(256) void k_halo_sums(const uint32_t *__restrict__ 
         H1.sum_vel[0] = s3, H1.sum_vel[1] = s4, H1.sum_vel[2] = s5;
         out[h] = H1;
       }
-      hhead[h] = lab;
       owned_cnt += own ? 1u : 0u;
     }
   }
@@ -3332,24 +3432,6 @@ __global__ __launch_bounds__(256) void k_halo_sums(const uint32_t *__restrict__ 
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) t += __shfl_down(t, o, 64);
   if ((threadIdx.x & 63) == 0 && t) ctr_add(ctr, kCtrOwned, t);
-}
-
-// halo_offsets[v] = first halo whose global head >= vbeg[v].
-__global__ void k_halo_offsets(const uint32_t *__restrict__ dH,
-                               const uint32_t *__restrict__ hhead,
-                               const uint32_t *__restrict__ vbeg, int nvol,
-                               uint64_t *__restrict__ off) {
-  const uint32_t H = *dH;
-  for (int v = blockIdx.x * blockDim.x + threadIdx.x; v <= nvol; v += gridDim.x * blockDim.x) {
-    const uint32_t key = vbeg[v];
-    uint32_t lo = 0, hi = H;
-    while (lo < hi) {
-      uint32_t mid = (lo + hi) >> 1;
-      if (hhead[mid] < key) lo = mid + 1;
-      else hi = mid;
-    }
-    off[v] = (v == nvol) ? H : lo;
-  }
 }
 
 // ---------------------------------------------------------------------------
@@ -3929,6 +4011,11 @@ static int enqueue_run(Run &r, hipStream_t st) {
   const uint32_t offid = pl.offid >= 0 ? (uint32_t)pl.offid : 0u;
   const uint32_t gN = grid_for(N);
   const uint32_t T = pl.T;
+  const bool direct = pl.direct_writes;
+  // direct writes and no minimum IDs: the key pass writes the outputs'
+  // defaults and k_label label_out itself, and k_out_init is not needed
+  const bool fused = direct && !r.d_minid;
+  uint32_t *label0 = fused ? r.d_label : nullptr, *next0 = fused ? r.d_next : nullptr;
 
   Grid G;
   G.start = start;
@@ -3945,8 +4032,9 @@ static int enqueue_run(Run &r, hipStream_t st) {
     // until k_subsort) where they fit
     const bool inf = pl.hist_in_fine;
     uint32_t *histA = inf ? reinterpret_cast<uint32_t *>(B.fine) : B.part;
-    uint32_t *offA = histA + nA + 32;      // nA + 1
-    uint32_t *histB = inf ? B.part : offA + nA + 32;  // nB
+    const uint64_t nA4 = (nA + 3) / 4 * 4 + 32;  // the scans' vector accesses stay aligned
+    uint32_t *offA = histA + nA4;                 // nA + 1
+    uint32_t *histB = inf ? B.part : offA + nA4;  // nB
     uint32_t *offB = histB + nB + 32;      // nB + 1
     uint32_t *cst = offB + nB + 32;        // Bc + 1
     uint32_t *t0 = cst + Bc + 32;          // Bc + 1
@@ -3959,15 +4047,14 @@ static int enqueue_run(Run &r, hipStream_t st) {
     const int fb = pl.fb, shift = pl.two_level ? fb + 8 : fb;
     if ((rc = tb(0))) return rc;
     k_pa_count<<<ntA, 256, 0, st>>>(dbase, stride, offpos, NN, dV, dVB, (int)nvol, Bc, ntA, ptile,
-                                    shift, key, histA, small + kSmErr);
+                                    shift, key, histA, label0, next0, small + kSmErr);
     FOF_HIP(hipGetLastError());
     if ((rc = te(0))) return rc;
     if ((rc = tb(1))) return rc;
     if ((rc = scan_u32(histA, offA, nA, B.tmp, st))) return rc;
-    uint32_t *starts = pl.two_level ? cst : fst;
-    k_pa_starts<<<grid_for(Bc + 1), 256, 0, st>>>(Bc, ntA, offA, starts);
-    FOF_HIP(hipGetLastError());
     if (pl.two_level) {
+      k_pa_starts<<<grid_for(Bc + 1), 256, 0, st>>>(Bc, ntA, offA, cst);
+      FOF_HIP(hipGetLastError());
       k_pb_tiles<<<1, kMaxCoarse, 0, st>>>(Bc, ntBmax, ptile, cst, t0, tinfo, small + kSmNtB);
       FOF_HIP(hipGetLastError());
     }
@@ -3992,9 +4079,10 @@ static int enqueue_run(Run &r, hipStream_t st) {
       k_pb_starts<<<grid_for(F + 1), 256, 0, st>>>(F, t0, cst, offB, NN, fst);
       FOF_HIP(hipGetLastError());
     }
-    k_pc_sort<<<F, kPcThreads, 0, st>>>((uint64_t)pl.C, fb, fst, k2, p2, start, pos4, dV,
+    k_pc_sort<<<F, kPcThreads, 0, st>>>((uint64_t)pl.C, fb, pl.two_level ? fst : offA,
+                                        pl.two_level ? 1u : ntA, k2, p2, start, pos4, dV,
                                         (int)nvol, T, dense, small + kSmNDense, dbig,
-                                        small + kSmNBig);
+                                        small + kSmNBig, par, runend, gsize);
     FOF_HIP(hipGetLastError());
     if ((rc = te(2))) return rc;
   } else {
@@ -4002,7 +4090,7 @@ static int enqueue_run(Run &r, hipStream_t st) {
     uint32_t *cnt = B.cnt;
     if ((rc = tb(0))) return rc;
     k_keys_sparse<<<gN, 256, 0, st>>>(dbase, stride, offpos, NN, dV, dVB, (int)nvol, G, sk0, key,
-                                      sv0, small + kSmErr);
+                                      sv0, label0, next0, small + kSmErr);
     FOF_HIP(hipGetLastError());
     if ((rc = te(0))) return rc;
     if ((rc = tb(1))) return rc;
@@ -4039,11 +4127,11 @@ static int enqueue_run(Run &r, hipStream_t st) {
                                                 label, dV, dVB, (int)nvol, T, dense,
                                                 small + kSmNDense, dbig, small + kSmNBig);
     FOF_HIP(hipGetLastError());
+    if ((rc = tb(3))) return rc;
+    k_init_uf<<<gN, 256, 0, st>>>(NN, par, runend, gsize);
+    FOF_HIP(hipGetLastError());
+    if ((rc = te(3))) return rc;
   }
-  if ((rc = tb(3))) return rc;
-  k_init_uf<<<gN, 256, 0, st>>>(NN, par, runend);
-  FOF_HIP(hipGetLastError());
-  if ((rc = te(3))) return rc;
   // 4: sub-cell sort of dense cells (tmp4 aliases the sort buffers s0..s3);
   // grids for the most dense cells there can be, the lists' lengths are read
   // on the device
@@ -4118,52 +4206,45 @@ static int enqueue_run(Run &r, hipStream_t st) {
   uint32_t *minorig = runend, *hsize = key;
   unsigned long long *idroot = pl.want_minid ? fine : nullptr;
   if ((rc = tb(7))) return rc;
-  if ((rc = fill_u32(minorig, N, ~0u, st))) return rc;
-  if ((rc = fill_u32(gsize, N, 0u, st))) return rc;
-  if (idroot && (rc = fill_u32(reinterpret_cast<uint32_t *>(idroot), 2 * N, ~0u, st))) return rc;
+  const uint64_t nw = (N + 31) / 32;
+  uint32_t *gbits = key;  // the label bitmap (the head sizes follow in k_label)
+  k_init_groups<<<gN, 256, 0, st>>>(NN, minorig, idroot, (uint32_t)nw, gbits);
+  FOF_HIP(hipGetLastError());
   k_flatten<<<gN, 256, 0, st>>>(NN, par, pos4, minorig, gsize, ctr, dbase, stride, offid, idroot);
   FOF_HIP(hipGetLastError());
   if ((rc = te(7))) return rc;
   // 8: the group list -- groups of two or more (and kept groups of one) in
-  // label order, each group's first slot in the member list -- then the
-  // labels, which also fill the list.  The label bitmap and its word prefix
-  // counts live where the cursors will (rtab), the sizes by label in the
-  // label array (before its defaults), the first slots in sk1 and the labels
-  // in order in sv1 (behind 64 words: R + 1 first slots may reach N + 1);
-  // large groups, halo flags and the halo list go to the cell-sorted
-  // positions once k_label has read them.
+  // label order, each group's first slot in the member list -- and the halo
+  // list (first slots of the groups passing the size cut), then the labels,
+  // which also fill the member list.  The sizes by label live in the label
+  // array (before its defaults), the first slots in sk1 and the labels in
+  // order in sv1 (behind 64 words: R + 1 first slots may reach N + 1); lists
+  // of larger groups go to the cell-sorted positions once k_label has read them.
   const int single = pl.single_halos ? 1 : 0;
   const uint64_t rcap = std::max<uint64_t>(single ? N : N / 2, 1);
-  const uint64_t nw = (N + 31) / 32;
-  uint32_t *gbits = rtab, *wpre = rtab + nw, *lsize = label;
+  uint32_t *lsize = label;
   uint32_t *offs = sk1, *glist = sv1 + 64;
   uint32_t *cursor = rtab;             // per label, from its group's first slot
   uint32_t *p32 = reinterpret_cast<uint32_t *>(pos4);
   // groups above kSegLds, kSegWave and four members (at most N / 4096,
   // N / 1024 and N / 5 of them)
   uint32_t *huge = p32 + 3 * N, *large = huge + N / kSegLds, *mid = large + N / kSegWave;
-  uint32_t *hflags = p32 + 2 * N;
+  uint32_t *hlist = pl.want_halos ? B.hhead : nullptr;
   if ((rc = tb(9))) return rc;
-  if ((rc = fill_u32(gbits, nw, 0u, st))) return rc;
   k_group_bits<<<gN, 256, 0, st>>>(NN, par, gsize, minorig, pos4, gbits, lsize, single, dV, dVB,
                                    (int)nvol);
   FOF_HIP(hipGetLastError());
-  k_word_counts<<<grid_for(nw), 256, 0, st>>>(nw, gbits, wpre);
+  const uint32_t runs = group_runs(nw), gb = (uint32_t)((nw + 256ull * runs - 1) / (256ull * runs));
+  GroupTot *gtot = static_cast<GroupTot *>(B.tmp);
+  k_group_sums<<<gb, 256, 0, st>>>(nw, runs, gbits, lsize, dV, dVB, (int)nvol, gtot);
   FOF_HIP(hipGetLastError());
-  if ((rc = scan_u32(wpre, wpre, nw, B.tmp, st))) return rc;
-  k_group_list<<<grid_for(nw), 256, 0, st>>>(nw, gbits, wpre, lsize, glist, offs, small + kSmR);
+  k_group_emit<<<gb, 256, 0, st>>>(nw, runs, gbits, lsize, dV, dVB, (int)nvol, gtot, glist, offs,
+                                   cursor, hlist, small);
   FOF_HIP(hipGetLastError());
-  if ((rc = scan_u32_count(offs, offs, rcap, small + kSmR, B.tmp, st))) return rc;
-  k_group_cursors<<<grid_for(rcap), 256, 0, st>>>(small + kSmR, glist, offs, cursor, small + kSmM);
-  FOF_HIP(hipGetLastError());
-  const bool direct = pl.direct_writes;
-  // direct writes and no minimum IDs: k_label writes label_out itself and
-  // k_out_init is not needed
-  const bool fused = direct && !r.d_minid;
-  k_label_init<<<tiles_for(N), 256, 0, st>>>(NN, dV, dVB, (int)nvol, fused ? nullptr : label,
-                                             fused ? nullptr : hsize, fused ? r.d_label : nullptr,
-                                             fused ? r.d_next : nullptr);
-  FOF_HIP(hipGetLastError());
+  if (!fused) {
+    k_label_init<<<tiles_for(N), 256, 0, st>>>(NN, dV, dVB, (int)nvol, label, hsize);
+    FOF_HIP(hipGetLastError());
+  }
   if ((rc = te(9))) return rc;
   if ((rc = tb(8))) return rc;
   const uint32_t glab = (uint32_t)((N + kLabTile - 1) / kLabTile);
@@ -4206,8 +4287,8 @@ static int enqueue_run(Run &r, hipStream_t st) {
   {
     // ring pairs (the partitioned way) in the free cell-sorted positions
     uint32_t *pidx = (r.d_next && !direct) ? p32 : nullptr;
-    k_ring<<<tiles_for(N), 256, 0, st>>>(small + kSmM, sk0, sv0, hsize, dV, dVB, (int)nvol,
-                                        r.d_next, pidx, p32 + N, nullptr);
+    k_ring<<<tiles_for(N), 256, 0, st>>>(small + kSmM, sk0, sv0, dVB, (int)nvol, r.d_next, pidx,
+                                        p32 + N);
     FOF_HIP(hipGetLastError());
     if (pidx && (rc = scatter_u32(p32, p32 + N, p32 + 2 * N, p32 + 3 * N, N, small + kSmM, N,
                                   r.d_next, 0u, B.tmp, st)))
@@ -4215,30 +4296,18 @@ static int enqueue_run(Run &r, hipStream_t st) {
   }
   if ((rc = te(11))) return rc;
   if (pl.want_halos) {
-    // halo starts: first slots of the groups passing the size cut, in label
-    // order
-    if ((rc = tb(12))) return rc;
-    k_halo_flags<<<grid_for(rcap), 256, 0, st>>>(small + kSmR, glist, offs, dV, dVB, (int)nvol,
-                                                  hflags);
-    FOF_HIP(hipGetLastError());
-    if ((rc = compact_flagged(hflags, rcap, small + kSmR, kFlag, p32, p32 + N, small + kSmH, B.tmp,
-                              st)))
-      return rc;
-    if ((rc = te(12))) return rc;
     if ((rc = tb(13))) return rc;
     const uint32_t gh = (uint32_t)std::min<uint64_t>((pl.Hbound * 64 + 255) / 256, 8192);
     if (r.d_mom)
-      k_halo_sums<true><<<gh, 256, 0, st>>>(small + kSmH, p32, sk0, sv0, hsize, dbase, stride,
+      k_halo_sums<true><<<gh, 256, 0, st>>>(small + kSmH, hlist, sk0, sv0, hsize, dbase, stride,
                                             offpos, offvel, dV, dVB, (int)nvol, r.d_halo, r.d_mom,
-                                            r.hcap, B.hhead, ctr);
+                                            r.hcap, B.hoff, ctr);
     else
-      k_halo_sums<false><<<gh, 256, 0, st>>>(small + kSmH, p32, sk0, sv0, hsize, dbase, stride,
+      k_halo_sums<false><<<gh, 256, 0, st>>>(small + kSmH, hlist, sk0, sv0, hsize, dbase, stride,
                                              offpos, offvel, dV, dVB, (int)nvol, r.d_halo, nullptr,
-                                             r.hcap, B.hhead, ctr);
+                                             r.hcap, B.hoff, ctr);
     FOF_HIP(hipGetLastError());
     if ((rc = te(13))) return rc;
-    k_halo_offsets<<<grid_for(nvol + 1), 256, 0, st>>>(small + kSmH, B.hhead, dVB, (int)nvol, B.hoff);
-    FOF_HIP(hipGetLastError());
   }
   return 0;
 }
@@ -4415,9 +4484,10 @@ static std::vector<uint32_t> split_volumes(const fof_volume_v1 *vols, uint32_t n
   return cut;
 }
 
-// The streams and events of a pipeline (its workspace grows with the calls).
-static int open_pipe(Pipe &pp) {
-  FOF_HIP(hipStreamCreate(&pp.stream));
+// A pipeline's side stream, made by its first eager call (0.2 ms; a context
+// that only replays graphs has none).
+static int open_side(Pipe &pp) {
+  if (pp.side) return 0;
   FOF_HIP(hipStreamCreate(&pp.side));
   FOF_HIP(hipEventCreateWithFlags(&pp.side_fork, hipEventDisableTiming));
   FOF_HIP(hipEventCreateWithFlags(&pp.side_join, hipEventDisableTiming));
@@ -4442,7 +4512,7 @@ static int run_call(fof_ctx *ctx, const fof_particles_v1 *P, const fof_volume_v1
   if (S.pipes.empty()) S.pipes.push_back(nullptr);  // pipeline 0 is S.main
   while (S.pipes.size() < K) {
     S.pipes.push_back(new Pipe);
-    if ((rc = open_pipe(*S.pipes.back()))) return rc;
+    FOF_HIP(hipStreamCreate(&S.pipes.back()->stream));
   }
   if (!S.sync_events) {  // created at context set-up; kept for safety
     FOF_HIP(hipEventCreateWithFlags(&S.fork, hipEventDisableTiming));
@@ -4489,6 +4559,8 @@ static int run_call(fof_ctx *ctx, const fof_particles_v1 *P, const fof_volume_v1
     for (uint32_t g = 0; g < K; g++) {
       runs[g].timing = with_timing && g == 0;
       runs[g].side = !graph && !with_timing;
+      if (runs[g].side)
+        if (int e = open_side(*runs[g].pp)) return e;
     }
     if (K > 1) FOF_HIP(hipEventRecord(S.fork, st));
     for (uint32_t g = 0; g < K; g++) {
@@ -4734,8 +4806,7 @@ uint8_t *g_scratch[64];  // per device, from hipGetSymbolAddress
 
 extern "C" int fof_engine_init(fof_ctx *ctx) {
   EngineState &S = ctx->st;
-  int rc = open_pipe(S.main);
-  if (rc) return rc;
+  FOF_HIP(hipStreamCreate(&S.main.stream));
   // everything a later call may need besides workspace: the fork / join and
   // timing events, and the fixed workspace's address on this device
   FOF_HIP(hipEventCreateWithFlags(&S.fork, hipEventDisableTiming));

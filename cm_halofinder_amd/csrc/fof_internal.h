@@ -57,9 +57,6 @@ void release(Scratch &s);
 size_t scan_tmp_bytes(uint64_t n);
 int scan_u32(const uint32_t *in, uint32_t *out, uint64_t n, void *tmp,
              hipStream_t st);
-// The same over min(*dn, n) values (the count left on the device).
-int scan_u32_count(const uint32_t *in, uint32_t *out, uint64_t n, const uint32_t *dn, void *tmp,
-                   hipStream_t st);
 
 // Passes over a list whose length an earlier kernel left in device memory
 // take the host-known capacity n and dn (the device count, n when dn is

@@ -76,14 +76,27 @@ __global__ __launch_bounds__(kBlock) void k_scan_reduce(const uint32_t *__restri
   if (threadIdx.x == 0) bsum[blockIdx.x] = s;
 }
 
-// in may alias out.  boff[b] is the exclusive prefix of tile b; boff[nb] is
-// the grand total, copied to out[n] by the last block.
+// in may alias out.  boff[b] is the exclusive prefix of tile b and boff[nb]
+// the grand total, or (RAW) boff[b] is tile b's own sum and each block adds up
+// those before it: up to kRawTiles tiles that spares the launch that scans
+// them.  The total goes to out[n] by the last block.
+constexpr uint32_t kRawTiles = 2048;
+
+template <bool RAW>
 __global__ __launch_bounds__(kBlock) void k_scan_down(const uint32_t *in, uint32_t *out,
                                                       uint64_t ncap, const uint32_t *dn,
                                                       const uint32_t *__restrict__ boff) {
   __shared__ uint32_t ws[kBlock / 64];
   const uint64_t n = dev_count(dn, ncap);
   if ((uint64_t)blockIdx.x * kTile > n) return;  // past the count (block sums are 0)
+  uint32_t before;
+  if (RAW) {
+    before = 0;
+    for (uint32_t b = threadIdx.x; b < blockIdx.x; b += kBlock) before += boff[b];
+    before = block_reduce(before, ws);
+  } else {
+    before = boff[blockIdx.x];
+  }
   const uint64_t base = (uint64_t)blockIdx.x * kTile + (uint64_t)threadIdx.x * kItems;
   uint32_t v[kItems];
   if (base + kItems <= n) {
@@ -101,7 +114,7 @@ __global__ __launch_bounds__(kBlock) void k_scan_down(const uint32_t *in, uint32
 #pragma unroll
   for (int i = 0; i < kItems; i++) s += v[i];
   uint32_t tot;
-  uint32_t pre = block_excl_scan(s, ws, &tot) + boff[blockIdx.x];
+  uint32_t pre = block_excl_scan(s, ws, &tot) + before;
 #pragma unroll
   for (int i = 0; i < kItems; i++) {
     uint32_t x = v[i];
@@ -119,7 +132,62 @@ __global__ __launch_bounds__(kBlock) void k_scan_down(const uint32_t *in, uint32
       if (base + i < n) out[base + i] = v[i];
   }
   if (threadIdx.x == 0 && (uint64_t)blockIdx.x == min(n / kTile, (uint64_t)gridDim.x - 1))
-    out[n] = boff[gridDim.x];
+    out[n] = before + tot;
+}
+
+// A scan of few elements by one workgroup, tile after tile.
+constexpr int kOneThreads = 1024;
+constexpr uint64_t kOneMax = 4ull * kOneThreads * kItems;
+
+__global__ __launch_bounds__(kOneThreads) void k_scan_one(const uint32_t *in, uint32_t *out,
+                                                          uint64_t ncap, const uint32_t *dn) {
+  __shared__ uint32_t ws[kOneThreads / 64];
+  const uint64_t n = dev_count(dn, ncap);
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  uint32_t carry = 0;
+  for (uint64_t t0 = 0; t0 < n; t0 += kOneThreads * kItems) {
+    const uint64_t base = t0 + (uint64_t)threadIdx.x * kItems;
+    uint32_t v[kItems], s = 0;
+    if (base + kItems <= n) {
+#pragma unroll
+      for (int q = 0; q < kItems / 4; q++) {
+        const uint4 t = reinterpret_cast<const uint4 *>(in + base)[q];
+        v[4 * q] = t.x, v[4 * q + 1] = t.y, v[4 * q + 2] = t.z, v[4 * q + 3] = t.w;
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < kItems; i++) v[i] = (base + i < n) ? in[base + i] : 0u;
+    }
+#pragma unroll
+    for (int i = 0; i < kItems; i++) s += v[i];
+    const uint32_t inc = wave_incl_scan(s);
+    __syncthreads();
+    if (lane == 63) ws[w] = inc;
+    __syncthreads();
+    uint32_t pre = carry + inc - s;
+#pragma unroll
+    for (int q = 0; q < kOneThreads / 64; q++) {
+      if (q < w) pre += ws[q];
+      carry += ws[q];
+    }
+#pragma unroll
+    for (int i = 0; i < kItems; i++) {
+      const uint32_t x = v[i];
+      v[i] = pre;
+      pre += x;
+    }
+    if (base + kItems <= n) {
+#pragma unroll
+      for (int q = 0; q < kItems / 4; q++)
+        reinterpret_cast<uint4 *>(out + base)[q] =
+            make_uint4(v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]);
+    } else {
+#pragma unroll
+      for (int i = 0; i < kItems; i++)
+        if (base + i < n) out[base + i] = v[i];
+    }
+  }
+  if (threadIdx.x == 0) out[n] = carry;
 }
 
 __global__ void k_scan_single(uint32_t *bsum, uint32_t nb) {
@@ -345,7 +413,7 @@ int scan_bsums(uint32_t *bs, uint64_t nb, hipStream_t st) {
   FOF_HIP(hipGetLastError());
   int rc = scan_bsums(next, nb2, st);
   if (rc) return rc;
-  k_scan_down<<<(uint32_t)nb2, kBlock, 0, st>>>(bs, bs, nb, nullptr, next);
+  k_scan_down<false><<<(uint32_t)nb2, kBlock, 0, st>>>(bs, bs, nb, nullptr, next);
   FOF_HIP(hipGetLastError());
   return 0;
 }
@@ -354,13 +422,25 @@ int scan_bsums(uint32_t *bs, uint64_t nb, hipStream_t st) {
 int scan_u32_dev(const uint32_t *in, uint32_t *out, uint64_t n, const uint32_t *dn, void *tmp,
                  hipStream_t st) {
   if (n == 0) return fill_u32(out, 1, 0u, st);
+  // launches are what a short scan costs: one up to kOneMax elements (8 us for
+  // 65536 against 3 x 5), two up to kRawTiles tiles
+  if (n <= kOneMax) {
+    k_scan_one<<<1, kOneThreads, 0, st>>>(in, out, n, dn);
+    FOF_HIP(hipGetLastError());
+    return 0;
+  }
   uint32_t *bs = static_cast<uint32_t *>(tmp);
   uint64_t nb = (n + kTile - 1) / kTile;
   k_scan_reduce<<<(uint32_t)nb, kBlock, 0, st>>>(in, n, dn, bs);
   FOF_HIP(hipGetLastError());
+  if (nb <= kRawTiles) {
+    k_scan_down<true><<<(uint32_t)nb, kBlock, 0, st>>>(in, out, n, dn, bs);
+    FOF_HIP(hipGetLastError());
+    return 0;
+  }
   int rc = scan_bsums(bs, nb, st);
   if (rc) return rc;
-  k_scan_down<<<(uint32_t)nb, kBlock, 0, st>>>(in, out, n, dn, bs);
+  k_scan_down<false><<<(uint32_t)nb, kBlock, 0, st>>>(in, out, n, dn, bs);
   FOF_HIP(hipGetLastError());
   return 0;
 }
@@ -371,11 +451,6 @@ size_t scan_tmp_bytes(uint64_t n) { return scan_levels_bytes(n) + 256; }
 
 int scan_u32(const uint32_t *in, uint32_t *out, uint64_t n, void *tmp, hipStream_t st) {
   return scan_u32_dev(in, out, n, nullptr, tmp, st);
-}
-
-int scan_u32_count(const uint32_t *in, uint32_t *out, uint64_t n, const uint32_t *dn, void *tmp,
-                   hipStream_t st) {
-  return scan_u32_dev(in, out, n, dn, tmp, st);
 }
 
 size_t compact_tmp_bytes(uint64_t n) { return scan_levels_bytes(n) + 256; }

@@ -161,12 +161,13 @@ typedef struct fof_halo_v1 {
  * (HIP events on the library's stream) of span k of the last call, 0 when the
  * span did not run:
  *   0 cell keys                     1 bucket offsets (scan) or key sort (sparse)
- *   2 partitions + bucket sort      3 union-find init
+ *   2 partitions + bucket sort      3 union-find init (occupied-cell addressing;
+ *                                     else part of span 2)
  *   4 sub-cell sort of dense cells  5 pair tests, sparse cells
  *     of 256 particles or more
  *   6 pair tests, dense cells of    7 union-find flatten + group minima
  *     256 particles or more
- *   8 labels, member list filled    9 label defaults + group list
+ *   8 labels, member list filled    9 group and halo lists
  *  10 members sorted in each group 11 ring
  *  12 halo list                    13 halo sums
  *  14 output copies                15 pair tests, dense cells below 256
