@@ -3671,6 +3671,21 @@ struct Bufs {
 
 constexpr size_t kSmallBytes = 256 + (size_t)kCtrSlots * kCtrStride * 8;
 
+// The head block of a workspace: counts, flags and counters (zero at first),
+// halo offsets, volume table, variable-l tables, volume starts -- one upload
+// ahead of a call's kernels; the first two are read back in one copy after
+// them.  Byte offsets in it:
+struct HeadLayout {
+  size_t hoff, vols, vtab, vbeg, bytes;
+  HeadLayout(uint32_t nvol, size_t vt_entries) {
+    hoff = kSmallBytes;
+    vols = (hoff + (nvol + 1) * 8ull + 15) & ~(size_t)15;
+    vtab = vols + nvol * sizeof(VolDev);
+    vbeg = vtab + vt_entries * sizeof(double);
+    bytes = vbeg + (nvol + 1) * 4ull;
+  }
+};
+
 static size_t layout(const Plan &pl, uint8_t *base, Bufs &b) {
   Carve c;
   c.base = base;
@@ -3687,12 +3702,16 @@ static size_t layout(const Plan &pl, uint8_t *base, Bufs &b) {
   b.sortbuf = c.take<uint32_t>(16 * q4 + 256);
   b.dense = c.take<uint32_t>(2 * pl.ndense_cap * 4 + 64);
   b.tmp = c.take<void>(pl.tmpb);
-  b.vols = c.take<VolDev>(pl.nvol * sizeof(VolDev));
-  b.vtab = c.take<double>(pl.vt_entries * sizeof(double) + 8);
-  b.vbeg = c.take<uint32_t>((pl.nvol + 1) * 4 + 64);
-  b.small = c.take<uint32_t>(kSmallBytes);
+  const HeadLayout hl(pl.nvol, pl.vt_entries);
+  uint8_t *head = c.take<uint8_t>(hl.bytes + 64);
+  if (head) {
+    b.small = reinterpret_cast<uint32_t *>(head);
+    b.hoff = reinterpret_cast<uint64_t *>(head + hl.hoff);
+    b.vols = reinterpret_cast<VolDev *>(head + hl.vols);
+    b.vtab = reinterpret_cast<double *>(head + hl.vtab);
+    b.vbeg = reinterpret_cast<uint32_t *>(head + hl.vbeg);
+  }
   b.hhead = c.take<uint32_t>(pl.Hbound * 4 + 64);
-  b.hoff = c.take<uint64_t>((pl.nvol + 1) * 8 + 64);
   b.cnt = pl.sparse ? c.take<uint32_t>(N * 4 + 64) : nullptr;
   b.part = pl.sparse ? nullptr
                      : c.take<uint32_t>(((pl.hist_in_fine ? 0 : 2 * pl.nA) + 2 * pl.nB +
@@ -3825,26 +3844,26 @@ static int make_plan(const fof_particles_v1 *P, const fof_volume_v1 *vols, uint3
   return 0;
 }
 
-// The volume table (VolDev[nvol], varlink tables, volume starts) as uploaded.
-static void build_vblob(const Plan &pl, const Bufs &b, std::vector<uint8_t> &blob) {
-  const size_t nv = pl.nvol * sizeof(VolDev);
-  blob.resize(nv + pl.vt_entries * sizeof(double) + (pl.nvol + 1) * 4);
+// The volume table of the head block as uploaded.
+static void build_vols(const Plan &pl, const Bufs &b, uint8_t *vols) {
   for (uint32_t v = 0; v < pl.nvol; v++) {
     VolDev V = pl.hv[v].d;
     if (pl.vt_off[v] != ~0u) V.vtab = b.vtab + pl.vt_off[v];
-    memcpy(&blob[v * sizeof(VolDev)], &V, sizeof(VolDev));
+    memcpy(vols + v * sizeof(VolDev), &V, sizeof(VolDev));
   }
-  if (pl.vt_entries) memcpy(&blob[nv], pl.vt_host.data(), pl.vt_entries * sizeof(double));
-  memcpy(&blob[nv + pl.vt_entries * sizeof(double)], pl.vbeg.data(), (pl.nvol + 1) * 4);
 }
 
-static int upload_vblob(const Plan &pl, const Bufs &b, const std::vector<uint8_t> &blob,
-                        hipStream_t st) {
-  const size_t nv = pl.nvol * sizeof(VolDev), nt = pl.vt_entries * sizeof(double);
-  FOF_HIP(hipMemcpyAsync(b.vols, blob.data(), nv, hipMemcpyHostToDevice, st));
-  if (nt) FOF_HIP(hipMemcpyAsync(b.vtab, blob.data() + nv, nt, hipMemcpyHostToDevice, st));
-  FOF_HIP(hipMemcpyAsync(b.vbeg, blob.data() + nv + nt, (pl.nvol + 1) * 4, hipMemcpyHostToDevice,
-                         st));
+// The head block in the pipeline's page-locked buffer (its last upload is
+// done: every call ends synchronised).
+static int build_head(const Plan &pl, const Bufs &b, Pipe &pp) {
+  const HeadLayout hl(pl.nvol, pl.vt_entries);
+  int rc;
+  if ((rc = ensure_host(pp.up, hl.bytes)) || (rc = ensure_host(pp.down, hl.vols))) return rc;
+  uint8_t *h = static_cast<uint8_t *>(pp.up.ptr);
+  memset(h, 0, hl.vols);
+  build_vols(pl, b, h + hl.vols);
+  if (pl.vt_entries) memcpy(h + hl.vtab, pl.vt_host.data(), pl.vt_entries * sizeof(double));
+  memcpy(h + hl.vbeg, pl.vbeg.data(), (pl.nvol + 1) * 4);
   return 0;
 }
 
@@ -3921,18 +3940,18 @@ static int prepare_run(Run &r, Pipe &pp, const fof_particles_v1 *P, const fof_vo
   r.d_halo = pl.want_halos ? (direct ? out->halos : r.B.st_halo) : nullptr;
   r.d_mom = pl.want_mom ? (direct ? out->moments : r.B.st_mom) : nullptr;
   r.hcap = r.d_halo ? (direct ? out->halo_cap : pl.Hstage) : 0;
-  build_vblob(pl, r.B, pp.vblob);
-  pp.hres.resize(kSmallBytes + (nv + 1) * 8);
-  return 0;
+  return build_head(pl, r.B, pp);
 }
 
-// Uploads that precede a pipeline's kernels: the volume table and, for
+// Uploads that precede a pipeline's kernels: the head block and, for
 // host-resident input, the particle records.
 static int upload_run(Run &r, hipStream_t st) {
   if (r.pl.N == 0) return 0;
   if (r.host_src)
     FOF_HIP(hipMemcpyAsync(r.B.input, r.host_src, r.pl.N * r.pl.stride, hipMemcpyHostToDevice, st));
-  return upload_vblob(r.pl, r.B, r.pp->vblob, st);
+  const HeadLayout hl(r.pl.nvol, r.pl.vt_entries);
+  FOF_HIP(hipMemcpyAsync(r.B.small, r.pp->up.ptr, hl.bytes, hipMemcpyHostToDevice, st));
+  return 0;
 }
 
 // Every kernel of a pipeline, in stream order.  Without a variable linking
@@ -3949,7 +3968,7 @@ static int enqueue_run(Run &r, hipStream_t st) {
   const uint8_t *dbase = r.dbase;
   uint32_t *small = B.small;
   unsigned long long *ctr = reinterpret_cast<unsigned long long *>(small + kSmCtr);
-  uint32_t *hsm = reinterpret_cast<uint32_t *>(pp.hres.data());
+  uint32_t *hsm = static_cast<uint32_t *>(pp.down.ptr);
   const bool timing = r.timing;
   if (timing && !pp.events) {
     for (auto &e : pp.ev) FOF_HIP(hipEventCreate(&e));
@@ -3972,8 +3991,6 @@ static int enqueue_run(Run &r, hipStream_t st) {
     }
     return 0;
   };
-  if ((rc = fill_u32(small, kSmallBytes / 4, 0u, st))) return rc;
-
   if (pl.varlink) {
     // A variable l: the sub-cell size follows the smallest l of any occupied
     // cell (only occupied cells are home cells of a pair), not of the table.
@@ -3991,8 +4008,10 @@ static int enqueue_run(Run &r, hipStream_t st) {
       memcpy(&l2, &hmin[v], 8);
       set_subcells(pl.hv[v].d, l2);
     }
-    build_vblob(pl, B, pp.vblob);
-    if ((rc = upload_vblob(pl, B, pp.vblob, st))) return rc;
+    const HeadLayout hl(nvol, pl.vt_entries);
+    build_vols(pl, B, static_cast<uint8_t *>(pp.up.ptr) + hl.vols);
+    FOF_HIP(hipMemcpyAsync(B.vols, static_cast<uint8_t *>(pp.up.ptr) + hl.vols,
+                           nvol * sizeof(VolDev), hipMemcpyHostToDevice, st));
   }
 
   const VolDev *dV = B.vols;
@@ -4316,16 +4335,15 @@ static int enqueue_run(Run &r, hipStream_t st) {
 // pipeline's kernels, on the same stream).
 static int readback_run(Run &r, hipStream_t st) {
   if (r.pl.N == 0) return 0;
-  FOF_HIP(hipMemcpyAsync(r.pp->hres.data(), r.B.small, kSmallBytes, hipMemcpyDeviceToHost, st));
-  if (r.pl.want_halos)
-    FOF_HIP(hipMemcpyAsync(r.pp->hres.data() + kSmallBytes, r.B.hoff, (r.pl.nvol + 1) * 8,
-                           hipMemcpyDeviceToHost, st));
+  const HeadLayout hl(r.pl.nvol, r.pl.vt_entries);
+  FOF_HIP(hipMemcpyAsync(r.pp->down.ptr, r.B.small, r.pl.want_halos ? hl.vols : kSmallBytes,
+                         hipMemcpyDeviceToHost, st));
   return 0;
 }
 
 static uint32_t run_nhalos(const Run &r) {
   if (r.pl.N == 0 || !r.pl.want_halos) return 0;
-  return reinterpret_cast<const uint32_t *>(r.pp->hres.data())[kSmH];
+  return static_cast<const uint32_t *>(r.pp->down.ptr)[kSmH];
 }
 
 // Staged halos (and moments) of the pipelines of a call into the output, at
@@ -4589,10 +4607,19 @@ static int run_call(fof_ctx *ctx, const fof_particles_v1 *P, const fof_volume_v1
     }
     return 0;
   };
-  // uploads, on the main stream ahead of everything
+  // uploads, on the main stream ahead of everything; they leave from the
+  // pipelines' page-locked buffers, so an early return waits for them too
+  struct Settle {
+    hipStream_t st;
+    bool on;
+    ~Settle() {
+      if (on) (void)hipStreamSynchronize(st);
+    }
+  } settle{st, true};
   for (auto &r : runs)
     if ((rc = upload_run(r, st))) return rc;
-  FOF_HIP(hipEventRecord(S.t0, st));
+  const bool timed = timing || wall_ms;
+  if (timed) FOF_HIP(hipEventRecord(S.t0, st));
   uint32_t graph_state = 0;
   if (graph) {
     Sig sig;
@@ -4633,12 +4660,13 @@ static int run_call(fof_ctx *ctx, const fof_particles_v1 *P, const fof_volume_v1
   } else {
     if ((rc = enqueue_all(timing))) return rc;
   }
-  FOF_HIP(hipEventRecord(S.t1, st));
+  if (timed) FOF_HIP(hipEventRecord(S.t1, st));
   for (auto &r : runs)
     if ((rc = readback_run(r, st))) return rc;
   FOF_HIP(hipStreamSynchronize(st));
+  settle.on = false;
   float tot_ms = 0;
-  FOF_HIP(hipEventElapsedTime(&tot_ms, S.t0, S.t1));
+  if (timed) FOF_HIP(hipEventElapsedTime(&tot_ms, S.t0, S.t1));
   if (wall_ms) *wall_ms = tot_ms;
 
   // ---- results ----
@@ -4646,7 +4674,7 @@ static int run_call(fof_ctx *ctx, const fof_particles_v1 *P, const fof_volume_v1
   bool dom_err = false;
   for (auto &r : runs) {
     if (r.pl.N == 0) continue;
-    const uint32_t *hsm = reinterpret_cast<const uint32_t *>(r.pp->hres.data());
+    const uint32_t *hsm = static_cast<const uint32_t *>(r.pp->down.ptr);
     dom_err = dom_err || hsm[kSmErr];
     H += run_nhalos(r);
   }
@@ -4660,7 +4688,7 @@ static int run_call(fof_ctx *ctx, const fof_particles_v1 *P, const fof_volume_v1
   if (out->halo_offsets && want_halos) {
     uint64_t base = 0;
     for (auto &r : runs) {
-      const uint64_t *ho = reinterpret_cast<const uint64_t *>(r.pp->hres.data() + kSmallBytes);
+      const uint64_t *ho = reinterpret_cast<const uint64_t *>(static_cast<const uint8_t *>(r.pp->down.ptr) + kSmallBytes);
       for (uint32_t v = 0; v < r.pl.nvol; v++) out->halo_offsets[r.v0 + v] = base + (r.pl.N ? ho[v] : 0);
       base += run_nhalos(r);
     }
@@ -4693,7 +4721,7 @@ static int run_call(fof_ctx *ctx, const fof_particles_v1 *P, const fof_volume_v1
     unsigned long long hc[kCtrStride] = {};
     for (auto &r : runs) {
       if (r.pl.N == 0) continue;
-      const uint32_t *hsm = reinterpret_cast<const uint32_t *>(r.pp->hres.data());
+      const uint32_t *hsm = static_cast<const uint32_t *>(r.pp->down.ptr);
       const unsigned long long *hcs = reinterpret_cast<const unsigned long long *>(hsm + kSmCtr);
       for (int q = 0; q < kCtrSlots; q++)
         for (int k = 0; k < kCtrStride; k++) hc[k] += hcs[q * kCtrStride + k];
@@ -4844,6 +4872,8 @@ extern "C" int fof_engine_run_noalloc(fof_ctx *ctx, const fof_particles_v1 *P,
 extern "C" uint64_t fof_engine_noalloc_bytes(void) { return kNoAllocBytes; }
 
 static void free_pipe(Pipe &pp) {
+  release_host(pp.up);
+  release_host(pp.down);
   release(pp.arena);
   release(pp.hash);
   if (pp.events)

@@ -51,6 +51,9 @@ struct Scratch {
 };
 int ensure(Scratch &s, size_t bytes);
 void release(Scratch &s);
+// The same for page-locked host memory.
+int ensure_host(Scratch &s, size_t bytes);
+void release_host(Scratch &s);
 
 // Exclusive scan of n u32 values in[0..n) into out[0..n]; out[n] = total.
 // tmp must hold scan_tmp_bytes(n).
@@ -97,8 +100,8 @@ struct Pipe {
   hipStream_t stream = nullptr;
   Scratch arena;  // every buffer of a call
   Scratch hash;   // occupied-cell hash table (sized once the cell count is known)
-  std::vector<uint8_t> vblob;  // volume table, varlink tables, volume starts
-  std::vector<uint8_t> hres;   // counts, flags and counters read back
+  // page-locked: what a call uploads ahead of its kernels and reads back
+  Scratch up, down;
   hipEvent_t ev[2 * FOF_NPHASE] = {};
   bool events = false;
   // a side stream of the link kernels, forked from and joined to `stream`

@@ -600,6 +600,25 @@ int ensure(Scratch &s, size_t bytes) {
   return 0;
 }
 
+int ensure_host(Scratch &s, size_t bytes) {
+  if (bytes <= s.bytes) return 0;
+  release_host(s);
+  const size_t b = (bytes + 4095) / 4096 * 4096;
+  if (hipHostMalloc(&s.ptr, b, 0) != hipSuccess) {
+    (void)hipGetLastError();
+    s.ptr = nullptr;
+    return FOF_E_NOMEM;
+  }
+  s.bytes = b;
+  return 0;
+}
+
+void release_host(Scratch &s) {
+  if (s.ptr) (void)hipHostFree(s.ptr);
+  s.ptr = nullptr;
+  s.bytes = 0;
+}
+
 void release(Scratch &s) {
   if (s.ptr) (void)hipFree(s.ptr);
   s.ptr = nullptr;
