@@ -2221,13 +2221,13 @@ __device__ __forceinline__ void small_cell(SmallLds &S, uint32_t sA, uint32_t nA
                                            uint32_t nbS, uint32_t nbN,
                                            const float4 *__restrict__ pos4, const Grid &G,
                                            uint32_t *__restrict__ par, uint32_t nxt,
-                                           uint32_t &nS, uint32_t &nE, uint32_t &tests,
+                                           uint32_t part, uint32_t parts, uint32_t &nS, uint32_t &nE, uint32_t &tests,
                                            uint32_t &rechecks) {
   const uint32_t lane = threadIdx.x & 63;
   volatile uint32_t *const lp = S.lp;
   // (A, A)
   small_cell_own<NW>(S, nA, R, rechecks);
-  tests += (lane == 0) ? nA * (nA - 1) / 2 : 0u;
+  tests += (lane == 0 && part == 0) ? nA * (nA - 1) / 2 : 0u;
   wave_sync();
   // the next cell's bounds (its index has arrived by now)
   if (nxt != kNone) nS = G.start[nxt], nE = G.start[nxt + 1];
@@ -2372,7 +2372,7 @@ __device__ __forceinline__ void small_cell(SmallLds &S, uint32_t sA, uint32_t nA
       qn -= 64;
     }
   };
-  for (uint32_t g0 = 0; g0 < total; g0 += 128) {
+  for (uint32_t g0 = 128 * part; g0 < total; g0 += 128 * parts) {
     const uint32_t ga = g0 + lane, gb = g0 + 64 + lane;
     const bool va = ga < total, vb = gb < total;
     const uint32_t ja = locate(g0);
@@ -2399,6 +2399,18 @@ __device__ __forceinline__ void small_cell(SmallLds &S, uint32_t sA, uint32_t nA
 // 1024^3 box: 33.4 ms with blocks of 8 partners and no cap (134 VGPRs, three
 // waves), 28.3 ms at four waves, 25.0 ms with blocks of 4 at five, 23.5 ms
 // with the x, y, z tables; six waves (80 VGPRs) spill enough to take 31.4 ms.
+// Waves a cell's neighbour particles are split over while there are few cells
+// (each part links the cell's own particles anew).  The kernel then waits for
+// its largest cell, whose candidates one wave tests 64 at a time: in the 64^3
+// box 230 particles against 1096 candidates took all of its 290 us, eight times
+// the mean cell.  Eight parts while all still run at once, beyond that only for
+// the larger cells: 64^3 box (815 cells) 291 -> 125 us, 144^3 (8e3) 427 -> 269,
+// 192^3 (2.2e4) 565 -> 434, 256^3 (4.2e4) 881 -> 754; 512^3 (3.2e5) is not split
+// (3.6 ms either way).
+__device__ __forceinline__ uint32_t small_parts(uint32_t cells) {
+  return cells <= 512u ? 8u : cells <= 16384u ? 4u : cells <= 49152u ? 2u : 1u;
+}
+
 __global__ __launch_bounds__(64 * kSmallWaves) __attribute__((amdgpu_waves_per_eu(5))) void k_link_small(
     const uint32_t *__restrict__ dense, const uint32_t *__restrict__ ndense,
     const float4 *__restrict__ pos4, const Grid G, uint32_t T, uint32_t *__restrict__ par,
@@ -2411,18 +2423,28 @@ __global__ __launch_bounds__(64 * kSmallWaves) __attribute__((amdgpu_waves_per_e
   SmallLds &S = Sall[wv];
   uint32_t tests = 0, rechecks = 0;
   const uint32_t lane = threadIdx.x & 63;
-  const uint32_t nd = *ndense;
+  // work items: (cell, part), `parts` (a power of two) to a cell
+  const uint32_t parts = small_parts(*ndense);
+  const uint32_t psh = (uint32_t)__builtin_ctz(parts);
+  const uint32_t nd = *ndense << psh;
   const uint32_t w0 = blockIdx.x * kSmallWaves + wv;
   const uint32_t ws = gridDim.x * kSmallWaves;
   // bounds of the wave's next cell, fetched ahead
   uint32_t nS = 0, nE = 0;
   if (w0 < nd) {
-    const uint32_t c = dense[w0];
+    const uint32_t c = dense[w0 >> psh];
     nS = G.start[c], nE = G.start[c + 1];
   }
   for (uint32_t d = w0; d < nd; d += ws) {
+    const uint32_t part = d & (parts - 1);
     const uint32_t sA = nS, nA = nE - nS;  // T <= nA < kBigCell
-    const uint32_t cN = (d + ws < nd) ? dense[d + ws] : 0u;
+    const uint32_t cN = (d + ws < nd) ? dense[(d + ws) >> psh] : 0u;
+    // only cells worth it: the others are their first part's alone
+    const uint32_t mine = parts == 8 ? 8u : min(parts, nA >= 160 ? 4u : nA >= 96 ? 2u : 1u);
+    if (part >= mine) {
+      if (d + ws < nd) nS = G.start[cN], nE = G.start[cN + 1];
+      continue;
+    }
     const VolDev &V = vols[vol_of(vbeg, nvol, sA)];
     const float4 p0 = pos4[sA];
     for (uint32_t i = lane; i < nA; i += 64) {
@@ -2448,10 +2470,10 @@ __global__ __launch_bounds__(64 * kSmallWaves) __attribute__((amdgpu_waves_per_e
     wave_sync();
     const uint32_t nw = (nA + 63) >> 6;
     const uint32_t nxt = (d + ws < nd) ? cN : kNone;
-    if (nw <= 1) small_cell<1>(S, sA, nA, V, cp, R, nbS, nbN, pos4, G, par, nxt, nS, nE, tests, rechecks);
-    else if (nw == 2) small_cell<2>(S, sA, nA, V, cp, R, nbS, nbN, pos4, G, par, nxt, nS, nE, tests, rechecks);
-    else if (nw == 3) small_cell<3>(S, sA, nA, V, cp, R, nbS, nbN, pos4, G, par, nxt, nS, nE, tests, rechecks);
-    else small_cell<4>(S, sA, nA, V, cp, R, nbS, nbN, pos4, G, par, nxt, nS, nE, tests, rechecks);
+    if (nw <= 1) small_cell<1>(S, sA, nA, V, cp, R, nbS, nbN, pos4, G, par, nxt, part, mine, nS, nE, tests, rechecks);
+    else if (nw == 2) small_cell<2>(S, sA, nA, V, cp, R, nbS, nbN, pos4, G, par, nxt, part, mine, nS, nE, tests, rechecks);
+    else if (nw == 3) small_cell<3>(S, sA, nA, V, cp, R, nbS, nbN, pos4, G, par, nxt, part, mine, nS, nE, tests, rechecks);
+    else small_cell<4>(S, sA, nA, V, cp, R, nbS, nbN, pos4, G, par, nxt, part, mine, nS, nE, tests, rechecks);
   }
   add_counters(ctr, kCtrTestsSmall, tests, rechecks);
 }
@@ -4203,9 +4225,18 @@ static int enqueue_run(Run &r, hipStream_t st) {
     if ((rc = tb(6))) return rc;
     constexpr int kRB = 448;
     const uint32_t ra = std::min(maxbins, (uint32_t)kMaxRuns);
-    k_link_dense<256, 6, kMaxRuns, kRB><<<gbig, 256, dense_lds(ra, kRB), st>>>(
-        dbig, small + kSmNBig, pos4, G, runend, fine, rtoff, rtab, T, par, dV, dVB, (int)nvol, ctr,
-        ra, small + kSmDq);
+    // wider workgroups while there are too few cells to fill the chip and the
+    // largest one's chain is what is waited for: 31^3, 64^3, 144^3, 192^3 and
+    // 256^3 boxes 134, 249, 525, 530 and 777 us with 256 threads, 92, 203, 436,
+    // 499 and 872 with 512, 74, 186, 420, - and 1418 with 1024
+    auto link_dense = [&](auto kernel, int nt) {
+      kernel<<<gbig, nt, dense_lds(ra, kRB), st>>>(dbig, small + kSmNBig, pos4, G, runend, fine,
+                                                   rtoff, rtab, T, par, dV, dVB, (int)nvol, ctr, ra,
+                                                   small + kSmDq);
+    };
+    if (N <= (1u << 20)) link_dense(k_link_dense<1024, 4, kMaxRuns, kRB>, 1024);
+    else if (N <= (1u << 23)) link_dense(k_link_dense<512, 6, kMaxRuns, kRB>, 512);
+    else link_dense(k_link_dense<256, 6, kMaxRuns, kRB>, 256);
     FOF_HIP(hipGetLastError());
     if ((rc = te(6))) return rc;
   }
