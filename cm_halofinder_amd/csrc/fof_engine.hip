@@ -13,7 +13,7 @@
 //                    (coarse, then 256 fine buckets of 2^14 cells), then a
 //                    counting sort per fine bucket -> cell starts, dense-cell
 //                    lists and float4 {x,y,z,index} in cell order
-//                    (sparse addressing: composite keys, radix sort, hash)
+//                    (sparse addressing: composite keys, radix sort, cell list)
 //   4 k_subsort      cells with >= max(T, 256) particles: counting sort by
 //                    sub-cell; sub-cells have side <= l/sqrt(3), so each is a
 //                    clique and its particles start in one union-find set
@@ -170,31 +170,16 @@ __device__ __forceinline__ uint32_t cell_id(const VolDev &V, int ix, int iy, int
 
 // Cell addressing.  Dense: a table of cell starts over every cell of every
 // volume (cell id = cbeg + linear index).  Sparse: only occupied cells, in
-// (volume, linear index) order, found through an open-addressing hash table
-// keyed by the composite key (volume << volshift) | linear index.
-// A hash slot: the composite key (empty = ~0) and the cell index side by side,
-// so that a probe is one 16-byte load (the table is gigabytes: every probe
-// misses the caches).
-struct __align__(16) HEntry {
-  unsigned long long k;
-  unsigned long long v;
-};
-
+// (volume, linear index) order, listed with their composite keys
+// (volume << volshift) | linear index and found by binary search.
 struct Grid {
-  const uint32_t *start;           // cell start offsets (+1 entry)
-  const struct HEntry *htab;       // sparse: hash table (key, cell index)
-  const uint32_t *cell_of;         // sparse: cell of each sorted particle
-  unsigned long long hmask;
+  const uint32_t *start;       // cell start offsets (+1 entry)
+  const uint32_t *cell_of;     // sparse: cell of each sorted particle
+  const uint32_t *klo, *khi;   // sparse: key of each cell
+  const uint32_t *ncell;       // sparse: cells in the list
   int sparse;
   int volshift;
 };
-
-__device__ __forceinline__ unsigned long long mix64d(unsigned long long z) {
-  z += 0x9E3779B97F4A7C15ull;
-  z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
-  z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
-  return z ^ (z >> 31);
-}
 
 __device__ __forceinline__ unsigned long long comp_key(const Grid &G, const VolDev &V, int ix,
                                                        int iy, int iz) {
@@ -203,56 +188,37 @@ __device__ __forceinline__ unsigned long long comp_key(const Grid &G, const VolD
           (unsigned)ix);
 }
 
-// Home slot of a key: four consecutive x-cells (keys k with one k >> 2) get
-// four consecutive slots, so that the three cells of a neighbour row mostly
-// share one 64-byte line of the table.
-__device__ __forceinline__ unsigned long long hslot(const Grid &G, unsigned long long k) {
-  return ((mix64d(k >> 2) << 2) | (k & 3ull)) & G.hmask;
+__device__ __forceinline__ unsigned long long cell_key(const Grid &G, uint32_t c) {
+  return (unsigned long long)G.klo[c] | ((unsigned long long)G.khi[c] << 32);
 }
 
-__device__ __forceinline__ uint32_t hlookup(const Grid &G, unsigned long long k) {
-  unsigned long long i = hslot(G, k);
-  for (;;) {
-    const HEntry h = G.htab[i];
-    const unsigned long long kk = h.k;
-    if (kk == k) return (uint32_t)h.v;
-    if (kk == ~0ull) return kNone;
-    i = (i + 1) & G.hmask;
+// First occupied cell with a key >= k.
+__device__ __forceinline__ uint32_t cell_lower(const Grid &G, uint32_t U, unsigned long long k) {
+  uint32_t lo = 0, hi = U;
+  while (lo < hi) {
+    const uint32_t mid = (lo + hi) >> 1;
+    if (cell_key(G, mid) < k) lo = mid + 1;
+    else hi = mid;
   }
+  return lo;
 }
 
 // Cell index of (ix,iy,iz) (in range), kNone when a sparse cell is empty.
 __device__ __forceinline__ uint32_t cell_index(const Grid &G, const VolDev &V, int ix, int iy,
                                                int iz) {
   if (!G.sparse) return cell_id(V, ix, iy, iz);
-  return hlookup(G, comp_key(G, V, ix, iy, iz));
+  const uint32_t U = *G.ncell;
+  const unsigned long long k = comp_key(G, V, ix, iy, iz);
+  const uint32_t c = cell_lower(G, U, k);
+  return c < U && cell_key(G, c) == k ? c : kNone;
 }
 
-// Particle range covering cells (x0..x1, iy, iz).  Sparse: the occupied
-// cells among consecutive keys are consecutive in the cell list.
+// Particle range covering cells (x0..x1, iy, iz) of a dense grid.
 __device__ __forceinline__ void row_range(const Grid &G, const VolDev &V, int x0, int x1, int iy,
                                           int iz, uint32_t &r0, uint32_t &r1) {
-  if (!G.sparse) {
-    const uint32_t c0 = cell_id(V, x0, iy, iz);
-    r0 = G.start[c0];
-    r1 = G.start[c0 + (uint32_t)(x1 - x0) + 1];
-    return;
-  }
-  uint32_t lo = kNone, hi = kNone;
-  const unsigned long long k0 = comp_key(G, V, x0, iy, iz);
-  for (int x = 0; x <= x1 - x0; x++) {
-    const uint32_t c = hlookup(G, k0 + (unsigned long long)x);
-    if (c != kNone) {
-      if (lo == kNone) lo = c;
-      hi = c;
-    }
-  }
-  if (lo == kNone) {
-    r0 = r1 = 0;
-    return;
-  }
-  r0 = G.start[lo];
-  r1 = G.start[hi + 1];
+  const uint32_t c0 = cell_id(V, x0, iy, iz);
+  r0 = G.start[c0];
+  r1 = G.start[c0 + (uint32_t)(x1 - x0) + 1];
 }
 
 // Squared linking length of a home cell: constant, or the variable rule
@@ -1029,67 +995,55 @@ __global__ __launch_bounds__(256) void k_cell_flags(uint32_t N, const uint32_t *
     flags[x] = (x == 0 || sklo[x] != sklo[x - 1] || skhi[x] != skhi[x - 1]) ? kFlag : 0u;
 }
 
-// Per occupied cell: close the start list, record each particle's cell,
-// insert the key into the hash table, list dense cells.
+// Per occupied cell: close the start list, record the cell's key, list dense
+// cells.  (Each particle's cell comes with the list; the dense cells' 26
+// neighbours are found by binary search over the keys.  Writing the former
+// here, one thread to a cell's particles, inserting the keys into a hash table
+// for the latter and appending to the lists wave by wave took 1.0 ms for the
+// 9.8e6 cells of a lightcone.)
+constexpr uint32_t kCellTile = 4096;  // cells of a block: two appends a block at most
+
 __global__ __launch_bounds__(256) void k_cells_finish(
     const uint32_t *__restrict__ dU, uint32_t N, uint32_t *__restrict__ cstart,
-    const uint32_t *__restrict__ sklo, const uint32_t *__restrict__ skhi, Grid G,
-    HEntry *__restrict__ htab,
-    uint32_t *__restrict__ cell_of, const VolDev *__restrict__ vols,
+    const uint32_t *__restrict__ sklo, const uint32_t *__restrict__ skhi,
+    uint32_t *__restrict__ klo, uint32_t *__restrict__ khi,
+    const VolDev *__restrict__ vols,
     const uint32_t *__restrict__ vbeg, int nvol, uint32_t T, uint32_t *__restrict__ dense,
     uint32_t *__restrict__ ndense, uint32_t *__restrict__ dbig, uint32_t *__restrict__ nbig) {
+  // the tile's dense cells: the small ones from the front, the others from the back
+  __shared__ uint16_t lst[kCellTile];
+  __shared__ uint32_t cnt[2], base[2];
   const uint32_t U = *dU;
-  const uint32_t lane = threadIdx.x & 63;
-  int hint = 0;
-  // wave-uniform trip count: the dense-cell lists are appended per wave
-  for (uint32_t cb = blockIdx.x * blockDim.x + (threadIdx.x & ~63u); cb < U;
-       cb += gridDim.x * blockDim.x) {
-    const uint32_t c = cb + lane;
-    bool sml = false, big = false;
-    if (c < U) {
-      const uint32_t s = cstart[c], e = (c + 1 < U) ? cstart[c + 1] : N;
-      if (c + 1 == U) cstart[U] = N;
-      for (uint32_t x = s; x < e; x++) cell_of[x] = c;
-      const unsigned long long k = (unsigned long long)sklo[s] | ((unsigned long long)skhi[s] << 32);
-      unsigned long long i = hslot(G, k);
-      for (;;) {
-        if (atomicCAS(&htab[i].k, ~0ull, k) == ~0ull) {
-          htab[i].v = c;
-          break;
-        }
-        i = (i + 1) & G.hmask;
-      }
-      const VolDev &V = vols[vol_of_sorted(vbeg, nvol, s, hint)];  // s ascends with c
-      if (e - s >= T) {  // dense: below kBigCell always, from it only with sub-cells
-        sml = e - s < kBigCell;
-        big = !sml && V.m[0] > 0;
-      }
-    }
-    const unsigned long long bs = __ballot(sml), bb = __ballot(big);
-    const unsigned long long below = (1ull << lane) - 1;
-    if (bs) {
-      uint32_t base = 0;
-      if (lane == 0) base = atomicAdd(ndense, (uint32_t)__popcll(bs));
-      base = __shfl(base, 0, 64);
-      if (sml) dense[base + __popcll(bs & below)] = c;
-    }
-    if (bb) {
-      uint32_t base = 0;
-      if (lane == 0) base = atomicAdd(nbig, (uint32_t)__popcll(bb));
-      base = __shfl(base, 0, 64);
-      if (big) dbig[base + __popcll(bb & below)] = c;
-    }
+  const uint64_t t0 = (uint64_t)blockIdx.x * kCellTile;
+  if (t0 >= U) return;
+  if (threadIdx.x < 2) cnt[threadIdx.x] = 0;
+  __syncthreads();
+  for (uint32_t q = threadIdx.x; q < kCellTile && t0 + q < U; q += 256) {
+    const uint32_t c = (uint32_t)t0 + q;
+    const uint32_t s = cstart[c], e = (c + 1 < U) ? cstart[c + 1] : N;
+    if (c + 1 == U) cstart[U] = N;
+    klo[c] = sklo[s], khi[c] = skhi[s];
+    if (e - s < T) continue;
+    // dense: below kBigCell always, from it only with sub-cells
+    if (e - s < kBigCell) lst[atomicAdd(&cnt[0], 1u)] = (uint16_t)q;
+    else if (vols[vol_of(vbeg, nvol, s)].m[0] > 0)
+      lst[kCellTile - 1 - atomicAdd(&cnt[1], 1u)] = (uint16_t)q;
   }
+  __syncthreads();
+  if (threadIdx.x < 2 && cnt[threadIdx.x])
+    base[threadIdx.x] = atomicAdd(threadIdx.x ? nbig : ndense, cnt[threadIdx.x]);
+  __syncthreads();
+  for (uint32_t k = threadIdx.x; k < cnt[0]; k += 256) dense[base[0] + k] = (uint32_t)t0 + lst[k];
+  for (uint32_t k = threadIdx.x; k < cnt[1]; k += 256)
+    dbig[base[1] + k] = (uint32_t)t0 + lst[kCellTile - 1 - k];
 }
 
 __global__ __launch_bounds__(256) void k_init_uf(uint32_t N, uint32_t *__restrict__ par,
-                                                 uint32_t *__restrict__ run_end,
-                                                 uint32_t *__restrict__ gsize) {
+                                                 uint32_t *__restrict__ run_end) {
   for (uint32_t x = blockIdx.x * blockDim.x + threadIdx.x; x < N;
        x += gridDim.x * blockDim.x) {
     par[x] = x;
     run_end[x] = x + 1;
-    gsize[x] = 0;
   }
 }
 
@@ -1209,6 +1163,81 @@ __global__ __launch_bounds__(NT) void k_subsort(const uint32_t *__restrict__ den
 // ---------------------------------------------------------------------------
 // 5: sparse cells -- one thread per particle.
 // ---------------------------------------------------------------------------
+// A particle against the particles j .. je - 1, each joined where it links.  rx:
+// the particle's root, refreshed by every join.
+__device__ __forceinline__ void scan_range(const float4 px, const Rule &R, uint32_t j, uint32_t je,
+                                           const float4 *__restrict__ pos4,
+                                           uint32_t *__restrict__ par, uint32_t &rx,
+                                           uint32_t &tests, uint32_t &rechecks) {
+  for (; j + 4 <= je; j += 4) {
+    float4 q[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) q[k] = ld4(pos4 + j + k);
+    uint32_t hit = 0;
+#pragma unroll
+    for (int k = 0; k < 4; k++) hit |= pair_linked(px, q[k], R, rechecks) ? (1u << k) : 0u;
+    tests += 4;
+    while (hit) {
+      const int k = __builtin_ctz(hit);
+      hit &= hit - 1;
+      rx = uf_join(par, rx, j + k);
+    }
+  }
+  for (; j < je; j++) {
+    tests++;
+    if (pair_linked(px, pos4[j], R, rechecks)) rx = uf_join(par, rx, j);
+  }
+}
+
+// A particle against the particle ranges r0[k] .. r1[k) of its forward
+// neighbours where dense cells are scanned run by run (sub-sorted cells) or
+// particle by particle.
+__device__ __forceinline__ void scan_rows(const float4 px, const CellPos &cp, const VolDev &V,
+                                          const Rule &R, const uint32_t (&r0)[5],
+                                          const uint32_t (&r1)[5], int nr, uint32_t T,
+                                          const float4 *__restrict__ pos4,
+                                          const uint32_t *__restrict__ run_end,
+                                          const unsigned long long *__restrict__ fine,
+                                          uint32_t *__restrict__ par, uint32_t &rx,
+                                          uint32_t &tests, uint32_t &rechecks) {
+  const bool subcells = V.m[0] > 0;
+  for (int r = 0; r < nr; r++) {
+    uint32_t j = r0[r];
+    const uint32_t je = r1[r];
+    if (!subcells || je - j < T) {
+      // fewer than T particles: no dense cell here, every particle is a run
+      scan_range(px, R, j, je, pos4, par, rx, tests, rechecks);
+      continue;
+    }
+    while (j < je) {
+      const uint32_t re = run_end[j];
+      if (re == j + 1) {
+        tests++;
+        if (pair_linked(px, pos4[j], R, rechecks)) rx = uf_join(par, rx, j);
+        j++;
+        continue;
+      }
+      // a clique run of a dense cell: skip it when out of reach or joined
+      const unsigned long long fj = fine[j];
+      const int gx = max(abs(fine_x(fj) - cp.fx) - 1, 0);
+      const int gy = max(abs(fine_y(fj) - cp.fy) - 1, 0);
+      const int gz = max(abs(fine_z(fj) - cp.fz) - 1, 0);
+      const double g2 = (double)(gx * gx) * V.s2[0] + (double)(gy * gy) * V.s2[1] +
+                        (double)(gz * gz) * V.s2[2];
+      if (!(g2 > R.prune2) && uf_find(par, rx) != uf_find(par, j)) {
+        for (uint32_t k = j; k < re; k++) {
+          tests++;
+          if (pair_linked(px, pos4[k], R, rechecks)) {
+            rx = uf_join(par, rx, k);
+            break;
+          }
+        }
+      }
+      j = re;
+    }
+  }
+}
+
 // FAST: every volume of the call has a constant l, a dense grid and
 // sub-cells, so only the first branch below is compiled (it then fits 8
 // waves per SIMD without spilling); otherwise both branches.  Both run at 8
@@ -1231,7 +1260,7 @@ __global__ __launch_bounds__(256, 8) void k_link_sparse(uint32_t N, const float4
     const float4 px = pos4[x];
     const VolDev &V = vols[vol_of_run(vbeg, nvol, x, N, hint)];
     const CellPos cp = cell_pos(V, px.x, px.y, px.z);
-    const uint32_t c = G.sparse ? G.cell_of[x] : cell_id(V, cp.ix, cp.iy, cp.iz);
+    const uint32_t c = cell_id(V, cp.ix, cp.iy, cp.iz);
     const uint32_t s = G.start[c], e = G.start[c + 1];
     // dense cells are linked by k_link_small (below kBigCell particles) and
     // k_link_dense (from it, with sub-cells)
@@ -1240,7 +1269,7 @@ __global__ __launch_bounds__(256, 8) void k_link_sparse(uint32_t N, const float4
     uint32_t rx = x;  // x's root, refreshed by every join
     const int nx = V.nx, ny = V.ny, nz = V.nz;
     const int xl = (cp.ix > 0) ? 1 : 0, xr = (cp.ix + 1 < nx) ? 1 : 0;
-    if (FAST || (!G.sparse && V.vntab == 0 && V.m[0] > 0)) {
+    if (FAST || (V.vntab == 0 && V.m[0] > 0)) {
       // Constant l on a dense grid: k_link_dense links every pair that has a
       // particle in a dense cell (its forward cells, and its backward cells
       // that are sparse).  Here: the sparse cells among the own cell (after
@@ -1308,15 +1337,7 @@ __global__ __launch_bounds__(256, 8) void k_link_sparse(uint32_t N, const float4
     uint32_t r0[5], r1[5];
     int nr = 0;
     r0[nr] = x + 1;
-    if (!G.sparse) {
-      r1[nr] = G.start[c + 1 + xr];
-    } else {
-      r1[nr] = e;
-      if (xr) {
-        const uint32_t c1 = hlookup(G, comp_key(G, V, cp.ix + 1, cp.iy, cp.iz));
-        if (c1 != kNone) r1[nr] = G.start[c1 + 1];
-      }
-    }
+    r1[nr] = G.start[c + 1 + xr];
     nr++;
     if (cp.iy + 1 < ny) {
       row_range(G, V, cp.ix - xl, cp.ix + xr, cp.iy + 1, cp.iz, r0[nr], r1[nr]);
@@ -1329,57 +1350,230 @@ __global__ __launch_bounds__(256, 8) void k_link_sparse(uint32_t N, const float4
         nr++;
       }
     }
-    const bool subcells = V.m[0] > 0;
-    for (int r = 0; r < nr; r++) {
-      uint32_t j = r0[r];
-      const uint32_t je = r1[r];
-      if (!subcells || je - j < T) {
-        // fewer than T particles: no dense cell here, every particle is a run
-        for (; j + 4 <= je; j += 4) {
-          float4 q[4];
+    scan_rows(px, cp, V, R, r0, r1, nr, T, pos4, run_end, fine, par, rx, tests, rechecks);
+  }
+  add_counters(ctr, kCtrTestsSparse, tests, rechecks);
+}
+
+// The same over occupied cells (sparse addressing).  Particles, cells and keys
+// are in one order, and a neighbour row's keys are the cell's own plus a
+// constant: the rows of consecutive particles are consecutive stretches of
+// the key list.  A wave takes kRowRun consecutive particles, keeps a place in
+// the list for each of the four rows above its own, reads the keys there 128
+// at a time into LDS, and each lane finds its first key by binary search.
+// Thirteen probes of a hash table a particle, each a random line of gigabytes,
+// took 4.09 ms for a lightcone of 1.6e7 particles in 16 shells.  A dense cell of
+// a row is linked by the whole wave for one particle after the other, a run a
+// lane and runs above 8 particles 64 at a time: a lane that went through the
+// hundreds of runs of a big cell alone kept 63 waiting (2.98 ms, now 2.16).
+// What bounds it now: the chain of dependent loads of such cells and of the
+// scans (search 13, scans 25 thousand cycles a wave's 64 particles).
+constexpr uint32_t kRowRun = 512;  // particles of a wave
+constexpr uint32_t kRowWin = 128;   // keys of a window
+
+// A cell at or before the first one with key >= t in [lo, U) (t uniform), at
+// most 64 before it: 64 samples a step.
+__device__ __forceinline__ uint32_t wave_lower(const Grid &G, uint32_t lo, uint32_t U,
+                                               unsigned long long t) {
+  const uint32_t lane = threadIdx.x & 63;
+  uint32_t hi = U;
+  while (hi - lo > 64) {
+    const uint32_t step = (hi - lo + 63) / 64;
+    const uint32_t at = lo + (lane + 1) * step - 1;
+    const bool below = at < hi && cell_key(G, at) < t;
+    lo = min(hi, lo + (uint32_t)__popcll(__ballot(below)) * step);
+    hi = min(hi, lo + step);
+  }
+  return lo;
+}
+
+__global__ __launch_bounds__(256, 6) void k_link_rows(uint32_t N, const float4 *__restrict__ pos4,
+                                                   const Grid G,
+                                                   const uint32_t *__restrict__ run_end,
+                                                   const unsigned long long *__restrict__ fine,
+                                                   const uint32_t *__restrict__ rtoff,
+                                                   const uint32_t *__restrict__ rtab,
+                                                   uint32_t *__restrict__ par,
+                                                   const VolDev *__restrict__ vols,
+                                                   const uint32_t *__restrict__ vbeg, int nvol,
+                                                   uint32_t T,
+                                                   unsigned long long *__restrict__ ctr) {
+  __shared__ unsigned long long wins[4][kRowWin];
+  __shared__ uint32_t rowc[4][5][64];  // a lane's first cell in each row
+  const uint32_t lane = threadIdx.x & 63;
+  const uint32_t wv = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  unsigned long long *const win = wins[wv];
+  uint32_t(*const row)[64] = rowc[wv];
+  const uint32_t U = *G.ncell;
+  const uint64_t x0 = ((uint64_t)blockIdx.x * 4 + wv) * kRowRun;
+  uint32_t tests = 0, rechecks = 0;
+  uint32_t place[4] = {kNone, kNone, kNone, kNone};
+  int hint = 0, last_v = -1;
+  for (uint32_t q = 0; q < kRowRun && x0 + q < N; q += 64) {
+    const uint32_t x = (uint32_t)(x0 + q) + lane;
+    const bool valid = x < N;
+    const uint32_t xc = min(x, N - 1);
+    const float4 px = ld4(pos4 + xc);
+    const int v = vol_of_run(vbeg, nvol, xc, N, hint);
+    const VolDev &V = vols[v];
+    const CellPos cp = cell_pos(V, px.x, px.y, px.z);
+    const uint32_t c = G.cell_of[xc];
+    const uint32_t s = G.start[c], e = G.start[c + 1];
+    // dense cells are linked by k_link_small and k_link_dense
+    const bool active = valid && !(e - s >= T && (e - s < kBigCell || V.m[0] > 0));
+    if (!__ballot(active)) continue;
+    // a wave in two volumes looks each row up on its own
+    const int v0 = __builtin_amdgcn_readfirstlane(v);
+    const bool one = __ballot(v != v0) == 0;
+    if (!one || v0 != last_v) place[0] = place[1] = place[2] = place[3] = kNone;
+    last_v = one ? v0 : -1;
+    const int nx = V.nx, ny = V.ny, nz = V.nz;
+    const unsigned long long key = cell_key(G, c);
+    uint32_t ncell[5];  // occupied cells of each row (own row: behind the own cell)
+    row[0][lane] = c + 1;
+    ncell[0] = active && cp.ix + 1 < nx && c + 1 < U && cell_key(G, c + 1) == key + 1 ? 1u : 0u;
 #pragma unroll
-          for (int k = 0; k < 4; k++) q[k] = ld4(pos4 + j + k);
-          uint32_t hit = 0;
+    for (int r = 1; r < 5; r++) {
+      ncell[r] = 0;
+      const int dy = r == 1 ? 1 : r - 3, dz = r == 1 ? 0 : 1;
+      const bool want = active && cp.iy + dy >= 0 && cp.iy + dy < ny && cp.iz + dz < nz;
+      const long long d = ((long long)dz * ny + dy) * nx;
+      // the row's keys a .. b (ascending over the lanes of one volume)
+      const unsigned long long a = key + (unsigned long long)(d - (cp.ix > 0 ? 1 : 0));
+      const unsigned long long b = key + (unsigned long long)(d + (cp.ix + 1 < nx ? 1 : 0));
+      unsigned long long need = __ballot(want);
+      if (!need) continue;
+      if (one) {
+        auto first = [&]() -> unsigned long long {
+          const int l = __builtin_ctzll(need);
+          return (unsigned long long)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)a, l) |
+                 ((unsigned long long)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(a >> 32), l) << 32);
+        };
+        uint32_t w = place[r - 1] == kNone ? wave_lower(G, 0, U, first()) : place[r - 1];
+        for (;;) {
+          wave_sync();
+          win[lane] = w + lane < U ? cell_key(G, w + lane) : ~0ull;
+          win[lane + 64] = w + 64 + lane < U ? cell_key(G, w + 64 + lane) : ~0ull;
+          wave_sync();
+          // resolved when the first key >= a and the two behind it are here
+          const bool here = ((need >> lane) & 1ull) && a <= win[kRowWin - 4];
+          if (here) {
+            uint32_t lo = 0;
 #pragma unroll
-          for (int k = 0; k < 4; k++) hit |= pair_linked(px, q[k], R, rechecks) ? (1u << k) : 0u;
-          tests += 4;
-          while (hit) {
-            const int k = __builtin_ctz(hit);
-            hit &= hit - 1;
-            rx = uf_join(par, rx, j + k);
+            for (uint32_t st = kRowWin / 2; st > 0; st >>= 1)
+              if (win[lo + st - 1] < a) lo += st;
+            uint32_t n = 0;
+#pragma unroll
+            for (uint32_t k = 0; k < 3; k++) n += win[lo + k] <= b ? 1u : 0u;
+            ncell[r] = n;
+            row[r][lane] = w + lo;
           }
+          const unsigned long long done = __ballot(here);
+          need &= ~done;
+          if (!need) break;
+          // the next window behind this one, or where the first lane left lies
+          w = done ? w + kRowWin - 3 : wave_lower(G, w + kRowWin - 3, U, first());
         }
-        for (; j < je; j++) {
-          tests++;
-          if (pair_linked(px, pos4[j], R, rechecks)) rx = uf_join(par, rx, j);
-        }
-        continue;
+        place[r - 1] = w;
+      } else if (want) {
+        const uint32_t lo = cell_lower(G, U, a);
+        uint32_t n = 0;
+        while (n < 3 && lo + n < U && cell_key(G, lo + n) <= b) n++;
+        ncell[r] = n;
+        row[r][lane] = lo;
       }
-      while (j < je) {
-        const uint32_t re = run_end[j];
-        if (re == j + 1) {
-          tests++;
-          if (pair_linked(px, pos4[j], R, rechecks)) rx = uf_join(par, rx, j);
-          j++;
+    }
+    Rule R;
+    uint32_t rx = x, dcells = 0;  // bit 3 r + k: cell k of row r is dense
+    if (active) {
+      R = make_rule(V, cp.ix, cp.iy, cp.iz);
+      const bool subcells = V.m[0] > 0;
+      scan_range(px, R, x + 1, e, pos4, par, rx, tests, rechecks);
+#pragma unroll
+      for (int r = 0; r < 5; r++) {
+        if (!ncell[r]) continue;
+        const uint32_t cf = row[r][lane];
+        uint32_t j = G.start[cf], je = G.start[cf + ncell[r]];
+        if (subcells && je - j >= T) {
+          // sub-sorted cells among them are left to the wave where the
+          // particle's sub-cell is within reach of the cell
+          const int dy = r == 0 ? 0 : r == 1 ? 1 : r - 3, dz = r < 2 ? 0 : 1;
+          const unsigned long long mid = key + (unsigned long long)(((long long)dz * ny + dy) * nx);
+          const int gy = dy > 0 ? (cp.iy + 1) * V.m[1] - cp.fy - 1 : dy < 0 ? cp.fy - cp.iy * V.m[1] : 0;
+          const int gz = dz > 0 ? (cp.iz + 1) * V.m[2] - cp.fz - 1 : 0;
+          for (uint32_t k = 0; k < ncell[r]; k++) {
+            const uint32_t ke = G.start[cf + k + 1];
+            if (ke - j >= T) {
+              const int dx = (int)(long long)(cell_key(G, cf + k) - mid);
+              const int gx = dx > 0 ? (cp.ix + 1) * V.m[0] - cp.fx - 1 : dx < 0 ? cp.fx - cp.ix * V.m[0] : 0;
+              const double g2 = (double)(gx * gx) * V.s2[0] + (double)(gy * gy) * V.s2[1] +
+                                (double)(gz * gz) * V.s2[2];
+              if (!(g2 > R.prune2)) dcells |= 1u << (3 * r + k);
+            } else {
+              scan_range(px, R, j, ke, pos4, par, rx, tests, rechecks);
+            }
+            j = ke;
+          }
           continue;
         }
-        // a clique run of a dense cell: skip it when out of reach or joined
-        const unsigned long long fj = fine[j];
-        const int gx = max(abs(fine_x(fj) - cp.fx) - 1, 0);
-        const int gy = max(abs(fine_y(fj) - cp.fy) - 1, 0);
-        const int gz = max(abs(fine_z(fj) - cp.fz) - 1, 0);
-        const double g2 = (double)(gx * gx) * V.s2[0] + (double)(gy * gy) * V.s2[1] +
-                          (double)(gz * gz) * V.s2[2];
-        if (!(g2 > R.prune2) && uf_find(par, rx) != uf_find(par, j)) {
-          for (uint32_t k = j; k < re; k++) {
+        scan_range(px, R, j, je, pos4, par, rx, tests, rechecks);
+      }
+    }
+    wave_sync();
+    while (const unsigned long long pend = __ballot(dcells != 0)) {
+      // the lowest lane's next dense cell
+      const int l = __builtin_ctzll(pend);
+      const uint32_t dl = (uint32_t)__builtin_amdgcn_readlane((int)dcells, l);
+      const uint32_t t = (uint32_t)__builtin_ctz(dl);
+      if ((int)lane == l) dcells &= dcells - 1;
+      auto lf = [&](float f) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f), l)); };
+      auto li = [&](int i) { return __builtin_amdgcn_readlane(i, l); };
+      auto ld = [&](double q) { return __hiloint2double(li(__double2hiint(q)), li(__double2loint(q))); };
+      const VolDev &W = vols[li(v)];
+      const float4 q = make_float4(lf(px.x), lf(px.y), lf(px.z), 0.f);
+      const Rule Q = {ld(R.linksq), ld(R.prune2), lf(R.lo), lf(R.hi)};
+      const int qx = li(cp.fx), qy = li(cp.fy), qz = li(cp.fz);
+      const uint32_t xl = (uint32_t)li((int)x), sB = G.start[row[t / 3][l] + t % 3];
+      const uint32_t runs = rtoff[sB];
+      for (uint32_t i0 = 0; i0 < runs; i0 += 64) {
+        uint32_t j = 0, je = 0;
+        if (i0 + lane < runs) {
+          j = rtab[sB + i0 + lane];
+          const unsigned long long fj = fine[j];
+          const int gx = max(abs(fine_x(fj) - qx) - 1, 0);
+          const int gy = max(abs(fine_y(fj) - qy) - 1, 0);
+          const int gz = max(abs(fine_z(fj) - qz) - 1, 0);
+          const double g2 = (double)(gx * gx) * W.s2[0] + (double)(gy * gy) * W.s2[1] +
+                            (double)(gz * gz) * W.s2[2];
+          je = g2 > Q.prune2 ? j : run_end[j];
+        }
+        // short runs a lane each, longer ones 64 particles at a time
+        unsigned long long big = __ballot(je - j > 8);
+        if (je - j <= 8)
+          for (; j < je; j++) {
             tests++;
-            if (pair_linked(px, pos4[k], R, rechecks)) {
-              rx = uf_join(par, rx, k);
+            if (pair_linked(q, pos4[j], Q, rechecks)) {
+              uf_union(par, xl, j);
               break;
             }
           }
+        while (big) {
+          const int b = __builtin_ctzll(big);
+          big &= big - 1;
+          const uint32_t bj = (uint32_t)__builtin_amdgcn_readlane((int)j, b);
+          const uint32_t be = (uint32_t)__builtin_amdgcn_readlane((int)je, b);
+          for (uint32_t k0 = bj; k0 < be; k0 += 64) {
+            bool hit = false;
+            if (k0 + lane < be) {
+              tests++;
+              hit = pair_linked(q, pos4[k0 + lane], Q, rechecks);
+            }
+            const unsigned long long h = __ballot(hit);
+            if (!h) continue;
+            if (lane == 0) uf_union(par, xl, k0 + (uint32_t)__builtin_ctzll(h));
+            break;
+          }
         }
-        j = re;
       }
     }
   }
@@ -2552,14 +2746,16 @@ __global__ __launch_bounds__(256) void k_flatten(uint32_t N, uint32_t *__restric
   if ((threadIdx.x & 63) == 0 && t) ctr_add(ctr, kCtrGroups, t);
 }
 
-// The accumulators of k_flatten (minimum index, with idroot minimum ID) and
-// the label bitmap.
+// The accumulators of k_flatten (minimum index, with idroot minimum ID; sizes
+// where the bucket sort has not cleared them) and the label bitmap.
 __global__ __launch_bounds__(256) void k_init_groups(uint32_t N, uint32_t *__restrict__ minorig,
                                                      unsigned long long *__restrict__ idroot,
+                                                     uint32_t *__restrict__ gsize,
                                                      uint32_t nw, uint32_t *__restrict__ bits) {
   for (uint32_t x = blockIdx.x * blockDim.x + threadIdx.x; x < N; x += gridDim.x * blockDim.x) {
     minorig[x] = ~0u;
     if (idroot) idroot[x] = ~0ull;
+    if (gsize) gsize[x] = 0;
     if (x < nw) bits[x] = 0;
   }
 }
@@ -3990,7 +4186,6 @@ static int enqueue_run(Run &r, hipStream_t st) {
   const uint8_t *dbase = r.dbase;
   uint32_t *small = B.small;
   unsigned long long *ctr = reinterpret_cast<unsigned long long *>(small + kSmCtr);
-  uint32_t *hsm = static_cast<uint32_t *>(pp.down.ptr);
   const bool timing = r.timing;
   if (timing && !pp.events) {
     for (auto &e : pp.ev) FOF_HIP(hipEventCreate(&e));
@@ -4060,9 +4255,10 @@ static int enqueue_run(Run &r, hipStream_t st) {
 
   Grid G;
   G.start = start;
-  G.htab = nullptr;
   G.cell_of = label;  // sparse: the label buffer is free until k_label
-  G.hmask = 0;
+  G.klo = B.cnt;      // sparse: the flags' buffer and the sizes' (cleared after linking)
+  G.khi = gsize;
+  G.ncell = small + kSmU;
   G.sparse = pl.sparse ? 1 : 0;
   G.volshift = pl.volshift;
   if (!pl.sparse) {
@@ -4127,7 +4323,7 @@ static int enqueue_run(Run &r, hipStream_t st) {
     FOF_HIP(hipGetLastError());
     if ((rc = te(2))) return rc;
   } else {
-    // 1-3: composite keys, LSD sort by (volume, cell), occupied cells, hash
+    // 1-3: composite keys, LSD sort by (volume, cell), occupied cells
     uint32_t *cnt = B.cnt;
     if ((rc = tb(0))) return rc;
     k_keys_sparse<<<gN, 256, 0, st>>>(dbase, stride, offpos, NN, dV, dVB, (int)nvol, G, sk0, key,
@@ -4151,25 +4347,14 @@ static int enqueue_run(Run &r, hipStream_t st) {
     if ((rc = te(2))) return rc;
     k_cell_flags<<<gN, 256, 0, st>>>(NN, par, runend, cnt);
     FOF_HIP(hipGetLastError());
-    if ((rc = compact_flagged(cnt, N, nullptr, kFlag, nullptr, start, small + kSmU, B.tmp, st)))
+    if ((rc = compact_flagged(cnt, N, nullptr, kFlag, nullptr, start, label, small + kSmU, B.tmp, st)))
       return rc;
-    // the hash table is sized from the occupied-cell count
-    FOF_HIP(hipMemcpyAsync(hsm, small, 64, hipMemcpyDeviceToHost, st));
-    FOF_HIP(hipStreamSynchronize(st));
-    const uint32_t U = hsm[kSmU];
-    uint64_t hsz = 1024;
-    while (hsz < 2ull * U) hsz <<= 1;
-    if ((rc = ensure(pp.hash, hsz * sizeof(HEntry) + 256))) return rc;
-    HEntry *htab = static_cast<HEntry *>(pp.hash.ptr);
-    if ((rc = fill_u32(reinterpret_cast<uint32_t *>(htab), hsz * 4, ~0u, st))) return rc;
-    G.htab = htab;
-    G.hmask = hsz - 1;
-    k_cells_finish<<<grid_for(U), 256, 0, st>>>(small + kSmU, NN, start, par, runend, G, htab,
-                                                label, dV, dVB, (int)nvol, T, dense,
-                                                small + kSmNDense, dbig, small + kSmNBig);
+    k_cells_finish<<<(uint32_t)((N + kCellTile - 1) / kCellTile), 256, 0, st>>>(small + kSmU, NN, start, par, runend, cnt, gsize, dV, dVB,
+                                       (int)nvol, T, dense, small + kSmNDense, dbig,
+                                       small + kSmNBig);
     FOF_HIP(hipGetLastError());
     if ((rc = tb(3))) return rc;
-    k_init_uf<<<gN, 256, 0, st>>>(NN, par, runend, gsize);
+    k_init_uf<<<gN, 256, 0, st>>>(NN, par, runend);
     FOF_HIP(hipGetLastError());
     if ((rc = te(3))) return rc;
   }
@@ -4243,6 +4428,9 @@ static int enqueue_run(Run &r, hipStream_t st) {
   if ((rc = tb(5))) return rc;
   if (fast)
     k_link_sparse<true><<<gN, 256, 0, st>>>(NN, pos4, G, runend, fine, par, dV, dVB, (int)nvol, T, ctr);
+  else if (pl.sparse)
+    k_link_rows<<<(uint32_t)((N + 4 * kRowRun - 1) / (4 * kRowRun)), 256, 0, st>>>(
+        NN, pos4, G, runend, fine, rtoff, rtab, par, dV, dVB, (int)nvol, T, ctr);
   else
     k_link_sparse<false><<<gN, 256, 0, st>>>(NN, pos4, G, runend, fine, par, dV, dVB, (int)nvol, T, ctr);
   FOF_HIP(hipGetLastError());
@@ -4258,7 +4446,8 @@ static int enqueue_run(Run &r, hipStream_t st) {
   if ((rc = tb(7))) return rc;
   const uint64_t nw = (N + 31) / 32;
   uint32_t *gbits = key;  // the label bitmap (the head sizes follow in k_label)
-  k_init_groups<<<gN, 256, 0, st>>>(NN, minorig, idroot, (uint32_t)nw, gbits);
+  k_init_groups<<<gN, 256, 0, st>>>(NN, minorig, idroot, pl.sparse ? gsize : nullptr, (uint32_t)nw,
+                                    gbits);
   FOF_HIP(hipGetLastError());
   k_flatten<<<gN, 256, 0, st>>>(NN, par, pos4, minorig, gsize, ctr, dbase, stride, offid, idroot);
   FOF_HIP(hipGetLastError());
@@ -4906,7 +5095,6 @@ static void free_pipe(Pipe &pp) {
   release_host(pp.up);
   release_host(pp.down);
   release(pp.arena);
-  release(pp.hash);
   if (pp.events)
     for (auto &e : pp.ev) (void)hipEventDestroy(e);
   pp.events = false;

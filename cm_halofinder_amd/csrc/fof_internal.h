@@ -82,11 +82,12 @@ int scatter_u32(const uint32_t *idx, const uint32_t *val, uint32_t *idx2, uint32
                 void *tmp, hipStream_t st);
 
 // Stable compaction: for every i in [0,n) with (src[i] & flag) != 0, in
-// ascending i, append key = src[i] & ~flag and value = i.  The count goes to
+// ascending i, append key = src[i] & ~flag and value = i.  orank[i] (may be
+// null): the list place of the last entry at or before i.  The count goes to
 // *dcount (device; must not alias dn).  tmp: compact_tmp_bytes(n).
 size_t compact_tmp_bytes(uint64_t n);
 int compact_flagged(const uint32_t *src, uint64_t n, const uint32_t *dn, uint32_t flag,
-                    uint32_t *out_key, uint32_t *out_val, uint32_t *dcount, void *tmp,
+                    uint32_t *out_key, uint32_t *out_val, uint32_t *orank, uint32_t *dcount, void *tmp,
                     hipStream_t st);
 
 // p[0..n) = v (a kernel, not hipMemsetAsync: captured sequences hold kernel
@@ -99,7 +100,6 @@ int fill_u32(uint32_t *p, uint64_t n, uint32_t v, hipStream_t st);
 struct Pipe {
   hipStream_t stream = nullptr;
   Scratch arena;  // every buffer of a call
-  Scratch hash;   // occupied-cell hash table (sized once the cell count is known)
   // page-locked: what a call uploads ahead of its kernels and reads back
   Scratch up, down;
   hipEvent_t ev[2 * FOF_NPHASE] = {};

@@ -234,6 +234,7 @@ __global__ __launch_bounds__(kBlock) void k_compact_emit(const uint32_t *__restr
                                                          const uint32_t *__restrict__ boff,
                                                          uint32_t *__restrict__ okey,
                                                          uint32_t *__restrict__ oval,
+                                                         uint32_t *__restrict__ orank,
                                                          uint32_t *__restrict__ dcount) {
   __shared__ uint32_t ws[kBlock / 64];
   const uint64_t n = dev_count(dn, ncap);
@@ -253,6 +254,7 @@ __global__ __launch_bounds__(kBlock) void k_compact_emit(const uint32_t *__restr
       oval[pre] = (uint32_t)(base + i);
       pre++;
     }
+    if (orank && base + i < n) orank[base + i] = pre - 1;
   }
   if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) *dcount = boff[gridDim.x];
 }
@@ -456,7 +458,7 @@ int scan_u32(const uint32_t *in, uint32_t *out, uint64_t n, void *tmp, hipStream
 size_t compact_tmp_bytes(uint64_t n) { return scan_levels_bytes(n) + 256; }
 
 int compact_flagged(const uint32_t *src, uint64_t n, const uint32_t *dn, uint32_t flag,
-                    uint32_t *okey, uint32_t *oval, uint32_t *dcount, void *tmp,
+                    uint32_t *okey, uint32_t *oval, uint32_t *orank, uint32_t *dcount, void *tmp,
                     hipStream_t st) {
   if (n == 0) return fill_u32(dcount, 1, 0u, st);
   uint32_t *bs = static_cast<uint32_t *>(tmp);
@@ -465,7 +467,7 @@ int compact_flagged(const uint32_t *src, uint64_t n, const uint32_t *dn, uint32_
   FOF_HIP(hipGetLastError());
   int rc = scan_bsums(bs, nb, st);
   if (rc) return rc;
-  k_compact_emit<<<(uint32_t)nb, kBlock, 0, st>>>(src, n, dn, flag, bs, okey, oval, dcount);
+  k_compact_emit<<<(uint32_t)nb, kBlock, 0, st>>>(src, n, dn, flag, bs, okey, oval, orank, dcount);
   FOF_HIP(hipGetLastError());
   return 0;
 }

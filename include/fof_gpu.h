@@ -103,8 +103,8 @@ typedef struct fof_domain_v1 {
                                    identical arguments (device-resident input
                                    and outputs, constant linking length, dense
                                    cell addressing; other calls run eagerly)  */
-#define FOF_OPT_SPARSE 0x20u    /* address only occupied cells (sorted keys +
-                                   hash table); chosen automatically when a
+#define FOF_OPT_SPARSE 0x20u    /* address only occupied cells (a list in key
+                                   order); chosen automatically when a
                                    dense cell table would be much larger than
                                    the particle count or reach 2^31 cells     */
 #define FOF_OPT_AUTOTUNE 0x40u  /* pick the dense-cell threshold and the number

@@ -58,3 +58,25 @@ def test_dense_sort_matches_occupied_cells(ctx, grid, n):
     assert a[3] == b[3]
     for x, y in zip(a[:3], b[:3]):
         assert torch.equal(x, y)
+
+
+@pytest.mark.parametrize("full,thin", [(1, 1), (1, 40), (1, 400), (3, 2000), (130, 131)])
+def test_occupied_rows_of_uneven_density(ctx, full, thin):
+    # rows of 4000 cells holding a particle in every `full`-th or `thin`-th
+    # cell, alternating: a wave's stretch of one row meets fewer or many times
+    # more occupied cells in the next, against the oracle
+    from test_gpu_parity import check_against_oracle
+
+    rng = np.random.default_rng(full * 7 + thin)
+    nx, parts = 4000, []
+    for z in range(3):
+        for y in range(7):
+            x = np.arange(0, nx, full if (y + z) % 2 else thin)
+            parts.append(np.stack([x, np.full(len(x), y), np.full(len(x), z)], 1) + rng.random((len(x), 3)))
+    blob = np.array([1999.5, 3.5, 1.5]) + rng.normal(0, 0.3, (600, 3))  # a dense cell among them
+    pos = np.concatenate(parts + [blob.clip([1998, 2, 0.01], [2002, 5, 2.99])])
+    P = np.zeros(len(pos), L.PART_DTYPE)
+    P["Pos"] = pos[rng.permutation(len(pos))].astype(np.float32).clip([0, 0, 0], [3999.9, 6.999, 2.999])
+    P["ID"] = np.arange(len(pos))
+    dom = L.domain([0] * 3, [nx, 7, 3], [0] * 3, [nx, 7, 3], [1] * 3, 0.8, 2)
+    check_against_oracle(ctx, P, dom, flags=L.OPT_SPARSE)
