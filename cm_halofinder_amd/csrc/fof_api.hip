@@ -2,8 +2,8 @@
 // Argument checks run on the host before any device work, so a bad call
 // fails the same way with or without a GPU.  The domain check (every
 // particle inside [rmin_buff, rmax_buff]) runs on the host for host-resident
-// particles, before any device work, and inside the first kernel for
-// device-resident ones (reported when the call ends).
+// particles, with their upload and ahead of every kernel, and inside the first
+// kernel for device-resident ones (reported when the call ends).
 #include <stdio.h>
 #include <string.h>
 
@@ -14,6 +14,8 @@
 #include <vector>
 
 #include "fof_internal.h"
+
+using fof::HostCheck;
 
 static thread_local char g_last_error[256];
 
@@ -56,47 +58,60 @@ int check_opts(const fof_opts_v1 *o) {
   return 0;
 }
 
-// Domain check of host-resident particles, before any device work: every
-// position inside its volume's [rmin_buff, rmax_buff] (the bounds of
-// src_v2/read_data.c:810-812; NaN fails the comparisons).  Split over up to
-// 16 host threads.
-int check_domain_host(const fof_particles_v1 *P, const fof_volume_v1 *vols, uint32_t nvol) {
-  if (P->location != FOF_MEM_HOST || P->n == 0) return 0;
-  const uint8_t *base = static_cast<const uint8_t *>(P->base);
-  const uint64_t N = P->n;
-  const unsigned nth =
-      (unsigned)std::max<uint64_t>(1, std::min<uint64_t>({16u, std::thread::hardware_concurrency(), N / 65536 + 1}));
-  std::vector<int> bad(nth, 0);
-  auto work = [&](unsigned t) {
-    const uint64_t a = N * t / nth, e = N * (t + 1) / nth;
-    uint32_t v = 0;
-    while (v + 1 < nvol && vols[v].offset + vols[v].n <= a) v++;
-    for (uint64_t p = a; p < e; p++) {
-      while (p >= vols[v].offset + vols[v].n) v++;
-      const fof_domain_v1 &D = vols[v].domain;
-      const float *q = reinterpret_cast<const float *>(base + p * P->stride + P->off_pos);
-      for (int d = 0; d < 3; d++) {
-        const double x = q[d];
-        if (!(x >= D.rmin_buff[d] && x <= D.rmax_buff[d])) {
-          bad[t] = 1;
-          return;
-        }
-      }
-    }
-  };
-  std::vector<std::thread> th;
-  for (unsigned t = 1; t < nth; t++) th.emplace_back(work, t);
-  work(0);
-  for (auto &x : th) x.join();
-  for (int x : bad)
-    if (x) return FOF_E_DOMAIN;
-  return 0;
-}
-
 std::mutex g_default_mu;
 fof_ctx *g_default[64];
 
 }  // namespace
+
+namespace fof {
+
+bool HostCheck::range(uint64_t a, uint64_t e) const {
+  if (a >= e) return true;
+  const uint8_t *base = static_cast<const uint8_t *>(P->base);
+  uint32_t v = (uint32_t)(std::upper_bound(vols, vols + nvol, a,
+                                           [](uint64_t p, const fof_volume_v1 &q) { return p < q.offset + q.n; }) -
+                          vols);
+  for (uint64_t p = a; p < e; p++) {
+    while (p >= vols[v].offset + vols[v].n) v++;
+    const fof_domain_v1 &D = vols[v].domain;
+    const float *q = reinterpret_cast<const float *>(base + p * P->stride + P->off_pos);
+    for (int d = 0; d < 3; d++) {
+      const double x = q[d];
+      if (!(x >= D.rmin_buff[d] && x <= D.rmax_buff[d])) return false;
+    }
+  }
+  return true;
+}
+
+int HostCheck::finish() {
+  if (state.load() == 0) {
+    const uint64_t N = P->location == FOF_MEM_HOST ? P->n : 0;
+    const unsigned nth = (unsigned)std::max<uint64_t>(
+        1, std::min<uint64_t>({16u, std::thread::hardware_concurrency(), N / 65536 + 1}));
+    std::atomic<bool> bad{false};
+    auto work = [&](unsigned t) {
+      if (!range(N * t / nth, N * (t + 1) / nth)) bad = true;
+    };
+    run_threads(nth, work);
+    state = bad ? 2 : 1;
+  }
+  return state.load() == 2 ? FOF_E_DOMAIN : 0;
+}
+
+void run_threads(unsigned n, const std::function<void(unsigned)> &work) {
+  std::vector<std::thread> th;
+  for (unsigned t = 1; t < n; t++) {
+    try {
+      th.emplace_back(work, t);
+    } catch (...) {  // no more threads: this one does the share
+      work(t);
+    }
+  }
+  work(0);
+  for (auto &x : th) x.join();
+}
+
+}  // namespace fof
 
 extern "C" {
 
@@ -181,9 +196,13 @@ int fof_link_gpu_ex(fof_ctx *ctx, const fof_particles_v1 *particles, const fof_v
   int rc = check_batch(particles, vols, nvol, opts);
   if (rc) return rc;
   if (out->minid && particles->off_id < 0) return FOF_E_ARG;
-  if ((rc = check_domain_host(particles, vols, nvol))) return rc;
-  if ((rc = resolve_ctx(&ctx))) return rc;
-  return fof_engine_run(ctx, particles, vols, nvol, opts, out);
+  HostCheck check{particles, vols, nvol};
+  if (!(rc = resolve_ctx(&ctx))) rc = fof_engine_run(ctx, particles, vols, nvol, opts, out, &check);
+  if (const int bad = check.finish()) {  // ahead of any other error
+    out->nhalos = 0;
+    return bad;
+  }
+  return rc;
 }
 
 static fof_outputs_v1 legacy_outputs(const fof_opts_v1 *opts, uint32_t *next_out,

@@ -5,6 +5,9 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <atomic>
+#include <functional>
+#include <thread>
 #include <utility>
 #include <vector>
 
@@ -109,6 +112,23 @@ struct Pipe {
   hipEvent_t side_fork = nullptr, side_join = nullptr;
 };
 
+// work(0) .. work(n - 1), one thread each (the caller's does the first).
+void run_threads(unsigned n, const std::function<void(unsigned)> &work);
+
+// Domain check of host-resident particles: every position inside its volume's
+// [rmin_buff, rmax_buff] (the bounds of src_v2/read_data.c:810-812; NaN fails
+// the comparisons).  A staged upload checks the records on their way (range)
+// and leaves the answer in `state`; finish() checks whatever has not been and
+// answers 0 or FOF_E_DOMAIN.
+struct HostCheck {
+  const fof_particles_v1 *P;
+  const fof_volume_v1 *vols;
+  uint32_t nvol;
+  std::atomic<int> state{0};  // 0: not checked, 1: inside, 2: a bad particle
+  bool range(uint64_t a, uint64_t e) const;
+  int finish();
+};
+
 constexpr int kMaxPipes = 8;  // concurrent pipelines of one call
 
 // Autotuning: a workload shape and the parameters chosen for it.
@@ -123,7 +143,13 @@ struct TuneVal {
   uint32_t T, pipes, gbig;  // dense threshold, pipelines, dense-kernel grid (0: default)
 };
 
+// Page-locked pieces through which pageable host memory is copied.
+constexpr size_t kPiece = 2u << 20;
+constexpr unsigned kCopyThreads = 8;  // each with two pieces
+
 struct EngineState {
+  Scratch pieces;
+  hipEvent_t piece_ev[2 * kCopyThreads] = {};
   Pipe main;                       // pipeline 0, on the context's stream
   std::vector<Pipe *> pipes;       // pipelines 1.. (entry 0 unused)
   hipEvent_t fork = nullptr, join[kMaxPipes] = {}, t0 = nullptr, t1 = nullptr;
@@ -142,7 +168,8 @@ struct fof_ctx {
 
 // Engine entry (fof_engine.hip); arguments checked by the caller.
 extern "C" int fof_engine_run(fof_ctx *ctx, const fof_particles_v1 *P, const fof_volume_v1 *vols,
-                              uint32_t nvol, const fof_opts_v1 *opts, fof_outputs_v1 *out);
+                              uint32_t nvol, const fof_opts_v1 *opts, fof_outputs_v1 *out,
+                              fof::HostCheck *check);
 extern "C" int fof_engine_plan(const fof_particles_v1 *P, const fof_volume_v1 *vols,
                                uint32_t nvol, const fof_opts_v1 *opts, fof_plan_v1 *out);
 extern "C" int fof_engine_run_noalloc(fof_ctx *ctx, const fof_particles_v1 *P,
