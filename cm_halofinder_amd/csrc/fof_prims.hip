@@ -520,19 +520,33 @@ int radix_sort_u32(uint32_t *k0, uint32_t *v0, uint32_t *k1, uint32_t *v1, uint6
 }
 
 // ---- scatter through one partition pass -------------------------------------
-// One tile of kTile consecutive pairs per block: the blocks in flight then
-// cover one stretch of the partitioned list (a grid-stride loop would spread
-// them over many partitions).
+// One tile of kPutTile consecutive pairs per block, the tiles of one eighth of
+// the partitioned list on the workgroups of one XCD (workgroups go round the
+// eight XCDs): each L2 then sees the 4-byte writes of one or two partitions
+// at a time and puts them together to lines.  Labels and ring of a 512^3 box:
+// 2.30 ms with the tiles in launch order, 2.00 so; still bound by the L2 write
+// requests (four bytes each), not by bytes.
+constexpr int kPutItems = 4;
+constexpr uint32_t kPutTile = kBlock * kPutItems;
+constexpr uint32_t kXcds = 8;
 __global__ __launch_bounds__(kBlock) void k_put(const uint32_t *__restrict__ idx,
                                                 const uint32_t *__restrict__ val, uint64_t ncap,
                                                 const uint32_t *dn, uint32_t orv,
                                                 uint32_t *__restrict__ out) {
   const uint64_t n = dev_count(dn, ncap);
-  const uint64_t base = (uint64_t)blockIdx.x * kTile;
+  const uint64_t per = ((n + kPutTile - 1) / kPutTile + kXcds - 1) / kXcds;
+  if (blockIdx.x / kXcds >= per) return;
+  const uint64_t base = ((blockIdx.x % kXcds) * per + blockIdx.x / kXcds) * kPutTile;
+  uint32_t k[kPutItems], v[kPutItems];
 #pragma unroll
-  for (int r = 0; r < kItems; r++) {
+  for (int r = 0; r < kPutItems; r++) {
     const uint64_t i = base + (uint64_t)r * kBlock + threadIdx.x;
-    if (i < n) out[idx[i]] = val[i] | orv;
+    if (i < n) k[r] = idx[i], v[r] = val[i];
+  }
+#pragma unroll
+  for (int r = 0; r < kPutItems; r++) {
+    const uint64_t i = base + (uint64_t)r * kBlock + threadIdx.x;
+    if (i < n) out[k[r]] = v[r] | orv;
   }
 }
 
@@ -553,7 +567,7 @@ int scatter_u32(const uint32_t *idx, const uint32_t *val, uint32_t *idx2, uint32
   if (rc) return rc;
   k_rs_scatter<<<(uint32_t)nb, kBlock, 0, st>>>(idx, val, idx2, val2, n, dn, shift, hist);
   FOF_HIP(hipGetLastError());
-  k_put<<<(uint32_t)nb, kBlock, 0, st>>>(idx2, val2, n, dn, orv, out);
+  k_put<<<(uint32_t)((n + kPutTile * kXcds - 1) / (kPutTile * kXcds) * kXcds), kBlock, 0, st>>>(idx2, val2, n, dn, orv, out);
   FOF_HIP(hipGetLastError());
   return 0;
 }

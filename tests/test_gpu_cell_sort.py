@@ -80,3 +80,23 @@ def test_occupied_rows_of_uneven_density(ctx, full, thin):
     P["ID"] = np.arange(len(pos))
     dom = L.domain([0] * 3, [nx, 7, 3], [0] * 3, [nx, 7, 3], [1] * 3, 0.8, 2)
     check_against_oracle(ctx, P, dom, flags=L.OPT_SPARSE)
+
+
+# labels and ring through the partition by index or straight, where the members
+# end just before, at and after a tile of 1024 and an eighth of the list
+@pytest.mark.parametrize("n", [1, 2, 255, 1023, 1024, 1025, 8191, 8192, 8193, 65537, 300007])
+def test_partitioned_writes_match_direct_ones(ctx, n):
+    import torch
+
+    print("n", n, flush=True)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(n)
+    side = max(4.0, (n / 6.0) ** (1.0 / 3.0))  # most particles have a neighbour within l
+    rec = torch.zeros((n, 8), dtype=torch.float32, device="cuda")
+    rec[:, 2:5] = torch.rand((n, 3), generator=g, device="cuda") * side
+    dom = L.domain([0] * 3, [side] * 3, [0] * 3, [side] * 3, [1.0] * 3, 0.4, 2)
+    a = linked(ctx, rec, n, dom, L.OPT_WRITE_DIRECT)
+    b = linked(ctx, rec, n, dom, L.OPT_WRITE_PAIRS)
+    assert a[3] == b[3]
+    for x, y in zip(a[:3], b[:3]):
+        assert torch.equal(x, y)
