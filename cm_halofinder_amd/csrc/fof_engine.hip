@@ -429,29 +429,43 @@ constexpr uint32_t kBigCell = 256;
 // 256-way partitions keep a tile's open output lines few enough to be
 // combined in L2; all counting is in LDS.
 //
-// Sizes: tiles of kPartTile particles and buckets of 2^14 cells for large
-// calls; smaller ones shrink both (part_tile, fine_bits) until about 1024
+// Sizes: tiles of kPartTile particles and buckets of 2^14 cells at most;
+// smaller calls shrink both (part_tile, fine_bits) until about 1024
 // tiles and 256 buckets are in flight, since one workgroup's serial pass over
 // 32768 particles is what a small call waits for (64^3 box, 11 tiles and 22
 // buckets, passes A, B and C: 57 + 94, 35 + 44 and 35 us; now 7 + 8 and 15).
 // Up to kMaxBuckets fine buckets pass A places them directly and pass B is
-// not run: with the 1100 buckets of a 256^3 box 426 us for A's scatter against
-// 201 + 46 + 234 for the two (and seven launches fewer), although a sub-tile
-// then holds only two particles a bucket; more buckets than that leave the
-// scatter no room for a second workgroup on a compute unit.
+// not run: with the 1100 buckets of a 256^3 box 333 us for A's scatter, less
+// than the two scatters' reads and writes take (and seven launches fewer),
+// although a sub-tile then holds six particles a bucket.
+//
+// The scatters write a run per bucket and sub-tile, and C's writes are random
+// inside its bucket; what bounds all three is lines that leave L2 partly
+// written.  So a sub-tile is as much as LDS holds (kSub: 512^3 box, 2048
+// particles 1.88 ms for A's scatter and 2.07 for B's, 4096 1.68 and 1.80, 7168
+// 1.67 and 1.66; 256^3 box 444, 369 and 333 us), one workgroup of 1024 threads
+// a compute unit.  With two levels a bucket is 2^12 cells where that leaves
+// at most kMaxCoarse coarse buckets: passes A, B and C of the 512^3 box take
+// 1.67 + 1.66 + 2.73 ms with 2^14 cells, 1.72 + 1.53 + 2.34 with 2^13, 1.85 +
+// 1.52 + 2.12 with 2^12, 2.06 + 1.58 + 2.19 with 2^11.
 // ---------------------------------------------------------------------------
-constexpr uint32_t kPartTile = 32768;
+constexpr uint32_t kSub = 7168;  // particles a partition kernel lays out in LDS at a time
+constexpr uint32_t kPartTile = 5 * kSub;
 constexpr int kFineBits = 14;  // of the largest fine buckets
 constexpr uint32_t kFineCells = 1u << kFineBits;
 constexpr int kMaxBuckets = 1280;  // of pass A
-constexpr int kMaxCoarse = 512;    // coarse buckets (C < 2^31 cells)
+constexpr int kMaxCoarse = 1024;   // coarse buckets (C < 2^31 cells: at most 512 of 2^22)
 
 static uint32_t part_tile(uint64_t N) {
-  return (uint32_t)std::min<uint64_t>(kPartTile, std::max<uint64_t>(1, (N / 1024 + 2047) / 2048) * 2048);
+  const uint64_t n = N / 1024;
+  if (n >= kSub) return (uint32_t)std::min<uint64_t>(kPartTile, n / kSub * kSub);
+  return (uint32_t)std::min<uint64_t>(kSub, std::max<uint64_t>(1, (n + 2047) / 2048) * 2048);
 }
 static int fine_bits(uint64_t C) {
   int fb = kFineBits;
   while (fb > 11 && (C >> fb) < 256) fb--;
+  if ((C + (1u << fb) - 1) >> fb > (uint64_t)kMaxBuckets)  // two levels
+    while (fb > 12 && (C + (1ull << (fb + 7)) - 1) >> (fb + 7) <= (uint64_t)kMaxCoarse) fb--;
   return fb;
 }
 
@@ -548,26 +562,25 @@ __global__ __launch_bounds__(256) void k_pa_count(const uint8_t *__restrict__ ba
 // Partition scatter through LDS: a sub-tile of kSub elements is laid out in
 // bucket order in LDS, then each bucket's elements leave as one contiguous
 // run at the bucket's cursor.  cur[] holds the block's global cursors.
-// 2048 elements (8 per thread) give each of 256 buckets about 8 per flush,
-// so that most output lines are complete before L2 evicts them (1024 was
-// 10% slower on the 1024^3 box: partial lines written twice).
-constexpr int kSub = 2048;
-constexpr int kPartNT = 256;             // threads of the partition scatter kernels
+// 7168 elements (7 per thread) give each of 256 buckets 28 per flush,
+// so that most output lines are complete before L2 evicts them.
+constexpr int kPartNT = 1024;            // threads of the partition scatter kernels
 constexpr int kPer = kSub / kPartNT;     // elements a thread holds per sub-tile
 
 template <int NB>
 __device__ __forceinline__ void staged_part(uint32_t nsub, const uint32_t (&kk)[kPer],
                                             const float4 (&pp)[kPer],
-                                            const uint32_t (&bk)[kPer], uint32_t nbk,
+                                            int shift, uint32_t mask, uint32_t nbk,
                                             uint32_t *cur, uint32_t *lcnt, uint32_t *loff,
-                                            uint32_t *skey, float4 *spos, uint32_t *sbk,
-                                            uint32_t *ws, uint32_t *__restrict__ okey,
+                                            uint32_t *skey, float4 *spos, uint32_t *ws,
+                                            uint32_t *__restrict__ okey,
                                             float4 *__restrict__ opos) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   uint32_t rank[kPer];
 #pragma unroll
   for (int k = 0; k < kPer; k++)
-    if (threadIdx.x + k * kPartNT < nsub) rank[k] = atomicAdd(&lcnt[bk[k]], 1u);
+    if (threadIdx.x + k * kPartNT < nsub)
+      rank[k] = atomicAdd(&lcnt[(kk[k] >> shift) & mask], 1u);
   __syncthreads();
   // exclusive scan of lcnt over the buckets (kB consecutive per thread)
   constexpr int kB = (NB + kPartNT - 1) / kPartNT;
@@ -598,16 +611,15 @@ __device__ __forceinline__ void staged_part(uint32_t nsub, const uint32_t (&kk)[
 #pragma unroll
   for (int k = 0; k < kPer; k++)
     if (threadIdx.x + k * kPartNT < nsub) {
-      const uint32_t j = loff[bk[k]] + rank[k];
+      const uint32_t j = loff[(kk[k] >> shift) & mask] + rank[k];
       skey[j] = kk[k];
       spos[j] = pp[k];
-      sbk[j] = bk[k];
     }
   __syncthreads();
   for (uint32_t j = threadIdx.x; j < nsub; j += kPartNT) {
-    const uint32_t b = sbk[j];
+    const uint32_t key = skey[j], b = (key >> shift) & mask;
     const uint32_t g = cur[b] + (j - loff[b]);
-    okey[g] = skey[j];
+    okey[g] = key;
     opos[g] = spos[j];
   }
   __syncthreads();
@@ -621,7 +633,6 @@ __device__ __forceinline__ void staged_part(uint32_t nsub, const uint32_t (&kk)[
 
 // A, scatter: keys and {x,y,z,index} to the tile's slots of each of at most
 // NB buckets.
-template <int NB>
 __global__ __launch_bounds__(kPartNT) void k_pa_scatter(const uint8_t *__restrict__ base,
                                                     uint32_t stride, uint32_t offpos, uint32_t N,
                                                     uint32_t Bc, uint32_t ntiles,
@@ -630,8 +641,9 @@ __global__ __launch_bounds__(kPartNT) void k_pa_scatter(const uint8_t *__restric
                                                     const uint32_t *__restrict__ off,
                                                     uint32_t *__restrict__ okey,
                                                     float4 *__restrict__ opos) {
+  constexpr int NB = kMaxBuckets;
   __shared__ uint32_t cur[NB], lcnt[NB], loff[NB];
-  __shared__ uint32_t skey[kSub], sbk[kSub];
+  __shared__ uint32_t skey[kSub];
   __shared__ float4 spos[kSub];
   __shared__ uint32_t ws[kPartNT / 64];
   const uint32_t tile = blockIdx.x;
@@ -642,8 +654,8 @@ __global__ __launch_bounds__(kPartNT) void k_pa_scatter(const uint8_t *__restric
   __syncthreads();
   const uint32_t p0 = tile * ptile, p1 = min(N, p0 + ptile);
   for (uint32_t q0 = p0; q0 < p1; q0 += kSub) {
-    const uint32_t nsub = min((uint32_t)kSub, p1 - q0);
-    uint32_t kk[kPer], bk[kPer];
+    const uint32_t nsub = min(kSub, p1 - q0);
+    uint32_t kk[kPer];
     float4 pp[kPer];
 #pragma unroll
     for (int k = 0; k < kPer; k++) {
@@ -653,12 +665,10 @@ __global__ __launch_bounds__(kPartNT) void k_pa_scatter(const uint8_t *__restric
         const uint32_t c = key[p];
         const float *fp = reinterpret_cast<const float *>(base + (uint64_t)p * stride + offpos);
         kk[k] = c;
-        bk[k] = c >> shift;
         pp[k] = make_float4(fp[0], fp[1], fp[2], __uint_as_float(p));
       }
     }
-    staged_part<NB>(nsub, kk, pp, bk, Bc, cur, lcnt, loff, skey, spos, sbk, ws, okey,
-                            opos);
+    staged_part<NB>(nsub, kk, pp, shift, ~0u, Bc, cur, lcnt, loff, skey, spos, ws, okey, opos);
   }
 }
 
@@ -749,7 +759,7 @@ __global__ __launch_bounds__(kPartNT) void k_pb_scatter(uint32_t ptile, int fb,
                                                     uint32_t *__restrict__ okey,
                                                     float4 *__restrict__ opos) {
   __shared__ uint32_t cur[256], lcnt[256], loff[256];
-  __shared__ uint32_t skey[kSub], sbk[kSub];
+  __shared__ uint32_t skey[kSub];
   __shared__ float4 spos[kSub];
   __shared__ uint32_t ws[kPartNT / 64];
   if (tinfo[blockIdx.x] == kNone) return;  // past the last tile
@@ -761,8 +771,8 @@ __global__ __launch_bounds__(kPartNT) void k_pb_scatter(uint32_t ptile, int fb,
   }
   __syncthreads();
   for (uint32_t q0 = i0; q0 < i1; q0 += kSub) {
-    const uint32_t nsub = min((uint32_t)kSub, i1 - q0);
-    uint32_t kk[kPer], bk[kPer];
+    const uint32_t nsub = min(kSub, i1 - q0);
+    uint32_t kk[kPer];
     float4 pp[kPer];
 #pragma unroll
     for (int q = 0; q < kPer; q++) {
@@ -770,11 +780,10 @@ __global__ __launch_bounds__(kPartNT) void k_pb_scatter(uint32_t ptile, int fb,
       // staged_part), so the arrays live in registers, not scratch
       const uint32_t i = min(threadIdx.x + q * kPartNT, nsub - 1);
       kk[q] = ikey[q0 + i];
-      bk[q] = (kk[q] >> fb) & 255u;
       const float4 v = ipos[q0 + i];
       pp[q] = make_float4(v.x, v.y, v.z, v.w);
     }
-    staged_part<256>(nsub, kk, pp, bk, 256, cur, lcnt, loff, skey, spos, sbk, ws, okey, opos);
+    staged_part<256>(nsub, kk, pp, fb, 255u, 256, cur, lcnt, loff, skey, spos, ws, okey, opos);
   }
 }
 
@@ -4405,12 +4414,8 @@ static int enqueue_run(Run &r, hipStream_t st) {
     // one level: straight to pass C's input
     uint32_t *ka = pl.two_level ? k1 : k2;
     float4 *pa = pl.two_level ? p1 : p2;
-    if (Bc <= (uint32_t)kMaxCoarse)
-      k_pa_scatter<kMaxCoarse><<<ntA, kPartNT, 0, st>>>(dbase, stride, offpos, NN, Bc, ntA, ptile,
-                                                        shift, key, offA, ka, pa);
-    else
-      k_pa_scatter<kMaxBuckets><<<ntA, kPartNT, 0, st>>>(dbase, stride, offpos, NN, Bc, ntA, ptile,
-                                                         shift, key, offA, ka, pa);
+    k_pa_scatter<<<ntA, kPartNT, 0, st>>>(dbase, stride, offpos, NN, Bc, ntA, ptile, shift, key,
+                                          offA, ka, pa);
     FOF_HIP(hipGetLastError());
     if (pl.two_level) {
       k_pb_count<<<ntBmax, 256, 0, st>>>(ptile, fb, tinfo, t0, cst, k1, histB);

@@ -82,6 +82,13 @@ def test_occupied_rows_of_uneven_density(ctx, full, thin):
     check_against_oracle(ctx, P, dom, flags=L.OPT_SPARSE)
 
 
+# two levels: buckets of 2^12 cells, tiles of one and of several sub-tiles
+# (7168 particles, 1024 tiles) with a remainder
+@pytest.mark.parametrize("grid,n", [((300, 301, 280), 7340031), ((256, 256, 449), 14680065)])
+def test_two_level_sort_matches_occupied_cells(ctx, grid, n):
+    test_dense_sort_matches_occupied_cells(ctx, grid, n)
+
+
 # labels and ring through the partition by index or straight, where the members
 # end just before, at and after a tile of 1024 and an eighth of the list
 @pytest.mark.parametrize("n", [1, 2, 255, 1023, 1024, 1025, 8191, 8192, 8193, 65537, 300007])
