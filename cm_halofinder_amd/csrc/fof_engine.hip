@@ -2785,8 +2785,12 @@ __global__ __launch_bounds__(256) void k_init_groups(uint32_t N, uint32_t *__res
 //          (one 1.09e9-particle volume: 4 ms less than direct writes spread
 //          over 4.4 GB).
 constexpr uint32_t kLabTile = 4096;
-// Largest volume (particles) written directly: 128 MB of labels.
-constexpr uint64_t kDirectMax = 1ull << 25;
+// Largest volume (particles) written directly: 400 MB of labels, past the 256
+// MB last-level cache.  Whole calls on one periodic box, direct against
+// partitioned: 2.9e7 particles 5.74 against 5.87 ms, 3.8e7 7.46 / 7.70, 6.7e7
+// 12.7 / 13.2, 1.39e8 27.4 / 27.4, 2.7e8 54.9 / 53.3; with minimum IDs 6.7e7
+// 14.55 / 14.78, 9.5e7 21.1 / 21.1, 1.3e8 29.1 / 28.4.
+constexpr uint64_t kDirectMax = 3ull << 25;
 
 template <bool DIRECT>
 __global__ __launch_bounds__(256) void k_label(uint32_t N, const uint32_t *__restrict__ par,
@@ -3985,7 +3989,8 @@ static int make_plan(const fof_particles_v1 *P, const fof_volume_v1 *vols, uint3
   }
   pl.vbeg[nvol] = (uint32_t)pl.N;
   // labels and ring: straight random writes by index while every volume's
-  // range stays in the last-level cache, else through an index partition
+  // range is not much more than the last-level cache, else through an index
+  // partition
   uint64_t maxvol = 0;
   for (uint32_t v = 0; v < nvol; v++) maxvol = std::max<uint64_t>(maxvol, pl.vbeg[v + 1] - pl.vbeg[v]);
   pl.direct_writes = (pl.flags & FOF_OPT_WRITE_PAIRS) ? false
