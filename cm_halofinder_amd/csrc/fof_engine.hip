@@ -178,6 +178,7 @@ struct Grid {
   const uint32_t *cell_of;     // sparse: cell of each sorted particle
   const uint32_t *klo, *khi;   // sparse: key of each cell
   const uint32_t *ncell;       // sparse: cells in the list
+  const uint32_t *err;         // not 0: a particle lies outside its volume (see cell_of_xyz)
   int sparse;
   int volshift;
 };
@@ -473,6 +474,10 @@ static int fine_bits(uint64_t C) {
 __device__ __forceinline__ uint32_t cell_of_xyz(float x, float y, float z, const VolDev &V,
                                                 uint32_t *__restrict__ err) {
   // src_v2/read_data.c:810-812 bounds; non-finite values are rejected too.
+  // Such a particle is sorted as one of cell 0 while its coordinates say another
+  // cell, or none: ranges, sub-cells and key order made from them would not
+  // hold.  So a call with one lists no dense cell and links nothing (its
+  // answer is FOF_E_DOMAIN).
   const bool ok = ((double)x >= V.rmin_buff[0]) && ((double)x <= V.rmax_buff[0]) &&
                   ((double)y >= V.rmin_buff[1]) && ((double)y <= V.rmax_buff[1]) &&
                   ((double)z >= V.rmin_buff[2]) && ((double)z <= V.rmax_buff[2]);
@@ -830,6 +835,7 @@ __global__ __launch_bounds__(kPcThreads) void k_pc_sort(uint64_t C, int fb,
                                                  uint32_t *__restrict__ start,
                                                  float4 *__restrict__ pos4,
                                                  const VolDev *__restrict__ vols, int nvol,
+                                                 const uint32_t *__restrict__ err,
                                                  uint32_t T, uint32_t *__restrict__ dense,
                                                  uint32_t *__restrict__ ndense,
                                                  uint32_t *__restrict__ dbig,
@@ -845,6 +851,7 @@ __global__ __launch_bounds__(kPcThreads) void k_pc_sort(uint64_t C, int fb,
   __shared__ uint32_t lsml[kPcListS], lbig[kPcListB];
   // entries reserved, first reservation that did not fit, global bases
   __shared__ uint32_t nres[2], nfit[2], gbase[2];
+  if (*err) T = kNone;  // no cell is dense
   const uint32_t f = blockIdx.x;
   const uint32_t q0 = fstart[(uint64_t)f * fstride], q1 = fstart[(uint64_t)(f + 1) * fstride];
   const uint64_t c0 = (uint64_t)f << fb;
@@ -1018,14 +1025,16 @@ __global__ __launch_bounds__(256) void k_cells_finish(
     const uint32_t *__restrict__ sklo, const uint32_t *__restrict__ skhi,
     uint32_t *__restrict__ klo, uint32_t *__restrict__ khi,
     const VolDev *__restrict__ vols,
-    const uint32_t *__restrict__ vbeg, int nvol, uint32_t T, uint32_t *__restrict__ dense,
-    uint32_t *__restrict__ ndense, uint32_t *__restrict__ dbig, uint32_t *__restrict__ nbig) {
+    const uint32_t *__restrict__ vbeg, int nvol, const uint32_t *__restrict__ err, uint32_t T,
+    uint32_t *__restrict__ dense, uint32_t *__restrict__ ndense, uint32_t *__restrict__ dbig,
+    uint32_t *__restrict__ nbig) {
   // the tile's dense cells: the small ones from the front, the others from the back
   __shared__ uint16_t lst[kCellTile];
   __shared__ uint32_t cnt[2], base[2];
   const uint32_t U = *dU;
   const uint64_t t0 = (uint64_t)blockIdx.x * kCellTile;
   if (t0 >= U) return;
+  if (*err) T = kNone;  // no cell is dense
   if (threadIdx.x < 2) cnt[threadIdx.x] = 0;
   __syncthreads();
   for (uint32_t q = threadIdx.x; q < kCellTile && t0 + q < U; q += 256) {
@@ -1263,6 +1272,7 @@ __global__ __launch_bounds__(256, 8) void k_link_sparse(uint32_t N, const float4
                                                      const uint32_t *__restrict__ vbeg,
                                                      int nvol, uint32_t T,
                                                      unsigned long long *__restrict__ ctr) {
+  if (*G.err) return;  // a particle's cell may not be the one it is sorted in
   uint32_t tests = 0, rechecks = 0;
   int hint = 0;
   for (uint32_t x = blockIdx.x * blockDim.x + threadIdx.x; x < N;
@@ -1414,6 +1424,7 @@ __global__ __launch_bounds__(256, 6) void k_link_rows(uint32_t N, const float4 *
   const uint32_t wv = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   unsigned long long *const win = wins[wv];
   uint32_t(*const row)[64] = rowc[wv];
+  if (*G.err) return;  // the key list may be out of order
   const uint32_t U = *G.ncell;
   const uint64_t x0 = ((uint64_t)blockIdx.x * 4 + wv) * kRowRun;
   uint32_t tests = 0, rechecks = 0;
@@ -4386,6 +4397,7 @@ static int enqueue_run(Run &r, hipStream_t st) {
   G.klo = B.cnt;      // sparse: the flags' buffer and the sizes' (cleared after linking)
   G.khi = gsize;
   G.ncell = small + kSmU;
+  G.err = small + kSmErr;
   G.sparse = pl.sparse ? 1 : 0;
   G.volshift = pl.volshift;
   if (!pl.sparse) {
@@ -4441,7 +4453,7 @@ static int enqueue_run(Run &r, hipStream_t st) {
     }
     k_pc_sort<<<F, kPcThreads, 0, st>>>((uint64_t)pl.C, fb, pl.two_level ? fst : offA,
                                         pl.two_level ? 1u : ntA, k2, p2, start, pos4, dV,
-                                        (int)nvol, T, dense, small + kSmNDense, dbig,
+                                        (int)nvol, small + kSmErr, T, dense, small + kSmNDense, dbig,
                                         small + kSmNBig, par, runend, gsize);
     FOF_HIP(hipGetLastError());
     if ((rc = te(2))) return rc;
@@ -4473,7 +4485,7 @@ static int enqueue_run(Run &r, hipStream_t st) {
     if ((rc = compact_flagged(cnt, N, nullptr, kFlag, nullptr, start, label, small + kSmU, B.tmp, st)))
       return rc;
     k_cells_finish<<<(uint32_t)((N + kCellTile - 1) / kCellTile), 256, 0, st>>>(small + kSmU, NN, start, par, runend, cnt, gsize, dV, dVB,
-                                       (int)nvol, T, dense, small + kSmNDense, dbig,
+                                       (int)nvol, small + kSmErr, T, dense, small + kSmNDense, dbig,
                                        small + kSmNBig);
     FOF_HIP(hipGetLastError());
     if ((rc = tb(3))) return rc;
