@@ -139,6 +139,7 @@ int fof_ctx_create(int device, fof_ctx **out) {
   c->device = device;
   rc = fof_engine_init(c);
   if (rc) {
+    fof_engine_free(c);
     delete c;
     return rc;
   }

@@ -4857,13 +4857,12 @@ static std::vector<uint32_t> split_volumes(const fof_volume_v1 *vols, uint32_t n
   return cut;
 }
 
-// A pipeline's side stream, made by its first eager call (0.2 ms; a context
-// that only replays graphs has none).
+// A pipeline's side stream: pipeline 0's is made at context set-up (0.2 ms),
+// another's by its first eager call.
 static int open_side(Pipe &pp) {
-  if (pp.side) return 0;
-  FOF_HIP(hipStreamCreate(&pp.side));
-  FOF_HIP(hipEventCreateWithFlags(&pp.side_fork, hipEventDisableTiming));
-  FOF_HIP(hipEventCreateWithFlags(&pp.side_join, hipEventDisableTiming));
+  if (!pp.side) FOF_HIP(hipStreamCreate(&pp.side));
+  if (!pp.side_fork) FOF_HIP(hipEventCreateWithFlags(&pp.side_fork, hipEventDisableTiming));
+  if (!pp.side_join) FOF_HIP(hipEventCreateWithFlags(&pp.side_join, hipEventDisableTiming));
   return 0;
 }
 
@@ -5194,8 +5193,16 @@ uint8_t *g_scratch[64];  // per device, from hipGetSymbolAddress
 extern "C" int fof_engine_init(fof_ctx *ctx) {
   EngineState &S = ctx->st;
   FOF_HIP(hipStreamCreate(&S.main.stream));
-  // everything a later call may need besides workspace: the fork / join and
-  // timing events, and the fixed workspace's address on this device
+  // everything a later call on one pipeline may need besides workspace, so that
+  // fof_link_gpu_noalloc makes and allocates nothing, on the device or
+  // page-locked, from the first call on: the side stream, the head blocks of
+  // one volume, the fork / join and timing events, and the fixed workspace's
+  // address on this device
+  const HeadLayout hl(1, 0);
+  int rc;
+  if ((rc = open_side(S.main)) || (rc = ensure_host(S.main.up, hl.bytes)) ||
+      (rc = ensure_host(S.main.down, hl.vols)))
+    return rc;
   FOF_HIP(hipEventCreateWithFlags(&S.fork, hipEventDisableTiming));
   for (auto &e : S.join) FOF_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
   FOF_HIP(hipEventCreate(&S.t0));

@@ -284,10 +284,11 @@ int fof_link_gpu_ex(fof_ctx *ctx, const fof_particles_v1 *particles,
                     const fof_volume_v1 *vols, uint32_t nvol,
                     const fof_opts_v1 *opts, fof_outputs_v1 *out);
 
-/* fof_link_gpu_ex for one domain without allocating device memory.  This
- * entry point has no counterpart in the reference: it is for callers that
- * cannot allocate (code under HIP graph capture, tight serving loops,
- * harnesses that forbid hipMalloc).  The call's workspace is a fixed array
+/* fof_link_gpu_ex for one domain without allocating device or page-locked
+ * memory or creating streams or events (what it needs of those is made with
+ * the context).  This entry point has no counterpart in the reference: it is
+ * for callers that cannot allocate (code under HIP graph capture, tight
+ * serving loops, harnesses that forbid hipMalloc).  The call's workspace is a fixed array
  * of FOF_NOALLOC_BYTES in the library, one per device, held from the time
  * the library's code is loaded on the device until the process ends.
  * Particles and every output must be device-resident; constant linking
