@@ -1897,13 +1897,15 @@ __global__ __launch_bounds__(NT, WPE) void k_link_dense(const uint32_t *__restri
       if (live) {
         run_of(sa, ha, n1), run_of(sb, hb, n2);
         const uint32_t t1 = min(n1, kTile), t2 = min(n2, kTile);
+        uint32_t spare = 0;
         float4 a[kTile];
 #pragma unroll
         for (uint32_t k = 0; k < kTile; k++) a[k] = ld4(pos4 + ha + min(k, t1 - 1));
         for (uint32_t j = 0; j < t2 && !link; j++) {
           const float4 q = ld4(pos4 + hb + j);
 #pragma unroll
-          for (uint32_t k = 0; k < kTile; k++) link |= pair_linked(a[k], q, R, rechecks);
+          for (uint32_t k = 0; k < kTile; k++)  // past the run's end its last once more, not counted
+            link |= pair_linked(a[k], q, R, k < t1 ? rechecks : spare);
           tests += t1;
         }
         if (link) lunion(lp, sa, sb);
@@ -2278,14 +2280,16 @@ struct SmallLds {
 // nothing links them.  Returns bit k = linked under the reference's test: the FP32
 // decision outside the band; when any lane has a pair inside the band, the
 // block is re-decided pair by pair with pair_linked.  With COLS, cols[k] is
-// the lane mask of partner k's links (the transposed block).
+// the lane mask of partner k's links (the transposed block).  A re-decision
+// counts in the lanes below from + k: in a tile against itself each pair comes
+// up twice, and counts where the lane is the lower one.
 template <bool COLS>
 __device__ __forceinline__ uint32_t testblk(float xi, float yi, float zi,
                                            const float *__restrict__ px,
                                            const float *__restrict__ py,
                                            const float *__restrict__ pz, const Rule &R,
                                            uint32_t &rechecks,
-                                           unsigned long long (&cols)[kBlk]) {
+                                           unsigned long long (&cols)[kBlk], int from) {
   uint32_t lk = 0;
   unsigned long long band = 0;  // lanes with an undecided pair (uniform)
   float qx[kBlk], qy[kBlk], qz[kBlk];
@@ -2306,7 +2310,9 @@ __device__ __forceinline__ uint32_t testblk(float xi, float yi, float zi,
 #pragma unroll
     for (int k = 0; k < kBlk; k++) {
       const float4 q = make_float4(qx[k], qy[k], qz[k], 0.f);
-      const bool l = pair_linked(make_float4(xi, yi, zi, 0.f), q, R, rechecks);
+      uint32_t again = 0;
+      const bool l = pair_linked(make_float4(xi, yi, zi, 0.f), q, R, again);
+      if ((int)(threadIdx.x & 63) < from + k) rechecks += again;
       if (COLS) cols[k] = __ballot(l);
       lk |= l ? (1u << k) : 0u;
     }
@@ -2345,7 +2351,8 @@ __device__ __forceinline__ void small_cell_own(SmallLds &S, uint32_t nA, const R
         unsigned long long cols[kBlk];
         const uint32_t o = 64 * tb + j0;
         const uint32_t h =
-            testblk<true>(xr[ta], yr[ta], zr[ta], S.ax + o, S.ay + o, S.az + o, R, rechecks, cols);
+            testblk<true>(xr[ta], yr[ta], zr[ta], S.ax + o, S.ay + o, S.az + o, R, rechecks, cols,
+                          ta == tb ? (int)j0 : 64);
         rows[ta][tb] |= (unsigned long long)h << j0;
         if (tb != ta) {  // the transposed block: rows of 64 tb + j0 + k, word ta
 #pragma unroll
@@ -2447,8 +2454,10 @@ __device__ __forceinline__ void small_cell(SmallLds &S, uint32_t sA, uint32_t nA
                                            uint32_t &rechecks) {
   const uint32_t lane = threadIdx.x & 63;
   volatile uint32_t *const lp = S.lp;
-  // (A, A)
-  small_cell_own<NW>(S, nA, R, rechecks);
+  // (A, A), in every part and counted in the first
+  uint32_t again = 0;
+  small_cell_own<NW>(S, nA, R, again);
+  rechecks += part == 0 ? again : 0u;
   tests += (lane == 0 && part == 0) ? nA * (nA - 1) / 2 : 0u;
   wave_sync();
   // the next cell's bounds (its index has arrived by now)
@@ -2521,7 +2530,7 @@ __device__ __forceinline__ void small_cell(SmallLds &S, uint32_t sA, uint32_t nA
         unsigned long long cols[kBlk];
         const uint32_t o = 64 * w + j0;
         mw |= (unsigned long long)testblk<false>(bx, by, bz, S.ax + o, S.ay + o, S.az + o, R,
-                                                 rechecks, cols)
+                                                 rechecks, cols, 64)
               << j0;
       }
       m[w] = vb ? mw : 0ull;
