@@ -4013,7 +4013,8 @@ static int make_plan(const fof_particles_v1 *P, const fof_volume_v1 *vols, uint3
     if (pl.N >= 0x7FFFFFFFull) return FOF_E_RANGE;
     pl.hv[v].d.pend = (uint32_t)pl.N;
     pl.Cd += pl.hv[v].ncell_d;
-    nphmin = std::min(nphmin, vols[v].domain.nphalomin);
+    // a size cut that is no number keeps every group (no n is below it)
+    nphmin = std::min(nphmin, std::isnan(vols[v].domain.nphalomin) ? 0.0 : vols[v].domain.nphalomin);
   }
   pl.vbeg[nvol] = (uint32_t)pl.N;
   // labels and ring: straight random writes by index while every volume's
