@@ -2984,8 +2984,8 @@ __global__ __launch_bounds__(256) void k_out_init(uint32_t N, const uint32_t *__
 // bitmap over the input indices and puts its size at lsize[label].  Blocks of
 // consecutive words then total their groups, members and halos (groups passing
 // the size cut) in k_group_sums, and k_group_emit, each block behind the totals
-// of those before it, lists the labels in ascending order, each group's first
-// member slot, its cursor (by label) and the halos' first slots.  Two launches
+// of those before it, lists in label order each group's first member slot and
+// the halos' first slots, and sets its cursor (by label).  Two launches
 // in place of thirteen (bit counts, two scans, the list, the cursors, the halo
 // flags and their compaction), which is what a small call waits for; the sizes
 // are gathered twice for it.
@@ -3063,7 +3063,6 @@ __global__ __launch_bounds__(256) void k_group_sums(uint64_t nw, uint32_t runs,
                                                     const uint32_t *__restrict__ vbeg, int nvol,
                                                     GroupTot *__restrict__ tot) {
   __shared__ uint32_t ws[2][4];
-  uint32_t gh = 0, mem = 0;  // groups | halos << 16 of a run
   GroupTot t = {0, 0, 0, 0};
   for (uint32_t j = 0; j < runs; j++) {
     const uint64_t w = ((uint64_t)blockIdx.x * runs + j) * 256 + threadIdx.x;
@@ -3072,11 +3071,10 @@ __global__ __launch_bounds__(256) void k_group_sums(uint64_t nw, uint32_t runs,
       t.groups++, t.members += n, t.halos += halo ? 1u : 0u;
     });
   }
-  uint32_t g = t.groups, m = t.members, x, y;
-  block_scan2(g, m, gh, mem, ws);
-  uint32_t h = t.halos, z = 0;
-  block_scan2(h, z, x, y, ws);
-  if (threadIdx.x == 0) tot[blockIdx.x] = {gh, mem, x, 0};
+  uint32_t g = t.groups, m = t.members, h = t.halos, z = 0;
+  block_scan2(g, m, t.groups, t.members, ws);
+  block_scan2(h, z, t.halos, t.pad, ws);
+  if (threadIdx.x == 0) tot[blockIdx.x] = t;
 }
 
 __global__ __launch_bounds__(256) void k_group_emit(uint64_t nw, uint32_t runs,
@@ -3085,7 +3083,6 @@ __global__ __launch_bounds__(256) void k_group_emit(uint64_t nw, uint32_t runs,
                                                     const VolDev *__restrict__ vols,
                                                     const uint32_t *__restrict__ vbeg, int nvol,
                                                     const GroupTot *__restrict__ tot,
-                                                    uint32_t *__restrict__ glab,
                                                     uint32_t *__restrict__ offs,
                                                     uint32_t *__restrict__ cursor,
                                                     uint32_t *__restrict__ hk,
@@ -3112,7 +3109,6 @@ __global__ __launch_bounds__(256) void k_group_emit(uint64_t nw, uint32_t runs,
     block_scan2(gh, mem, tgh, tmem, ws);
     uint32_t g = pre.groups + (gh & 0xFFFFu), h = pre.halos + (gh >> 16), at = pre.members + mem;
     word_groups(m, w, lsize, vols, vbeg, nvol, [&](uint32_t lab, uint32_t n, bool halo) {
-      glab[g] = lab;
       offs[g++] = at;
       cursor[lab] = at;
       if (halo && hk) hk[h++] = at;
@@ -4601,13 +4597,13 @@ static int enqueue_run(Run &r, hipStream_t st) {
   // label order, each group's first slot in the member list -- and the halo
   // list (first slots of the groups passing the size cut), then the labels,
   // which also fill the member list.  The sizes by label live in the label
-  // array (before its defaults), the first slots in sk1 and the labels in
-  // order in sv1 (behind 64 words: R + 1 first slots may reach N + 1); lists
-  // of larger groups go to the cell-sorted positions once k_label has read them.
+  // array (before its defaults), the first slots in sk1 (and one word of sv1
+  // behind it: there may be N + 1 of them); lists of larger groups go to the
+  // cell-sorted positions once k_label has read them.
   const int single = pl.single_halos ? 1 : 0;
   const uint64_t rcap = std::max<uint64_t>(single ? N : N / 2, 1);
   uint32_t *lsize = label;
-  uint32_t *offs = sk1, *glist = sv1 + 64;
+  uint32_t *offs = sk1;
   uint32_t *cursor = rtab;             // per label, from its group's first slot
   uint32_t *p32 = reinterpret_cast<uint32_t *>(pos4);
   // groups above kSegLds, kSegWave and four members (at most N / 4096,
@@ -4622,8 +4618,8 @@ static int enqueue_run(Run &r, hipStream_t st) {
   GroupTot *gtot = static_cast<GroupTot *>(B.tmp);
   k_group_sums<<<gb, 256, 0, st>>>(nw, runs, gbits, lsize, dV, dVB, (int)nvol, gtot);
   FOF_HIP(hipGetLastError());
-  k_group_emit<<<gb, 256, 0, st>>>(nw, runs, gbits, lsize, dV, dVB, (int)nvol, gtot, glist, offs,
-                                   cursor, hlist, small);
+  k_group_emit<<<gb, 256, 0, st>>>(nw, runs, gbits, lsize, dV, dVB, (int)nvol, gtot, offs, cursor,
+                                   hlist, small);
   FOF_HIP(hipGetLastError());
   if (!fused) {
     k_label_init<<<tiles_for(N), 256, 0, st>>>(NN, dV, dVB, (int)nvol, label, hsize);
