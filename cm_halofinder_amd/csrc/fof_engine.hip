@@ -3164,11 +3164,10 @@ __device__ __forceinline__ void seg_sort_lane(uint32_t *__restrict__ p, uint32_t
   if (lane < n) p[lane] = v;
 }
 
-// n <= 64 E elements of p to o (may be p): element a = E lane + e in register
-// e of the lane
+// n <= 64 E elements of p, in place: element a = E lane + e in register e of
+// the lane
 template <int E>
-__device__ __forceinline__ void seg_sort_regs(const uint32_t *p, uint32_t *o, uint32_t n,
-                                              uint32_t lane) {
+__device__ __forceinline__ void seg_sort_regs(uint32_t *p, uint32_t n, uint32_t lane) {
   constexpr uint32_t P = 64u * E;
   uint32_t v[E];
 #pragma unroll
@@ -3203,7 +3202,7 @@ __device__ __forceinline__ void seg_sort_regs(const uint32_t *p, uint32_t *o, ui
 #pragma unroll
   for (int e = 0; e < E; e++) {
     const uint32_t a = lane * E + e;
-    if (a < n) o[a] = v[e];
+    if (a < n) p[a] = v[e];
   }
 }
 
@@ -3413,10 +3412,10 @@ __global__ __launch_bounds__(NT, 4) void k_seg_sort_list(const uint32_t *__restr
     const uint32_t n = (uint32_t)__builtin_amdgcn_readfirstlane((int)offs[g + 1]) - s;
     uint32_t *p = mval + s;
     if (n <= 64) seg_sort_lane(p, n, lane);
-    else if (n <= 128) seg_sort_regs<2>(p, p, n, lane);
-    else if (n <= 256) seg_sort_regs<4>(p, p, n, lane);
-    else if (n <= 512) seg_sort_regs<8>(p, p, n, lane);
-    else seg_sort_regs<16>(p, p, n, lane);
+    else if (n <= 128) seg_sort_regs<2>(p, n, lane);
+    else if (n <= 256) seg_sort_regs<4>(p, n, lane);
+    else if (n <= 512) seg_sort_regs<8>(p, n, lane);
+    else seg_sort_regs<16>(p, n, lane);
   }
 }
 
@@ -4472,12 +4471,12 @@ static int enqueue_run(Run &r, hipStream_t st) {
     FOF_HIP(hipGetLastError());
     if ((rc = te(0))) return rc;
     if ((rc = tb(1))) return rc;
-    if ((rc = radix_sort_u32(sk0, sv0, sk1, sv1, N, nullptr, std::min(pl.key_bits, 32), B.tmp, st)))
+    if ((rc = radix_sort_u32(sk0, sv0, sk1, sv1, N, std::min(pl.key_bits, 32), B.tmp, st)))
       return rc;
     if (pl.key_bits > 32) {
       k_gather_u32<<<gN, 256, 0, st>>>(NN, key, sv0, gsize);
       FOF_HIP(hipGetLastError());
-      if ((rc = radix_sort_u32(gsize, sv0, sk1, sv1, N, nullptr, pl.key_bits - 32, B.tmp, st)))
+      if ((rc = radix_sort_u32(gsize, sv0, sk1, sv1, N, pl.key_bits - 32, B.tmp, st)))
         return rc;
     }
     if ((rc = te(1))) return rc;
@@ -4488,11 +4487,10 @@ static int enqueue_run(Run &r, hipStream_t st) {
     if ((rc = te(2))) return rc;
     k_cell_flags<<<gN, 256, 0, st>>>(NN, par, runend, cnt);
     FOF_HIP(hipGetLastError());
-    if ((rc = compact_flagged(cnt, N, nullptr, kFlag, nullptr, start, label, small + kSmU, B.tmp, st)))
-      return rc;
-    k_cells_finish<<<(uint32_t)((N + kCellTile - 1) / kCellTile), 256, 0, st>>>(small + kSmU, NN, start, par, runend, cnt, gsize, dV, dVB,
-                                       (int)nvol, small + kSmErr, T, dense, small + kSmNDense, dbig,
-                                       small + kSmNBig);
+    if ((rc = compact_flagged(cnt, N, kFlag, start, label, small + kSmU, B.tmp, st))) return rc;
+    k_cells_finish<<<(uint32_t)((N + kCellTile - 1) / kCellTile), 256, 0, st>>>(
+        small + kSmU, NN, start, par, runend, cnt, gsize, dV, dVB, (int)nvol, small + kSmErr, T, dense,
+        small + kSmNDense, dbig, small + kSmNBig);
     FOF_HIP(hipGetLastError());
     if ((rc = tb(3))) return rc;
     k_init_uf<<<gN, 256, 0, st>>>(NN, par, runend);

@@ -72,8 +72,8 @@ int scan_u32(const uint32_t *in, uint32_t *out, uint64_t n, void *tmp,
 // Stable LSD radix sort of (key,val) u32 pairs on bits [0,bits).  Result is
 // left in (k0,v0); (k1,v1) are ping-pong buffers of the same size.
 size_t sort_tmp_bytes(uint64_t n);
-int radix_sort_u32(uint32_t *k0, uint32_t *v0, uint32_t *k1, uint32_t *v1,
-                   uint64_t n, const uint32_t *dn, int bits, void *tmp, hipStream_t st);
+int radix_sort_u32(uint32_t *k0, uint32_t *v0, uint32_t *k1, uint32_t *v1, uint64_t n, int bits,
+                   void *tmp, hipStream_t st);
 
 // out[idx[i]] = val[i] | orv for i in [0,n), every idx[i] < nout: the pairs
 // are first partitioned (one radix pass) by the top 8 bits of idx, so that
@@ -84,14 +84,12 @@ int scatter_u32(const uint32_t *idx, const uint32_t *val, uint32_t *idx2, uint32
                 uint64_t n, const uint32_t *dn, uint64_t nout, uint32_t *out, uint32_t orv,
                 void *tmp, hipStream_t st);
 
-// Stable compaction: for every i in [0,n) with (src[i] & flag) != 0, in
-// ascending i, append key = src[i] & ~flag and value = i.  orank[i] (may be
-// null): the list place of the last entry at or before i.  The count goes to
-// *dcount (device; must not alias dn).  tmp: compact_tmp_bytes(n).
+// Stable compaction: every i in [0,n) with (src[i] & flag) != 0, in ascending
+// order; orank[i]: the list place of the last entry at or before i.  The count
+// goes to *dcount (device).  tmp: compact_tmp_bytes(n).
 size_t compact_tmp_bytes(uint64_t n);
-int compact_flagged(const uint32_t *src, uint64_t n, const uint32_t *dn, uint32_t flag,
-                    uint32_t *out_key, uint32_t *out_val, uint32_t *orank, uint32_t *dcount, void *tmp,
-                    hipStream_t st);
+int compact_flagged(const uint32_t *src, uint64_t n, uint32_t flag, uint32_t *out, uint32_t *orank,
+                    uint32_t *dcount, void *tmp, hipStream_t st);
 
 // p[0..n) = v (a kernel, not hipMemsetAsync: captured sequences hold kernel
 // nodes only).

@@ -212,11 +212,9 @@ __global__ void k_scan_single(uint32_t *bsum, uint32_t nb) {
 
 // ---- compaction -------------------------------------------------------------
 __global__ __launch_bounds__(kBlock) void k_compact_count(const uint32_t *__restrict__ src,
-                                                          uint64_t ncap, const uint32_t *dn,
-                                                          uint32_t flag,
+                                                          uint64_t n, uint32_t flag,
                                                           uint32_t *__restrict__ bsum) {
   __shared__ uint32_t ws[kBlock / 64];
-  const uint64_t n = dev_count(dn, ncap);
   const uint64_t base = (uint64_t)blockIdx.x * kTile;
   uint32_t s = 0;
 #pragma unroll
@@ -229,15 +227,12 @@ __global__ __launch_bounds__(kBlock) void k_compact_count(const uint32_t *__rest
 }
 
 __global__ __launch_bounds__(kBlock) void k_compact_emit(const uint32_t *__restrict__ src,
-                                                         uint64_t ncap, const uint32_t *dn,
-                                                         uint32_t flag,
+                                                         uint64_t n, uint32_t flag,
                                                          const uint32_t *__restrict__ boff,
-                                                         uint32_t *__restrict__ okey,
-                                                         uint32_t *__restrict__ oval,
+                                                         uint32_t *__restrict__ out,
                                                          uint32_t *__restrict__ orank,
                                                          uint32_t *__restrict__ dcount) {
   __shared__ uint32_t ws[kBlock / 64];
-  const uint64_t n = dev_count(dn, ncap);
   const uint64_t base = (uint64_t)blockIdx.x * kTile + (uint64_t)threadIdx.x * kItems;
   uint32_t v[kItems], s = 0;
 #pragma unroll
@@ -249,12 +244,8 @@ __global__ __launch_bounds__(kBlock) void k_compact_emit(const uint32_t *__restr
   uint32_t pre = block_excl_scan(s, ws, &tot) + boff[blockIdx.x];
 #pragma unroll
   for (int i = 0; i < kItems; i++) {
-    if (v[i] & flag) {
-      if (okey) okey[pre] = v[i] & ~flag;
-      oval[pre] = (uint32_t)(base + i);
-      pre++;
-    }
-    if (orank && base + i < n) orank[base + i] = pre - 1;
+    if (v[i] & flag) out[pre++] = (uint32_t)(base + i);
+    if (base + i < n) orank[base + i] = pre - 1;
   }
   if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) *dcount = boff[gridDim.x];
 }
@@ -457,17 +448,16 @@ int scan_u32(const uint32_t *in, uint32_t *out, uint64_t n, void *tmp, hipStream
 
 size_t compact_tmp_bytes(uint64_t n) { return scan_levels_bytes(n) + 256; }
 
-int compact_flagged(const uint32_t *src, uint64_t n, const uint32_t *dn, uint32_t flag,
-                    uint32_t *okey, uint32_t *oval, uint32_t *orank, uint32_t *dcount, void *tmp,
-                    hipStream_t st) {
+int compact_flagged(const uint32_t *src, uint64_t n, uint32_t flag, uint32_t *out, uint32_t *orank,
+                    uint32_t *dcount, void *tmp, hipStream_t st) {
   if (n == 0) return fill_u32(dcount, 1, 0u, st);
   uint32_t *bs = static_cast<uint32_t *>(tmp);
   uint64_t nb = (n + kTile - 1) / kTile;
-  k_compact_count<<<(uint32_t)nb, kBlock, 0, st>>>(src, n, dn, flag, bs);
+  k_compact_count<<<(uint32_t)nb, kBlock, 0, st>>>(src, n, flag, bs);
   FOF_HIP(hipGetLastError());
   int rc = scan_bsums(bs, nb, st);
   if (rc) return rc;
-  k_compact_emit<<<(uint32_t)nb, kBlock, 0, st>>>(src, n, dn, flag, bs, okey, oval, orank, dcount);
+  k_compact_emit<<<(uint32_t)nb, kBlock, 0, st>>>(src, n, flag, bs, out, orank, dcount);
   FOF_HIP(hipGetLastError());
   return 0;
 }
@@ -482,8 +472,7 @@ __global__ __launch_bounds__(kBlock) void k_copy_pairs(uint32_t *__restrict__ k0
                                                        uint32_t *__restrict__ v0,
                                                        const uint32_t *__restrict__ k1,
                                                        const uint32_t *__restrict__ v1,
-                                                       uint64_t ncap, const uint32_t *dn) {
-  const uint64_t n = dev_count(dn, ncap);
+                                                       uint64_t n) {
   for (uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x; i < n;
        i += (uint64_t)gridDim.x * kBlock) {
     k0[i] = k1[i];
@@ -491,8 +480,8 @@ __global__ __launch_bounds__(kBlock) void k_copy_pairs(uint32_t *__restrict__ k0
   }
 }
 
-int radix_sort_u32(uint32_t *k0, uint32_t *v0, uint32_t *k1, uint32_t *v1, uint64_t n,
-                   const uint32_t *dn, int bits, void *tmp, hipStream_t st) {
+int radix_sort_u32(uint32_t *k0, uint32_t *v0, uint32_t *k1, uint32_t *v1, uint64_t n, int bits,
+                   void *tmp, hipStream_t st) {
   if (n <= 1 || bits <= 0) return 0;
   const uint64_t nb = (n + kTile - 1) / kTile;
   uint32_t *hist = static_cast<uint32_t *>(tmp);
@@ -501,19 +490,18 @@ int radix_sort_u32(uint32_t *k0, uint32_t *v0, uint32_t *k1, uint32_t *v1, uint6
   uint32_t *ka = k0, *va = v0, *kb = k1, *vb = v1;
   int passes = 0;
   for (int shift = 0; shift < bits; shift += 8, passes++) {
-    k_rs_hist<<<(uint32_t)nb, kBlock, 0, st>>>(ka, n, dn, shift, hist, hn);
+    k_rs_hist<<<(uint32_t)nb, kBlock, 0, st>>>(ka, n, nullptr, shift, hist, hn);
     FOF_HIP(hipGetLastError());
     int rc = scan_u32_dev(hist, hist, 256 * nb, hn, stmp, st);
     if (rc) return rc;
-    k_rs_scatter<<<(uint32_t)nb, kBlock, 0, st>>>(ka, va, kb, vb, n, dn, shift, hist);
+    k_rs_scatter<<<(uint32_t)nb, kBlock, 0, st>>>(ka, va, kb, vb, n, nullptr, shift, hist);
     FOF_HIP(hipGetLastError());
     uint32_t *t = ka;
     ka = kb, kb = t;
     t = va, va = vb, vb = t;
   }
   if (passes & 1) {
-    k_copy_pairs<<<(uint32_t)std::min<uint64_t>(nb * 4, 65536), kBlock, 0, st>>>(k0, v0, ka, va, n,
-                                                                                 dn);
+    k_copy_pairs<<<(uint32_t)std::min<uint64_t>(nb * 4, 65536), kBlock, 0, st>>>(k0, v0, ka, va, n);
     FOF_HIP(hipGetLastError());
   }
   return 0;
