@@ -4871,11 +4871,12 @@ static int open_side(Pipe &pp) {
 }
 
 // One call with a fixed configuration: pipelines `pipes`, graph replay when
-// asked for and possible.
+// asked for and possible; with one_stream the link kernels of a pipeline one
+// after the other, as in a captured or timed call.
 static int run_call(fof_ctx *ctx, const fof_particles_v1 *P, const fof_volume_v1 *vols,
                     uint32_t nvol, const fof_opts_v1 *opts, fof_outputs_v1 *out, uint32_t pipes,
-                    double *wall_ms, HostCheck *check = nullptr, uint8_t *fixed = nullptr,
-                    size_t fixed_bytes = 0) {
+                    double *wall_ms, HostCheck *check, bool one_stream = false,
+                    uint8_t *fixed = nullptr, size_t fixed_bytes = 0) {
   EngineState &S = ctx->st;
   const uint32_t flags = opts ? opts->flags : 0u;
   fof_stats_v1 *stats = out->stats;
@@ -4935,7 +4936,7 @@ static int run_call(fof_ctx *ctx, const fof_particles_v1 *P, const fof_volume_v1
   auto enqueue_all = [&](bool with_timing) -> int {
     for (uint32_t g = 0; g < K; g++) {
       runs[g].timing = with_timing && g == 0;
-      runs[g].side = !graph && !with_timing;
+      runs[g].side = !graph && !with_timing && !one_stream;
       if (runs[g].side)
         if (int e = open_side(*runs[g].pp)) return e;
     }
@@ -5141,6 +5142,11 @@ extern "C" int fof_engine_run(fof_ctx *ctx, const fof_particles_v1 *P, const fof
   if (!tune_lookup(S, key, best)) {
     fof_stats_v1 *user_stats = out->stats;
     out->stats = nullptr;
+    // the candidates run as the call itself will: eagerly, but with the link
+    // kernels overlapped only where the call overlaps them
+    const bool one_stream =
+        (o.flags & FOF_OPT_TIMING) ||
+        ((o.flags & FOF_OPT_GRAPH) && !pl.varlink && !pl.sparse && !pl.host_input && !pl.host_out);
     auto trial = [&](uint32_t T, uint32_t K, uint32_t gb, double &ms) -> int {
       fof_opts_v1 q = o;
       q.flags &= ~(FOF_OPT_TIMING | FOF_OPT_GRAPH);
@@ -5149,7 +5155,7 @@ extern "C" int fof_engine_run(fof_ctx *ctx, const fof_particles_v1 *P, const fof
       double best_ms = 1e300;
       for (int rep = 0; rep < 2; rep++) {  // the first run also warms the workspace
         double w = 0;
-        int e = run_call(ctx, P, vols, nvol, &q, out, K, &w, check);
+        int e = run_call(ctx, P, vols, nvol, &q, out, K, &w, check, one_stream);
         if (e) return e;
         best_ms = std::min(best_ms, w);
       }
@@ -5236,7 +5242,7 @@ extern "C" int fof_engine_run_noalloc(fof_ctx *ctx, const fof_particles_v1 *P,
   // no graph (instantiation allocates), no events, one pipeline, no tuning
   o.flags &= ~(FOF_OPT_TIMING | FOF_OPT_GRAPH | FOF_OPT_AUTOTUNE);
   o.pipelines = 1;
-  return run_call(ctx, P, vol, 1, &o, out, 1, nullptr, nullptr, g_scratch[ctx->device],
+  return run_call(ctx, P, vol, 1, &o, out, 1, nullptr, nullptr, false, g_scratch[ctx->device],
                   kNoAllocBytes);
 }
 

@@ -93,7 +93,10 @@ typedef struct fof_domain_v1 {
 } fof_domain_v1;
 
 /* Options. */
-#define FOF_OPT_TIMING 0x1u     /* record per-phase device times in stats     */
+#define FOF_OPT_TIMING 0x1u     /* record per-phase device times in stats; the
+                                   kernels of a pipeline then run one after
+                                   the other, where an untimed eager call
+                                   overlaps the link kernels                  */
 #define FOF_OPT_OUT_DEVICE 0x2u /* next_out / label_out / halos are device
                                    pointers                                   */
 #define FOF_OPT_NO_RING 0x4u    /* do not write next_out                      */
@@ -110,7 +113,10 @@ typedef struct fof_domain_v1 {
 #define FOF_OPT_AUTOTUNE 0x40u  /* pick the dense-cell threshold and the number
                                    of concurrent pipelines for this workload
                                    shape by timing candidates on the call's own
-                                   input (once per shape; results are cached
+                                   input, link kernels overlapped as in the
+                                   call (not with FOF_OPT_GRAPH or
+                                   FOF_OPT_TIMING; once per shape, whichever
+                                   call comes first; results are cached
                                    per context and in the file named by the
                                    environment variable FOF_TUNE_CACHE)       */
 #define FOF_OPT_WRITE_PAIRS 0x80u   /* write labels and the ring through a
