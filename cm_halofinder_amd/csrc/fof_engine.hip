@@ -4968,14 +4968,21 @@ static int run_call(fof_ctx *ctx, const fof_particles_v1 *P, const fof_volume_v1
     return 0;
   };
   // uploads, on the main stream ahead of everything; they leave from the
-  // pipelines' page-locked buffers, so an early return waits for them too
+  // pipelines' page-locked buffers, and kernels forked to other streams use
+  // the workspaces, so an early return waits for all of them
   struct Settle {
     hipStream_t st;
+    const std::vector<Run> &runs;
     bool on;
     ~Settle() {
-      if (on) (void)hipStreamSynchronize(st);
+      if (!on) return;
+      (void)hipStreamSynchronize(st);
+      for (const Run &r : runs) {
+        if (r.pp->side) (void)hipStreamSynchronize(r.pp->side);
+        if (r.pp->stream != st) (void)hipStreamSynchronize(r.pp->stream);
+      }
     }
-  } settle{st, true};
+  } settle{st, runs, true};
   bool all_seen = pl0.host_input;
   for (auto &r : runs)
     if ((rc = upload_run(ctx, r, st, check, all_seen))) return rc;
