@@ -7,19 +7,21 @@
 //
 // Pipeline (one launch per phase for all volumes of a batch):
 //   1 k_pa_count     reference cell of every particle (src_v2/FOF.c:79-83),
-//                    per-tile histograms of coarse cell buckets
+//                    per-tile histograms of cell buckets
 //   2 scan           (bucket, tile) offsets
-//   3 k_pa_scatter, k_pb_scatter, k_pc_sort   two LDS-staged partitions
-//                    (coarse, then 256 fine buckets of 2^14 cells), then a
-//                    counting sort per fine bucket -> cell starts, dense-cell
-//                    lists and float4 {x,y,z,index} in cell order
+//   3 k_pa_scatter, k_pb_scatter, k_pc_sort   one LDS-staged partition into
+//                    fine buckets of 2^11 to 2^14 cells, or two (coarse
+//                    buckets, then 256 fine ones in each), then a counting sort
+//                    per fine bucket -> cell starts, dense-cell lists and
+//                    float4 {x,y,z,index} in cell order
 //                    (sparse addressing: composite keys, radix sort, cell list)
 //   4 k_subsort      cells with >= max(T, 256) particles: counting sort by
 //                    sub-cell; sub-cells have side <= l/sqrt(3), so each is a
 //                    clique and its particles start in one union-find set
 //                    ("runs")
 //   5 k_link_sparse  one thread per particle of a sparse cell: own cell and
-//                    the 13 forward cells (src_v2/FOF.c:112-153)
+//                    the 13 forward cells (src_v2/FOF.c:112-153); with sparse
+//                    addressing k_link_rows, a wave per 512 particles
 //   6 k_link_dense   dense cells of 256 particles or more, each linked by
 //                    one workgroup that took it from a queue: run pairs with
 //                    early exit
@@ -377,7 +379,7 @@ constexpr int kCtrTestsSparse = 0;  // pair tests in k_link_sparse
 constexpr int kCtrRechecks = 1;     // tests re-decided in FP64 (all kernels)
 constexpr int kCtrGroups = 2;       // groups of any size
 constexpr int kCtrOwned = 3;        // owned halos
-constexpr int kCtrTestsBig = 4;     // pair tests in k_link_dense, 256 threads
+constexpr int kCtrTestsBig = 4;     // pair tests in k_link_dense
 constexpr int kCtrTestsSmall = 5;   // pair tests in k_link_small
 constexpr int kCtrJoined = 6;       // candidate run pairs found already joined
 constexpr int kCtrSlots = 64;
@@ -415,8 +417,8 @@ constexpr int kSmNtB = 10;      // tiles of the fine partition pass
 constexpr int kSmDq = 11;       // next cell of k_link_dense's queue
 constexpr int kSmCtr = 64;
 
-// Dense cells with at least this many particles are linked by a 256-thread
-// workgroup each, smaller ones by a single wave each.
+// Dense cells with at least this many particles are linked by a workgroup each
+// (of 256 to 1024 threads), smaller ones by a wave or a few of them.
 constexpr uint32_t kBigCell = 256;
 
 // ---------------------------------------------------------------------------
@@ -3878,7 +3880,7 @@ struct Plan {
   bool sparse = false;
   int key_bits = 0, volshift = 0;
   uint32_t T = kDefaultT;
-  uint32_t big_grid = 8192;  // workgroups of the 256-thread dense kernels
+  uint32_t big_grid = 8192;  // workgroups of k_link_dense and of its sub-cell sort
   double band = 1e-5;
   std::vector<HostVol> hv;
   std::vector<uint32_t> vbeg;
@@ -4731,8 +4733,8 @@ __global__ __launch_bounds__(256) void k_gather_halos(HaloParts hp, fof_halo_v1 
 }
 
 // ---------------------------------------------------------------------------
-// Autotuning: dense-cell threshold, concurrent pipelines and the grid of the
-// 256-thread dense kernels, per workload shape.
+// Autotuning: dense-cell threshold, concurrent pipelines and the grid of
+// k_link_dense, per workload shape.
 // ---------------------------------------------------------------------------
 static uint32_t ilog2(uint64_t x) {
   uint32_t b = 0;

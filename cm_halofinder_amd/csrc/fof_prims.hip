@@ -1,6 +1,7 @@
 // fof_prims.hip -- device-wide primitives for the FoF engine: exclusive scan,
 // stable compaction and stable LSD radix sort of u32 (key, value) pairs.
-// All kernels use 256-thread blocks (four wave64s) and 4096-element tiles.
+// 256-thread blocks (four wave64s) and 4096-element tiles, but for the
+// one-workgroup scan (1024 threads).
 #include "fof_internal.h"
 
 namespace fof {

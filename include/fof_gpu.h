@@ -141,7 +141,8 @@ typedef struct fof_opts_v1 {
                                pipelines (volumes in contiguous groups of
                                about equal particle counts, each on its own
                                stream and workspace); 0 or 1: one, at most 8 */
-  uint32_t big_grid;        /* workgroups of the 256-thread dense-cell kernels;
+  uint32_t big_grid;        /* workgroups of the kernels of dense cells of 256
+                               particles or more (sub-cell sort, k_link_dense);
                                0 = default (8192)                           */
   uint32_t reserved;
 } fof_opts_v1;
@@ -176,7 +177,8 @@ typedef struct fof_halo_v1 {
  *     256 particles or more
  *   8 labels, member list filled    9 group and halo lists
  *  10 members sorted in each group 11 ring
- *  12 halo list                    13 halo sums
+ *  12 (none: the halo list comes   13 halo sums
+ *     with span 9)
  *  14 output copies                15 pair tests, dense cells below 256
  *  16 total, first span to last                                             */
 #define FOF_NPHASE 17
@@ -188,7 +190,7 @@ typedef struct fof_stats_v1 {
                              sparse)                                         */
   uint64_t ndense;        /* cells linked at sub-cell level                  */
   uint64_t pair_tests;    /* particle-pair distance tests                    */
-  uint64_t rechecks;      /* tests re-decided in FP64                        */
+  uint64_t rechecks;      /* of those, re-decided in FP64                    */
   uint64_t ngroups;       /* groups of any size                              */
   uint64_t nmembers;      /* particles in groups of two or more (the ring)  */
   uint64_t nhalos;        /* groups passing the size cut                     */
@@ -205,7 +207,7 @@ typedef struct fof_stats_v1 {
                              in one set                                      */
   uint32_t pipelines;     /* concurrent pipelines the volumes were split over */
   uint32_t graph;         /* 1: replayed a captured graph, 2: captured one    */
-  uint32_t big_grid;      /* workgroups of the 256-thread dense kernels       */
+  uint32_t big_grid;      /* fof_opts_v1.big_grid in effect                   */
   uint32_t reserved;
 } fof_stats_v1;
 
