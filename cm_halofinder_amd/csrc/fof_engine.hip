@@ -3132,8 +3132,8 @@ __global__ __launch_bounds__(256) void k_group_emit(uint64_t nw, uint32_t runs,
 // per lane, lane-major, so that the stages below distance E stay inside a lane
 // and the others are lane shuffles), the rest for a workgroup each: an LSD
 // radix sort in LDS with as many digits as the indices have bits, up to
-// kSegLds members by 256 threads and up to kSegLdsBig by 1024; beyond that
-// runs of kSegLdsBig merged pairwise through scratch.
+// kSegLds members by 256 threads and up to kSegLdsBig by 1024; beyond that the
+// same passes through scratch, kSegLdsBig members at a time.
 //
 // Why lists: groups come in label order and a label is the group's lowest
 // index, so the first few hundred groups of a volume are its largest; a wave
@@ -3142,7 +3142,11 @@ __global__ __launch_bounds__(256) void k_group_emit(uint64_t nw, uint32_t runs,
 // group, now 5 + 33 + 23 us; 512^3 box 307 + 676 us, now 160 + 580 + 240 (of
 // these, merging chunks in LDS by binary search in place of the radix passes
 // took 45 us for the largest group of the 64^3 box, and a bitonic sort of
-// kSegLds members by 256 threads 676).  What bounds it now: the ranking of
+// kSegLds members by 256 threads 676).  Above kSegLdsBig one workgroup's pass
+// over 2^20 members takes 1.4 ms (three passes 4.4; four with 256 threads and
+// 256 members at a time took 16.4, and merging sorted runs of kSegLdsBig by
+// binary search in scratch 22.4; for 32768 members 0.12, 0.41 and 0.14 ms).
+// What bounds it now: the ranking of
 // the largest group on one compute unit while there are few groups (eight
 // ballots for 64 keys), shuffles and latency when many.  Four waves per SIMD:
 // six spill (508 us at 512^3, 37 at 64^3).
@@ -3270,38 +3274,9 @@ __global__ __launch_bounds__(256) void k_seg_sort(const uint32_t *__restrict__ d
   flush();
 }
 
-// One merge round of width W (a power of two) from a[0 .. n) to o[0 .. n) by
-// NT threads: an element's place in its merged pair of runs is its rank in its
-// own run plus its rank in the partner run (the values are distinct), found
-// for four elements at once so that their reads overlap.
-template <int NT>
-__device__ __forceinline__ void merge_round(const uint32_t *a, uint32_t *o, uint32_t n, uint32_t W) {
-  for (uint32_t i0 = threadIdx.x; i0 < n; i0 += 4 * NT) {
-    uint32_t key[4], at[4], run[4], rl[4], lo[4];
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-      const uint32_t i = min(i0 + j * NT, n - 1);
-      const uint32_t b = i & ~(2 * W - 1), mid = min(b + W, n), end = min(b + 2 * W, n);
-      const bool left = i < mid;
-      key[j] = a[i];
-      run[j] = left ? mid : b;
-      rl[j] = left ? end - mid : mid - b;
-      at[j] = left ? i : b + (i - mid);
-      lo[j] = 0;
-    }
-    for (uint32_t st = W; st > 0; st >>= 1) {
-#pragma unroll
-      for (int j = 0; j < 4; j++)
-        if (lo[j] + st <= rl[j] && a[run[j] + lo[j] + st - 1] < key[j]) lo[j] += st;
-    }
-#pragma unroll
-    for (int j = 0; j < 4; j++)
-      if (i0 + j * NT < n) o[at[j] + lo[j]] = key[j];
-  }
-}
-
-// Groups of list `large` by workgroups of NT threads (up to LDS members in
-// LDS), then, in the 256-thread form, the groups of list `mid` by waves.
+// Groups of list `large` by workgroups of NT threads, up to LDS members in LDS
+// and (the form without MID) larger ones through scratch; then, with MID, the
+// groups of list `mid` by waves.
 template <int NT, uint32_t LDS, bool MID>
 __global__ __launch_bounds__(NT, 4) void k_seg_sort_list(const uint32_t *__restrict__ dL,
                                                       const uint32_t *__restrict__ large,
@@ -3312,99 +3287,129 @@ __global__ __launch_bounds__(NT, 4) void k_seg_sort_list(const uint32_t *__restr
                                                       uint32_t *__restrict__ scratch, int bits) {
   constexpr int kWaves = NT / 64, kR = LDS / NT;  // waves, elements a thread holds
   static_assert(NT >= 256, "a thread for each digit");
-  __shared__ uint32_t sk[LDS], wcnt[kWaves][256], wsum[4];
+  __shared__ uint32_t sk[LDS], wcnt[kWaves][256], wsum[4], cur[MID ? 1 : 256];
   const uint32_t t = threadIdx.x, lane = t & 63;
   const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane((int)(t >> 6));
   const unsigned long long lt = (1ull << lane) - 1;
   const int passes = (bits + 7) / 8, width = (bits + passes - 1) / passes;
-  // n <= LDS elements at p, sorted in place: LSD radix, the keys of a pass in
-  // registers between its ranking and its scatter; wave w ranks the elements
-  // [w per, (w + 1) per) 64 at a time, lanes of one digit by ballots
-  auto sort_lds = [&](uint32_t *p, uint32_t n) {
-    const uint32_t per = (n + NT - 1) / NT * 64, i0 = w * per, i1 = min(n, i0 + per);
+  const uint32_t mask = (1u << width) - 1;
+  auto clear = [&]() {
+    __syncthreads();
+    for (uint32_t q = t; q < kWaves * 256u; q += NT) (&wcnt[0][0])[q] = 0;
+    __syncthreads();
+  };
+  // A digit's number of counted keys, in its thread.
+  auto digit_total = [&]() -> uint32_t {
+    uint32_t c = 0;
+    if (t < 256)
+#pragma unroll
+      for (int q = 0; q < kWaves; q++) c += wcnt[q][t];
+    return c;
+  };
+  // Exclusive scan of one value of each of the first 256 threads.
+  auto scan256 = [&](uint32_t c) -> uint32_t {
+    uint32_t inc = c;
+    if (t < 256) {
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t u = __shfl_up(inc, o, 64);
+        if (lane >= (uint32_t)o) inc += u;
+      }
+      if (lane == 63) wsum[w] = inc;
+    }
+    __syncthreads();
+    uint32_t pre = inc - c;
+    if (t < 256)
+      for (uint32_t q = 0; q < w; q++) pre += wsum[q];
+    return pre;
+  };
+  // The n elements at src in order: a stable pass a digit, LDS elements at a time.
+  // A chunk's keys are in registers between ranking and placing: wave w has the
+  // keys [w per, (w + 1) per) of it, 64 at a time, lanes of one digit found by
+  // ballots, wcnt[w][d] counting the wave's keys of digit d so far and then
+  // their first place.  Up to LDS elements stay in LDS between the passes
+  // and return to src; more go from src to dst and back (far), the digits'
+  // places counted ahead of each pass; the result's place is returned.
+  auto sort = [&](uint32_t *src, uint32_t *dst, uint32_t n) -> uint32_t * {
+    const bool far = !MID && n > LDS;
     for (int k = 0; k < passes; k++) {
       const int shift = k * width;
-      const uint32_t mask = (1u << width) - 1;
-      __syncthreads();
-      for (uint32_t q = t; q < kWaves * 256u; q += NT) (&wcnt[0][0])[q] = 0;
-      __syncthreads();
-      uint32_t key[kR], rk[kR];
-#pragma unroll
-      for (int r = 0; r < kR; r++) {
-        if (64u * r >= per) break;
-        const uint32_t i = i0 + 64 * r + lane;
-        const bool valid = i < i1;
-        key[r] = valid ? (k ? sk[i] : p[i]) : 0u;
+      if (far) {
+        clear();  // (and the pass before is visible to the workgroup)
+        for (uint32_t i = t; i < n; i += NT) atomicAdd(&wcnt[w][(src[i] >> shift) & mask], 1u);
+        __syncthreads();
+        const uint32_t pre = scan256(digit_total());
+        if (!MID && t < 256) cur[t] = pre;
       }
+      for (uint32_t c0 = 0; c0 < n; c0 += LDS) {
+        const uint32_t m = min(LDS, n - c0);
+        const uint32_t per = (m + NT - 1) / NT * 64, i0 = w * per, i1 = min(m, i0 + per);
+        clear();
+        uint32_t key[kR], rk[kR];
 #pragma unroll
-      for (int r = 0; r < kR; r++) {
-        if (64u * r >= per) break;
-        const bool valid = i0 + 64 * r + lane < i1;
-        const uint32_t d = (key[r] >> shift) & mask;
-        unsigned long long peers = __ballot(valid);
-        for (int b = 0; b < width; b++) {
-          const bool on = (d >> b) & 1u;
-          const unsigned long long bb = __ballot(on);
-          peers &= on ? bb : ~bb;
+        for (int r = 0; r < kR; r++) {
+          if (64u * r >= per) break;
+          const uint32_t i = i0 + 64 * r + lane;
+          key[r] = i < i1 ? (k && !far ? sk[i] : src[c0 + i]) : 0u;
         }
-        const uint32_t below = (uint32_t)__popcll(peers & lt);
-        uint32_t old = 0;
-        if (valid) old = wcnt[w][d];
-        wave_sync();
-        if (valid && below == 0) wcnt[w][d] = old + (uint32_t)__popcll(peers);
-        wave_sync();
-        rk[r] = old + below;
-      }
-      __syncthreads();
-      uint32_t c = 0, inc = 0;
-      if (t < 256) {  // each digit's total, scanned over the digits
 #pragma unroll
-        for (int q = 0; q < kWaves; q++) {
-          const uint32_t x = wcnt[q][t];
-          wcnt[q][t] = c;
-          c += x;
+        for (int r = 0; r < kR; r++) {
+          if (64u * r >= per) break;
+          const bool valid = i0 + 64 * r + lane < i1;
+          const uint32_t d = (key[r] >> shift) & mask;
+          unsigned long long peers = __ballot(valid);
+          for (int b = 0; b < width; b++) {
+            const bool on = (d >> b) & 1u;
+            const unsigned long long bb = __ballot(on);
+            peers &= on ? bb : ~bb;
+          }
+          const uint32_t below = (uint32_t)__popcll(peers & lt);
+          uint32_t old = 0;
+          if (valid) old = wcnt[w][d];
+          wave_sync();
+          if (valid && below == 0) wcnt[w][d] = old + (uint32_t)__popcll(peers);
+          wave_sync();
+          rk[r] = old + below;
         }
-        inc = c;
+        __syncthreads();
+        uint32_t at = far ? (t < 256 ? cur[MID ? 0 : t] : 0u) : scan256(digit_total());
+        if (t < 256) {
 #pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-          const uint32_t u = __shfl_up(inc, o, 64);
-          if (lane >= (uint32_t)o) inc += u;
+          for (int q = 0; q < kWaves; q++) {
+            const uint32_t x = wcnt[q][t];
+            wcnt[q][t] = at;
+            at += x;
+          }
+          if (far) cur[MID ? 0 : t] = at;
         }
-        if (lane == 63) wsum[w] = inc;
-      }
-      __syncthreads();
-      if (t < 256) {
-        uint32_t pre = inc - c;
-        for (uint32_t q = 0; q < w; q++) pre += wsum[q];
+        __syncthreads();
 #pragma unroll
-        for (int q = 0; q < kWaves; q++) wcnt[q][t] += pre;
+        for (int r = 0; r < kR; r++) {
+          if (64u * r >= per) break;
+          if (i0 + 64 * r + lane < i1) {
+            const uint32_t o = wcnt[w][(key[r] >> shift) & mask] + rk[r];
+            if (far) dst[o] = key[r];
+            else sk[o] = key[r];
+          }
+        }
       }
-      __syncthreads();
-#pragma unroll
-      for (int r = 0; r < kR; r++) {
-        if (64u * r >= per) break;
-        if (i0 + 64 * r + lane < i1) sk[wcnt[w][(key[r] >> shift) & mask] + rk[r]] = key[r];
+      if (far) {
+        uint32_t *x = src;
+        src = dst, dst = x;
       }
     }
     __syncthreads();
-    for (uint32_t i = t; i < n; i += NT) p[i] = sk[i];
+    if (!far)
+      for (uint32_t i = t; i < n; i += NT) src[i] = sk[i];
+    return src;
   };
   const uint32_t nl = *dL;
   for (uint32_t q = blockIdx.x; q < nl; q += gridDim.x) {
     const uint32_t g = large[q];
     const uint32_t s = offs[g], n = offs[g + 1] - s;
-    uint32_t *src = mval + s, *dst = scratch + s;
-    for (uint32_t c = 0; c < n; c += LDS) sort_lds(src + c, min(LDS, n - c));
-    for (uint32_t W = LDS; W < n; W <<= 1) {
-      __syncthreads();  // the workgroup's writes are visible to it
-      merge_round<NT>(src, dst, n, W);
-      uint32_t *x = src;
-      src = dst, dst = x;
-    }
-    if (src != mval + s) {
-      __syncthreads();
-      for (uint32_t i = t; i < n; i += NT) mval[s + i] = src[i];
-    }
+    const uint32_t *const r = sort(mval + s, scratch + s, n);
+    if (r != mval + s)
+      for (uint32_t i = t; i < n; i += NT) mval[s + i] = r[i];
   }
   if (!MID) return;
   const uint32_t nm = *dMid;

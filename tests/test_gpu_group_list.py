@@ -53,8 +53,9 @@ def test_pairs_far_apart_in_the_list(half, flags):
 @pytest.mark.parametrize("sizes", [
     (16384, 16385), (32768, 32769), (65536, 65537, 40000), (131072, 131073, 5000, 3)])
 def test_large_groups(ctx, sizes):
-    # members of a group at one place, in random input order: one to four
-    # merges of 16384-member runs, each group ending in either buffer
+    # members of a group at one place, in random input order: above 16384 the
+    # sort's passes go through scratch, two of them or three (by the bits of an
+    # index), so that a group ends in either buffer
     rng = np.random.default_rng(sum(sizes))
     who = np.repeat(np.arange(len(sizes)), sizes)
     at = np.stack([2.5 * np.arange(len(sizes)) + 0.3] + 2 * [np.full(len(sizes), 1.7)], 1)
