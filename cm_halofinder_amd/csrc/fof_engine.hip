@@ -1711,8 +1711,8 @@ __device__ __forceinline__ uint32_t div_small(uint32_t a, uint32_t d, float inv)
 // workgroup went through rounds of 768 slots, tested single pairs where they
 // were found and drained a common queue four pairs a wave at a time, each
 // behind two walks of the global union-find: the kernel took 630 us for the
-// 64^3 box (132 cells), 2.88 ms for 256^3 and 7.25 ms for 512^3; now 264, 773
-// and 3.43.  Walking whole rows first instead of the touching sub-cells made
+// 64^3 box (132 cells), 2.88 ms for 256^3 and 7.25 ms for 512^3; now 0.74 and
+// 3.36 ms, and 160 us for the 64^3 box with 1024 threads a cell.  Walking whole rows first instead of the touching sub-cells made
 // half as many pairs again (30 against 15 G cycles at 512^3).  Six waves per
 // SIMD: at eight (64 registers) the spills doubled the cycles per cell, five
 // was 10% slower.
@@ -4559,7 +4559,8 @@ static int enqueue_run(Run &r, hipStream_t st) {
     // wider workgroups while there are too few cells to fill the chip and the
     // largest one's chain is what is waited for: 31^3, 64^3, 144^3, 192^3 and
     // 256^3 boxes 134, 249, 525, 530 and 777 us with 256 threads, 92, 203, 436,
-    // 499 and 872 with 512, 74, 186, 420, - and 1418 with 1024
+    // 499 and 872 with 512, 74, 186, 420, - and 1418 with 1024 (with a division
+    // a test of long pairs; without it 74, 160, 356, 490 and 738 as chosen here)
     auto link_dense = [&](auto kernel, int nt) {
       kernel<<<gbig, nt, dense_lds(ra, kRB), st>>>(dbig, small + kSmNBig, pos4, G, runend, fine,
                                                    rtoff, rtab, T, par, dV, dVB, (int)nvol, ctr, ra,
