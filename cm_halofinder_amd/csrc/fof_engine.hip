@@ -384,6 +384,7 @@ constexpr int kCtrTestsSmall = 5;   // pair tests in k_link_small
 constexpr int kCtrJoined = 6;       // candidate run pairs found already joined
 constexpr int kCtrSlots = 64;
 constexpr int kCtrStride = 16;  // u64 per slot
+constexpr int kCtrWide = 8;     // of these the second half: listed pairs of long runs
 __device__ __forceinline__ void ctr_add(unsigned long long *ctr, int k, unsigned long long v) {
   atomicAdd(ctr + (blockIdx.x & (kCtrSlots - 1)) * kCtrStride + k, v);
 }
@@ -410,6 +411,7 @@ constexpr int kSmErr = 0;       // bit 0: particle outside [rmin_buff, rmax_buff
 constexpr int kSmNDense = 1;    // dense cells below kBigCell particles
 constexpr int kSmM = 2;         // members of groups of two or more (member list)
 constexpr int kSmH = 3;         // halos
+constexpr int kSmWide = 4;      // listed pairs of long runs (may pass kWideCap)
 constexpr int kSmU = 5;         // occupied cells (sparse addressing)
 constexpr int kSmNBig = 7;      // dense cells from kBigCell particles
 constexpr int kSmR = 8;         // groups of two or more (their roots)
@@ -1694,6 +1696,18 @@ __device__ __forceinline__ uint32_t div_small(uint32_t a, uint32_t d, float inv)
   return q;
 }
 
+// Run pairs of many particles, {first, number} of the home cell's run and of the
+// other's: listed by k_link_dense, tested by k_init_groups.  The list lies in
+// the unused half of the counters' lines, four pairs each, so that it costs
+// k_link_dense no register for an address of its own.
+constexpr uint32_t kWideCap = 4 * kCtrSlots;  // further pairs are tested where they are found
+__device__ __forceinline__ uint32_t *wide_count(unsigned long long *ctr) {
+  return reinterpret_cast<uint32_t *>(ctr) - kSmCtr + kSmWide;
+}
+__device__ __forceinline__ uint4 *wide_pair(unsigned long long *ctr, uint32_t k) {
+  return reinterpret_cast<uint4 *>(ctr + (k >> 2) * kCtrStride + kCtrWide) + (k & 3);
+}
+
 // WPE: waves per SIMD to fit (the register budget; LDS per workgroup is
 // sized at launch to the runs a cell of the batch can have).
 //
@@ -1884,8 +1898,9 @@ __global__ __launch_bounds__(NT, WPE) void k_link_dense(const uint32_t *__restri
     constexpr uint32_t kTile = 4;
     // particle pairs from which two walks of the global union-find cost less
     // than the tests they may spare (1024: 32 steps of a group; 1e6 particles
-    // in 10 clumps of sigma 5 l: 0.79 ms with the walks, 0.81 without)
-    constexpr unsigned long long kLongPair = 1024;
+    // in 10 clumps of sigma 5 l: 0.79 ms with the walks, 0.81 without), and
+    // from which a pair is left to a wave of its own (0.9 ms of a group's time)
+    constexpr unsigned long long kLongPair = 1024, kWidePair = 65536;
     auto flush = [&](uint32_t m) {
       wave_sync();
       qn -= m;
@@ -1932,18 +1947,24 @@ __global__ __launch_bounds__(NT, WPE) void k_link_dense(const uint32_t *__restri
         const uint32_t ga = __shfl(ha, src, 64), gb = __shfl(hb, src, 64);
         const uint32_t m1 = __shfl(n1, src, 64), m2 = __shfl(n2, src, 64);
         // joined by now?  (the group's first lane asks: one answer a group; of
-        // a long pair also whether other cells have joined the runs since)
+        // a long pair also whether other cells have joined the runs since, and
+        // the longest are listed for k_init_groups while the list has room)
         bool done = !mine;
         if (mine && gl == 0) {
+          const unsigned long long all = (unsigned long long)m1 * m2;
           done = lfind(lp, xa) == lfind(lp, xb);
-          if (!done && (unsigned long long)m1 * m2 >= kLongPair && uf_find(par, ga) == uf_find(par, gb))
+          if (!done && all >= kLongPair && uf_find(par, ga) == uf_find(par, gb))
             lunion(lp, xa, xb), done = true;
+          joined += done ? 1u : 0u;
+          if (!done && all >= kWidePair) {
+            const uint32_t k = atomicAdd(wide_count(ctr), 1u);
+            if (k < kWideCap) *wide_pair(ctr, k) = make_uint4(ga, m1, gb, m2), done = true;
+          }
         }
         done = __shfl((int)done, lane & ~15u, 64) != 0;
-        if (mine && done && gl == 0) joined++;
         uint32_t rows = done ? 0u : m1;
         const float4 *const qa = pos4 + ga, *const qb = pos4 + gb;
-        PairWalk p(gl, max(m2, 1u));  // (m1 m2 may pass 2^32)
+        PairWalk p(gl, max(m2, 1u));
         while (__ballot(p.i < rows)) {
           bool l = false;
 #pragma unroll
@@ -2785,18 +2806,100 @@ __global__ __launch_bounds__(256) void k_flatten(uint32_t N, uint32_t *__restric
   if ((threadIdx.x & 63) == 0 && t) ctr_add(ctr, kCtrGroups, t);
 }
 
+// Does a particle of run a (na of them) link to one of run b?  By a whole
+// wave: particles of a farther than l from the box of b are passed over 64 at
+// a time, each of the others is tested against b.  prune2 (l^2 with a margin of
+// 1e-4) is compared with differences of floats that are no larger than those
+// of the pairs, so nothing that links is passed over.  Two sub-cells of 20001
+// and 20000 particles 1.2 l apart took 5.2 s pair by pair, now 0.1 ms.
+__device__ __forceinline__ bool wave_runs_link(const float4 *__restrict__ a, uint32_t na,
+                                               const float4 *__restrict__ b, uint32_t nb,
+                                               const Rule &R, uint32_t &tests,
+                                               uint32_t &rechecks) {
+  const uint32_t lane = threadIdx.x & 63;
+  const float gp2 = (float)R.prune2;
+  float lo[3], hi[3];
+  {
+    const float4 q = ld4(b);
+    lo[0] = hi[0] = q.x, lo[1] = hi[1] = q.y, lo[2] = hi[2] = q.z;
+  }
+  for (uint32_t j = lane; j < nb; j += 64) {
+    const float4 q = ld4(b + j);
+    lo[0] = fminf(lo[0], q.x), lo[1] = fminf(lo[1], q.y), lo[2] = fminf(lo[2], q.z);
+    hi[0] = fmaxf(hi[0], q.x), hi[1] = fmaxf(hi[1], q.y), hi[2] = fmaxf(hi[2], q.z);
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1)
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+      lo[d] = fminf(lo[d], __shfl_xor(lo[d], o, 64));
+      hi[d] = fmaxf(hi[d], __shfl_xor(hi[d], o, 64));
+    }
+  for (uint32_t i0 = 0; i0 < na; i0 += 64) {
+    const float4 p = ld4(a + min(i0 + lane, na - 1));
+    const float gx = fmaxf(fmaxf(lo[0] - p.x, p.x - hi[0]), 0.f);
+    const float gy = fmaxf(fmaxf(lo[1] - p.y, p.y - hi[1]), 0.f);
+    const float gz = fmaxf(fmaxf(lo[2] - p.z, p.z - hi[2]), 0.f);
+    unsigned long long near = __ballot(i0 + lane < na && !(gx * gx + gy * gy + gz * gz > gp2));
+    while (near) {
+      const int l = __builtin_ctzll(near);
+      near &= near - 1;
+      auto at = [&](float f) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f), l)); };
+      const float4 q = make_float4(at(p.x), at(p.y), at(p.z), 0.f);
+      for (uint32_t j = lane; j - lane < nb; j += 64) {
+        bool hit = false;
+        if (j < nb) {
+          tests++;
+          hit = pair_linked(q, ld4(b + j), R, rechecks);
+        }
+        if (__ballot(hit)) return true;
+      }
+    }
+  }
+  return false;
+}
+
 // The accumulators of k_flatten (minimum index, with idroot minimum ID; sizes
-// where the bucket sort has not cleared them) and the label bitmap.
+// where the bucket sort has not cleared them) and the label bitmap.  Also
+// the listed pairs of long runs, a wave each unless they are joined by now:
+// k_link_dense has no register to spare for them (10% slower) and a
+// launch of their own costs every call 3 us.
 __global__ __launch_bounds__(256) void k_init_groups(uint32_t N, uint32_t *__restrict__ minorig,
                                                      unsigned long long *__restrict__ idroot,
                                                      uint32_t *__restrict__ gsize,
-                                                     uint32_t nw, uint32_t *__restrict__ bits) {
+                                                     uint32_t nw, uint32_t *__restrict__ bits,
+                                                     const float4 *__restrict__ pos4,
+                                                     uint32_t *__restrict__ par,
+                                                     const VolDev *__restrict__ vols,
+                                                     const uint32_t *__restrict__ vbeg, int nvol,
+                                                     unsigned long long *__restrict__ ctr) {
+  const uint32_t n = min(*wide_count(ctr), kWideCap);
   for (uint32_t x = blockIdx.x * blockDim.x + threadIdx.x; x < N; x += gridDim.x * blockDim.x) {
     minorig[x] = ~0u;
     if (idroot) idroot[x] = ~0ull;
     if (gsize) gsize[x] = 0;
     if (x < nw) bits[x] = 0;
   }
+  const uint32_t w0 = blockIdx.x * 4 + (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  if (w0 >= n) return;
+  const uint32_t lane = threadIdx.x & 63;
+  uint32_t tests = 0, rechecks = 0, joined = 0;
+  for (uint32_t k = w0; k < n; k += gridDim.x * 4) {
+    const uint4 e = *wide_pair(ctr, k);
+    uint32_t v = 0;
+    if (lane == 0) v = uf_find(par, e.x) == uf_find(par, e.z) ? 1u : 0u;
+    if (__builtin_amdgcn_readfirstlane((int)v)) {
+      joined += v;
+      continue;
+    }
+    const VolDev &V = vols[vol_of(vbeg, nvol, e.x)];
+    const float4 p = pos4[e.x];
+    const CellPos cp = cell_pos(V, p.x, p.y, p.z);
+    const Rule R = make_rule(V, cp.ix, cp.iy, cp.iz);
+    if (wave_runs_link(pos4 + e.x, e.y, pos4 + e.z, e.w, R, tests, rechecks) && lane == 0)
+      uf_union(par, e.x, e.z);
+  }
+  add_counters(ctr, kCtrTestsBig, tests, rechecks, joined);
 }
 
 // Members of groups of two or more: label[orig] = group minimum index |
@@ -4594,7 +4697,7 @@ static int enqueue_run(Run &r, hipStream_t st) {
   const uint64_t nw = (N + 31) / 32;
   uint32_t *gbits = key;  // the label bitmap (the head sizes follow in k_label)
   k_init_groups<<<gN, 256, 0, st>>>(NN, minorig, idroot, pl.sparse ? gsize : nullptr, (uint32_t)nw,
-                                    gbits);
+                                    gbits, pos4, par, dV, dVB, (int)nvol, ctr);
   FOF_HIP(hipGetLastError());
   k_flatten<<<gN, 256, 0, st>>>(NN, par, pos4, minorig, gsize, ctr, dbase, stride, offid, idroot);
   FOF_HIP(hipGetLastError());
